@@ -1,0 +1,284 @@
+// Row-register tile body of the fused Horn-Schunck Jacobi sweep for the
+// canonical 8-tap averaging stencil (hs_ring_taps).
+//
+// Like hs_tile, a work-group advances one output tile by k steps on chip: the
+// window is the tile grown by k pixels, and step `it` updates the tile grown
+// by k - it.  Here the window is 64 columns wide, one lane per column, and
+// wave q of the work-group owns P consecutive window rows: a thread keeps (u, v)
+// and the coefficients of its P cells of one column in registers.  A cell's
+// upper and lower neighbours are then the thread's own registers; only the
+// left and right ones go through LDS, and those are a wave's own rows, so a
+// step has one barrier, for the rows where two waves meet.
+//
+// What bounds it: vector issue.  hs_tile reads 8 neighbours per cell from LDS
+// (9 LDS operations of 4 cycles per wave-cell against 33 VALU instructions: the
+// two units are equally loaded and neither hides the other's latency); this
+// body does 3 LDS operations and 31 VALU instructions per cell, no activity
+// test (a row's activity is uniform over its wave) and no per-cell address
+// arithmetic, and its prologue takes ~20 instructions per cell instead of ~47.
+// Measured, us per 8 iterations, hs_tile's variant 24 / this body as
+// hs_rows_choice picks it: 135x240 12.5 / 5.8, 480x640 12.9 / 9.1, 613x977
+// 19.4 / 13.0, 1920x1080 33.6 / 31.2, 3840x2160 112 / 98.
+//
+// Replicated borders cost nothing per step: the lane a cell takes its left (right)
+// neighbour from is clamped to the image once per tile, a window never starts
+// above the image, and the row below the image's last row is that row itself
+// (its wave selects it; if it is the strip's last row, by the address it reads).
+// Cells outside the image load the pixel they clamp to and are never read by
+// an image cell.
+//
+// The arithmetic is hs_update's, in the same order, so results are bit-identical
+// to every other variant: averages as fma chains in tap order from 0, the
+// quotient from the per-cell reciprocal (hs_div.h).  Its range check is made once
+// for a group of up to G cells (|q| of all of them through one minimum and one maximum
+// chain, NaN propagating); a lane that fails it divides all of them.
+#pragma once
+
+#include <type_traits>
+
+#include "hmx_common.h"
+#include "hs_div.h"
+#include "hs_tile.h"
+
+#pragma clang fp contract(off)
+
+namespace hmx {
+
+constexpr int HS_ROWS_COLS = 64;  // window columns: one per lane
+
+// LDS of one work-group: the first and last row of every wave's strip, double
+// buffered (another wave reads them), and its other rows (read by the wave alone).
+template <int NW, int P>
+struct HsRowsLds {
+    float2 edge[2][NW][2][HS_ROWS_COLS];
+    float2 row[NW][P > 2 ? P - 2 : 1][HS_ROWS_COLS];
+};
+
+// a window row around one column: left neighbour, cell, right neighbour
+struct HsTri {
+    float2 l, c, r;
+};
+
+// Tile (txi, tyi) of the grid of tw x th tiles of image a, k steps; w: the
+// averaging weights in the canonical tap order.  The host keeps tw + 2k <= 64
+// and th + 2k <= NW * P.
+// PRE: a row's left and right neighbours for the next step are read as soon as
+// the row is written, so their latency is a step away from their use (four
+// more registers per row); otherwise they are read as the row is reached.
+// G: rows computed together (independent fma chains in flight, one range check).
+// LOUT: also store each step's (ubar, vbar) of the output tile (HsImage::lub).
+template <int NW, int P, bool PRE, int G, bool LOUT = false>
+__device__ __forceinline__ void hs_rows_tile(const HsImage &a, int txi, int tyi, int tw, int th,
+                                             int k, const float (&w)[8], HsRowsLds<NW, P> &lds) {
+    static_assert(P >= 2, "a strip has a first and a last row");
+    const int lane = threadIdx.x & 63;
+    const int wave = __builtin_amdgcn_readfirstlane((int)threadIdx.x >> 6);
+    const int H = a.H, W = a.W;
+    const int x0 = txi * tw, y0 = tyi * th;
+    const int x1 = min(x0 + tw, W), y1 = min(y0 + th, H);
+    // window: columns x0 - k .., rows from y0 - k, or from the image's first
+    const int gx0 = x0 - k, gy0 = max(y0 - k, 0);
+    const int gx = gx0 + lane;
+    const int r0 = wave * P;  // the strip's first window row
+
+    float cx[P], cy[P], ct[P], cd[P], cr[P], u[P], v[P];
+    {
+        // byte offsets from the image start fit 32 bits (H, W < 32768); every
+        // load of the thread is issued before any is used
+        const char *const pIx = reinterpret_cast<const char *>(a.Ix);
+        const char *const pIy = reinterpret_cast<const char *>(a.Iy);
+        const char *const pIt = reinterpret_cast<const char *>(a.It);
+        const char *const pu = reinterpret_cast<const char *>(a.u_in);
+        const char *const pv = reinterpret_cast<const char *>(a.v_in);
+        const char *const pd = reinterpret_cast<const char *>(a.den);
+        const unsigned rowb = (unsigned)W * 4u;
+        const unsigned co = (unsigned)clampi(gx, 0, W - 1) * 4u;
+#pragma unroll
+        for (int j = 0; j < P; ++j) {
+            const unsigned o = (unsigned)min(gy0 + r0 + j, H - 1) * rowb + co;
+            auto ld = [&](const char *p) { return ld_g(reinterpret_cast<const float *>(p + o)); };
+            u[j] = ld(pu);
+            v[j] = ld(pv);
+            cx[j] = ld(pIx);
+            cy[j] = ld(pIy);
+            ct[j] = ld(pIt);
+            if (pd) cd[j] = ld(pd);
+        }
+#pragma unroll
+        for (int j = 0; j < P; ++j) {
+            if (!pd) {
+                const float m1 = cx[j] * cx[j];
+                const float s1 = a.alpha2 + m1;
+                const float m2 = cy[j] * cy[j];
+                cd[j] = s1 + m2;
+            }
+            cr[j] = hs_recip(cd[j]);
+        }
+    }
+    // the lanes of the neighbouring columns, clamped to the image and the window
+    const int lmin = max(-gx0, 0), lmax = min(W - 1 - gx0, HS_ROWS_COLS - 1);
+    const int li = clampi(lane - 1, lmin, lmax), ri = clampi(lane + 1, lmin, lmax);
+    const int jb = H - 1 - gy0 - r0;  // the image's last row, as a strip row
+    const bool in = gx >= x0 && gx < x1;
+
+    auto slot = [&](int buf, int j) -> float2 * {
+        if (j == 0) return lds.edge[buf][wave][0];
+        if (j == P - 1) return lds.edge[buf][wave][1];
+        return lds.row[wave][j - 1];
+    };
+    // a wave's LDS writes before its reads of the same row (a wavefront's LDS
+    // accesses are performed in order; this keeps the compiler's order)
+    auto wave_fence = []() {
+        __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+        __builtin_amdgcn_wave_barrier();
+        __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+    };
+    float2 L[PRE ? P : 1], R[PRE ? P : 1];
+#pragma unroll
+    for (int j = 0; j < P; ++j) slot(0, j)[lane] = make_float2(u[j], v[j]);
+    wave_fence();
+    if (PRE) {
+#pragma unroll
+        for (int j = 0; j < P; ++j) {
+            L[j] = slot(0, j)[li];
+            R[j] = slot(0, j)[ri];
+        }
+    }
+    // BOT: the image's last row is in the strip and not its last row
+    auto steps = [&](auto bot_c) {
+        constexpr bool BOT = decltype(bot_c)::value;
+        for (int it = 1; it <= k; ++it) {
+            // step it reads edge buffer (it - 1) & 1 and writes the other, which
+            // was last read in step it - 1, before this barrier.  (A row that is
+            // not active in a step is not written, and never read as valid later.)
+            __syncthreads();
+            const int buf = (it - 1) & 1;
+            // active strip rows [lo, hi): the tile grown by k - it, inside the image
+            const int lo = max(y0 - (k - it), 0) - gy0 - r0;
+            const int hi = min(y1 + (k - it), H) - gy0 - r0;
+            if (lo >= P || hi <= 0) continue;
+            const float2 *const ra =
+                (gy0 + r0 == 0 || wave == 0) ? lds.edge[buf][wave][0] : lds.edge[buf][wave - 1][1];
+            const float2 *const rb = (jb == P - 1 || wave == NW - 1) ? lds.edge[buf][wave][1]
+                                                                     : lds.edge[buf][wave + 1][0];
+            auto row = [&](int j) {
+                HsTri q;
+                q.c = make_float2(u[j], v[j]);
+                q.l = PRE ? L[PRE ? j : 0] : slot(buf, j)[li];
+                q.r = PRE ? R[PRE ? j : 0] : slot(buf, j)[ri];
+                return q;
+            };
+            // the old rows above the group (prev) and its first (cur)
+            HsTri prev = {ra[li], ra[lane], ra[ri]};
+            HsTri cur = row(0);
+#pragma unroll
+            for (int j0 = 0; j0 < P; j0 += G) {
+                const int n = P - j0 < G ? P - j0 : G;
+                HsTri rows[G + 1];  // old rows j0 .. j0 + n
+                rows[0] = cur;
+#pragma unroll
+                for (int i = 1; i < n; ++i) rows[i] = row(j0 + i);
+                if (j0 + n < P)
+                    rows[n] = row(j0 + n < P ? j0 + n : 0);
+                else
+                    rows[n] = {rb[li], rb[lane], rb[ri]};
+                if (j0 + n > lo && j0 < hi) {
+                    float ub[G], vb[G], s2[G], q[G];
+#pragma unroll
+                    for (int i = 0; i < n; ++i) {
+                        const int j = j0 + i;
+                        const HsTri &up = i == 0 ? prev : rows[i > 0 ? i - 1 : 0];
+                        const HsTri &me = rows[i];
+                        HsTri dn = rows[i + 1];
+                        if (BOT && j == jb) dn = me;
+                        float x = 0.0f, y = 0.0f;
+                        auto tap = [&](int d, float2 z) {
+                            x = fmaf(w[d], z.x, x);
+                            y = fmaf(w[d], z.y, y);
+                        };
+                        tap(0, me.l);  // HS_RING_OX/OY order
+                        tap(1, me.r);
+                        tap(2, up.c);
+                        tap(3, dn.c);
+                        tap(4, up.l);
+                        tap(5, up.r);
+                        tap(6, dn.l);
+                        tap(7, dn.r);
+                        ub[i] = x;
+                        vb[i] = y;
+                        const float m1 = cx[j] * x;
+                        const float m2 = cy[j] * y;
+                        const float s1 = m1 + m2;
+                        s2[i] = s1 + ct[j];
+                        // hs_div_fast's quotient; its range check follows
+                        const float q0 = s2[i] * cr[j];
+                        const float e0 = fmaf(-q0, cd[j], s2[i]);
+                        const float q1 = fmaf(e0, cr[j], q0);
+                        const float e1 = fmaf(-q1, cd[j], s2[i]);
+                        q[i] = fmaf(e1, cr[j], q1);
+                    }
+                    float mx = fabsf(q[0]), mn = mx;
+#pragma unroll
+                    for (int i = 1; i < n; ++i) {
+                        mx = __builtin_elementwise_maximum(mx, fabsf(q[i]));
+                        mn = __builtin_elementwise_minimum(mn, fabsf(q[i]));
+                    }
+                    if (!(mn >= 0x1p-76f && mx <= 0x1p76f)) {
+#pragma unroll
+                        for (int i = 0; i < n; ++i) {
+                            float so = s2[i];  // opaque: the divisions stay in the branch
+                            asm volatile("" : "+v"(so));
+                            q[i] = so / cd[j0 + i];
+                        }
+                    }
+#pragma unroll
+                    for (int i = 0; i < n; ++i) {
+                        const int j = j0 + i;
+                        const float p1 = cx[j] * q[i];
+                        const float p2 = cy[j] * q[i];
+                        u[j] = ub[i] - p1;
+                        v[j] = vb[i] - p2;
+                        slot(buf ^ 1, j)[lane] = make_float2(u[j], v[j]);
+                        if (LOUT) {
+                            const int gy = gy0 + r0 + j;
+                            if (in && gy >= y0 && gy < y1) {
+                                const int64_t so = (int64_t)(it - 1) * a.lstride + (int64_t)gy * W;
+                                ((gfloat *)(a.lub + so))[gx] = ub[i];
+                                ((gfloat *)(a.lvb + so))[gx] = vb[i];
+                            }
+                        }
+                    }
+                    wave_fence();
+                    if (PRE) {
+#pragma unroll
+                        for (int i = 0; i < n; ++i) {
+                            L[PRE ? j0 + i : 0] = slot(buf ^ 1, j0 + i)[li];
+                            R[PRE ? j0 + i : 0] = slot(buf ^ 1, j0 + i)[ri];
+                        }
+                    }
+                }
+                prev = rows[n - 1];
+                cur = rows[n];
+            }
+        }
+    };
+    if (jb >= 0 && jb < P - 1)
+        steps(std::true_type());
+    else
+        steps(std::false_type());
+    // (plain stores: the tile's rows are partial cache lines, which the L2 merges
+    // with the neighbouring tiles' before they go to memory)
+    if (in) {
+#pragma unroll
+        for (int j = 0; j < P; ++j) {
+            const int gy = gy0 + r0 + j;
+            if (gy >= y0 && gy < y1) {
+                const unsigned o = (unsigned)gy * (unsigned)W + (unsigned)gx;
+                ((gfloat *)a.u_out)[o] = u[j];
+                ((gfloat *)a.v_out)[o] = v[j];
+            }
+        }
+    }
+}
+
+}  // namespace hmx

@@ -48,7 +48,7 @@ int hs_jacobi_run(const float *Ix, const float *Iy, const float *It, const float
                   float alpha2, int H, int W, const Taps &taps, int iters, float *u, float *v,
                   float *wu, float *wv, int variant, int k, hipStream_t s, int B,
                   const float *alpha2_b, bool start_in_work);
-void hs_choice(int H, int W, int &variant, int &k);
+void hs_choice(int H, int W, int B, int iters, const Taps &taps, int &variant, int &k);
 
 __device__ inline void tr_range(int p, int o, int n, int &lo, int &hi) {
     lo = (p == 0) ? 0 : p - o;
@@ -643,7 +643,7 @@ extern "C" int hmx_hs_forward_ckpt(const float *I1, const float *I2, int B, int 
     rc = setup_batch(I1, I2, B, H, W, T.dx, T.dy, T.dt, Ix, Iy, It, s);
     if (rc) return rc;
     int variant, k;
-    hs_choice(H, W, variant, k);
+    hs_choice(H, W, B, std::min(iters, ckpt_every), T.av, variant, k);
     const int nck = hmx_hs_ckpt_count(iters, ckpt_every);
     for (int c = 0; c < nck; ++c) {
         float *cu = ckpt + (int64_t)(2 * c) * n, *cv = ckpt + (int64_t)(2 * c + 1) * n;

@@ -20,6 +20,7 @@
 // region reaches past the image, its cells outside the image are ghosts that
 // hold the pixel they clamp to (hs_tile.h), so every tile reads its taps at
 // the same precomputed deltas.
+#include "hs_rows.h"
 #include "hs_tile.h"
 
 #include <algorithm>
@@ -44,6 +45,7 @@ struct HsArgs {
     int64_t bstride;        // elements between consecutive pairs (blockIdx.y)
     float *lt, *lub, *lvb;  // optional per-step linearisation output (see HsImage)
     int64_t lstride;
+    int tw, th;             // output tile of the row-register kernels (hs_rows_geom)
 };
 
 // The linearisation-output form (the adjoint's segment recompute) is compiled
@@ -131,6 +133,37 @@ __global__ __launch_bounds__(NT) void hs_strip_kernel(HsArgs a, Taps taps) {
     const HsTapTable<TW + 2 * KMAX> tp(taps, NTAP);
     hs_tile_strip<NT, TW, TH, KMAX, S, NTAP>(im, xcd_remap(blockIdx.x, a.ntiles, a.rev), a.k, tp,
                                              uv);
+}
+
+// Row-register form (hs_rows.h): a window of 64 columns x NW * P rows, the canonical
+// 8-tap averaging offsets.  WPE: waves per SIMD the build is held to.
+template <int NW, int P, bool PRE, int G, int WPE, bool LOUT = false>
+__global__ __launch_bounds__(64 * NW, WPE) void hs_rows_kernel(HsArgs a, Taps taps) {
+    __shared__ HsRowsLds<NW, P> lds;
+    const int64_t off = (int64_t)blockIdx.y * a.bstride;
+    HsImage im;
+    im.Ix = a.Ix + off;
+    im.Iy = a.Iy + off;
+    im.It = a.It + off;
+    im.den = a.den ? a.den + off : nullptr;
+    im.u_in = a.u_in + off;
+    im.v_in = a.v_in + off;
+    im.u_out = a.u_out + off;
+    im.v_out = a.v_out + off;
+    im.alpha2 = a.alpha2_b ? a.alpha2_b[blockIdx.y] : a.alpha2;
+    im.H = a.H;
+    im.W = a.W;
+    if (LOUT) {
+        im.lub = a.lub + off;
+        im.lvb = a.lvb + off;
+        im.lstride = a.lstride;
+    }
+    float w[8];
+#pragma unroll
+    for (int d = 0; d < 8; ++d) w[d] = taps.w[d];
+    const int t = xcd_remap(blockIdx.x, a.ntiles, a.rev);
+    const int tyi = t / a.tiles_x, txi = t - tyi * a.tiles_x;
+    hs_rows_tile<NW, P, PRE, G, LOUT>(im, txi, tyi, a.tw, a.th, a.k, w, lds);
 }
 
 // ---------------------------------------------------------------------------
@@ -248,6 +281,13 @@ struct HsVariant {
     void (*kernel[5])(HsArgs, Taps);  // by tap class: 4, 5, 8, 9 taps, any
     void (*ring)(HsArgs, Taps);       // ring-ordered kernel for the canonical 8 taps, or null
     bool persist;                     // whole solve in one persistent launch (hs_persist_run)
+    // Row-register forms: waves per work-group and rows per wave of the canonical
+    // stencil's kernel (in `ring`; other stencils run variant 24's kernels), the
+    // work-groups of it a CU holds, and its launch cost (rows_launch_us): us
+    // of a launch besides the steps, and per window row of each work-group a CU
+    // takes.  Zero for the others.
+    int nw, rows, wgs;
+    float us0, us_row;
 };
 
 // tap count -> kernel slot (straight-line kernels for the common stencils)
@@ -286,6 +326,15 @@ static int tap_class(int nd) {
      {hs_strip_kernel<NT, TW, TH, K, S, 4>, hs_strip_kernel<NT, TW, TH, K, S, 5>,      \
       hs_strip_kernel<NT, TW, TH, K, S, 8>, hs_strip_kernel<NT, TW, TH, K, S, 9>,      \
       hs_strip_kernel<NT, TW, TH, K, S, 0>}, nullptr}
+// row-register forms: the canonical stencil's kernel, and variant 24's for others
+#define HS_R(NW, P, PRE, G, WPE, WGS, KMAX, US0, USROW)                                 \
+    {1024, 64, 32, KMAX, 0,                                                             \
+     {hs_tb_kernel<1024, 64, 32, 8, 4, false, true, true>,                              \
+      hs_tb_kernel<1024, 64, 32, 8, 5, false, true, true>,                              \
+      hs_tb_kernel<1024, 64, 32, 8, 8, false, true, true>,                              \
+      hs_tb_kernel<1024, 64, 32, 8, 9, false, true, true>,                              \
+      hs_tb_kernel<1024, 64, 32, 8, 0, false, true, true>},                             \
+     hs_rows_kernel<NW, P, PRE, G, WPE>, false, NW, P, WGS, US0, USROW}
 static const HsVariant kVariants[] = {
     HS_V(256, 64, 16, 1),     // 0: one iteration per launch (plain sweep)
     HS_V(256, 64, 32, 4),     // 1
@@ -333,23 +382,116 @@ static const HsVariant kVariants[] = {
       hs_tb_kernel<1024, 64, 32, 8, 9, false, true, true>,
       hs_tb_kernel<1024, 64, 32, 8, 0, false, true, true>},
      nullptr, true},
+    // 29-36: row-register forms, chosen by hs_rows_choice.  One work-group of 16
+    // waves per CU, for images that give a CU at most one tile: the window's
+    // height sets how many pixels a CU takes (neighbours prefetched; 56 to 110
+    // VGPRs).  Two work-groups per CU for larger images, so that one's loads
+    // and barriers overlap the other's steps: 8 waves at up to 128 VGPRs, or 16 at
+    // 61 (one row at a time).
+    HS_R(16, 2, true, 2, 4, 1, 12, 4.39f, 0.0183f),   // 29: window 64 x 32
+    HS_R(16, 3, true, 3, 4, 1, 16, 3.22f, 0.0422f),   // 30: 64 x 48
+    HS_R(16, 4, true, 4, 4, 1, 16, 3.09f, 0.0437f),   // 31: 64 x 64
+    HS_R(16, 5, true, 5, 4, 1, 16, 2.89f, 0.0445f),   // 32: 64 x 80
+    HS_R(8, 7, false, 4, 4, 2, 16, 6.22f, 0.0077f),   // 33: 64 x 56
+    HS_R(8, 9, false, 3, 4, 2, 16, 7.28f, 0.0092f),   // 34: 64 x 72
+    HS_R(8, 10, false, 2, 4, 2, 16, 8.32f, 0.0099f),  // 35: 64 x 80
+    HS_R(16, 4, false, 1, 8, 2, 16, 5.80f, 0.0201f),  // 36: 64 x 64
 };
+#undef HS_R
 #undef HS_V
 #undef HS_D
 #undef HS_S
 #undef HS_F
 static constexpr int kNumVariants = sizeof(kVariants) / sizeof(kVariants[0]);
 
+// iterations of "a long solve", where a size's (variant, k) is asked for by itself
+constexpr int kLongSolve = 500;
+
 static std::mutex g_tune_mu;
 static std::map<std::pair<int, int>, std::pair<int, int>> g_tuned;  // (H,W) -> (variant,k)
 
-// Untuned sizes: double-buffered window with the reciprocal quotient, k = 8
-// (the fastest variant at 512^2 .. 3840x2160 in the sweeps).
-static void default_choice(int H, int W, int &variant, int &k) {
-    (void)H;
-    (void)W;
+// Whether a launch of variant V with these taps runs its row-register kernel.
+static bool hs_runs_rows(const HsVariant &V, const Taps &taps) {
+    return V.nw > 0 && hs_ring_taps(taps);
+}
+
+// Iterations per launch as the launches of a solve take them: a row-register
+// variant's other stencils run variant 24's kernels, 8 at most.
+static int hs_effective_k(int variant, int k, const Taps &taps) {
+    const HsVariant &V = kVariants[variant];
+    return V.nw > 0 && !hs_ring_taps(taps) ? std::min(k, 8) : k;
+}
+
+// Tile grid of a row-register launch of B images: as few columns and rows of
+// tiles as the window allows, then as many rows of tiles as the same number of
+// rounds of work-groups takes, each shorter: a round lasts as long as one tile,
+// so 3600 tiles on 512 places (8 rounds, the last of 16 tiles) cost 8 rounds
+// of 48 rows and 4080 tiles cost 8 of 43 (3840x2160: 107 and 98 us).
+struct RowsGeom {
+    int tw, th, tiles_x, ntiles;  // ntiles: of one image
+};
+constexpr int kCus = 256;
+static RowsGeom hs_rows_geom(const HsVariant &V, int H, int W, int k, int B) {
+    RowsGeom g;
+    const int mw = HS_ROWS_COLS - 2 * k, mh = V.nw * V.rows - 2 * k;
+    int nx = (W + mw - 1) / mw;
+    g.tw = (W + nx - 1) / nx;
+    nx = (W + g.tw - 1) / g.tw;
+    int ny = (H + mh - 1) / mh;
+    const int64_t slots = (int64_t)V.wgs * kCus, col = (int64_t)nx * B;
+    const int64_t rounds = (col * ny + slots - 1) / slots;
+    ny = (int)std::max<int64_t>(ny, std::min<int64_t>(rounds * slots / col, H));
+    g.th = (H + ny - 1) / ny;
+    ny = (H + g.th - 1) / g.th;
+    g.tiles_x = nx;
+    g.ntiles = nx * ny;
+    return g;
+}
+
+// Cost of a row-register launch of k steps in us, from what bounds it: the
+// busiest CU takes m tiles, each of which loads its window and updates its
+// active rows (th + k - 1 on average over the steps) at 31 VALU instructions
+// per wave-row.  The constants are a fit to 15 image sizes from 64^2 to
+// 3840x2160 at k = 5 .. 12, every variant (rms error 3-8 %); the choice it makes
+// was within 2.6 % of the fastest measured one at every size.
+constexpr float kRowsStepUs = 0.0150f;
+static float rows_launch_us(const HsVariant &V, int H, int W, int k, int B) {
+    const RowsGeom g = hs_rows_geom(V, H, W, k, B);
+    const int m = (int)(((int64_t)g.ntiles * B + kCus - 1) / kCus);
+    const int win = V.nw * V.rows;
+    const int active = std::min(std::min(g.th + k - 1, win), H);
+    return V.us0 + (float)m * (V.us_row * (float)win + kRowsStepUs * (float)(k * active));
+}
+
+// The row-register variant and iterations per launch with the least cost for
+// iters iterations of B images (the iterations split evenly over the launches).
+static void hs_rows_choice(int H, int W, int B, int iters, int &variant, int &k) {
+    float best = 1e30f;
+    for (int vi = 0; vi < kNumVariants; ++vi) {
+        const HsVariant &V = kVariants[vi];
+        if (!V.nw) continue;
+        const int k_lo = std::min(iters, 5), k_hi = std::min(iters, V.kmax);
+        for (int n = (iters + k_hi - 1) / k_hi; n <= (iters + k_lo - 1) / k_lo; ++n) {
+            const int kk = (iters + n - 1) / n;
+            const float us = (float)n * rows_launch_us(V, H, W, kk, B);
+            if (us < best) {
+                best = us;
+                variant = vi;
+                k = kk;
+            }
+            // longer solves: the next launch count that changes k
+            if (kk > k_lo) n = std::max(n, (iters + kk - 2) / (kk - 1) - 1);
+        }
+    }
+}
+
+// Untuned sizes.  The canonical averaging stencil: a row-register variant.  Other
+// stencils: double-buffered window with the reciprocal quotient, k = 8 (the
+// fastest variant at 512^2 .. 3840x2160 in the sweeps).
+static void default_choice(int H, int W, int B, int iters, bool canonical, int &variant, int &k) {
     variant = 24;
     k = 8;
+    if (canonical) hs_rows_choice(H, W, B, std::max(iters, 1), variant, k);
 }
 
 int launch_hs_tb(int variant, const float *Ix, const float *Iy, const float *It,
@@ -383,7 +525,18 @@ int launch_hs_tb(int variant, const float *Ix, const float *Iy, const float *It,
     const int tiles_y = (H + V.th - 1) / V.th;
     a.ntiles = a.tiles_x * tiles_y;
     auto kern = V.kernel[tap_class(taps.nd)];
+    int nt = V.nt;
+    a.tw = V.tw;
+    a.th = V.th;
     if (V.ring && hs_ring_taps(taps)) kern = V.ring;
+    if (hs_runs_rows(V, taps)) {
+        const RowsGeom g = hs_rows_geom(V, H, W, k, B);
+        a.tw = g.tw;
+        a.th = g.th;
+        a.tiles_x = g.tiles_x;
+        a.ntiles = g.ntiles;
+        nt = 64 * V.nw;
+    }
     if (lt || lub) {
         // linearisation output exists only for the 1024-thread 64x32 k<=8 shape
         // (with the reciprocal quotient: the same bits as the division, fewer
@@ -404,7 +557,7 @@ int launch_hs_tb(int variant, const float *Ix, const float *Iy, const float *It,
         if (hs_ring_taps(taps) && !(staged && staged[0] == '1'))
             kern = hs_tb_kernel<1024, 64, 32, 8, 8, true, true, true, true>;
     }
-    hipLaunchKernelGGL(kern, dim3(a.ntiles, B), dim3(V.nt), 0, s, a, taps);
+    hipLaunchKernelGGL(kern, dim3(a.ntiles, B), dim3(nt), 0, s, a, taps);
     HMX_LAUNCH_CHECK("hs_tb");
     return HMX_OK;
 }
@@ -580,6 +733,7 @@ int hs_jacobi_run(const float *Ix, const float *Iy, const float *It, const float
                   float *wu, float *wv, int variant, int k, hipStream_t s, int B,
                   const float *alpha2_b, bool start_in_work) {
     if (iters <= 0) return HMX_OK;
+    k = hs_effective_k(variant, k, taps);
     if (hs_runs_persistent(variant, iters, k, B, alpha2_b))
         return hs_persist_run(Ix, Iy, It, den, alpha2, H, W, taps, iters, u, v, k, s);
     const bool odd = hs_launch_count(iters, k) & 1;
@@ -614,14 +768,16 @@ int hs_jacobi_run(const float *Ix, const float *Iy, const float *It, const float
                          s, 1, nullptr, false);
 }
 
-void hs_choice(int H, int W, int &variant, int &k) {
+// (variant, k) for iters iterations of B images of one size: the tuned choice, if
+// hs_tune ran for the size, else the default.
+void hs_choice(int H, int W, int B, int iters, const Taps &taps, int &variant, int &k) {
     std::lock_guard<std::mutex> lk(g_tune_mu);
     auto it = g_tuned.find({H, W});
     if (it != g_tuned.end()) {
         variant = it->second.first;
         k = it->second.second;
     } else {
-        default_choice(H, W, variant, k);
+        default_choice(H, W, B, iters, hs_ring_taps(taps), variant, k);
     }
 }
 
@@ -687,8 +843,13 @@ extern "C" int hmx_hs_recip_check(int e_lo, int e_hi, unsigned long long *bad, v
 
 extern "C" int hmx_hs_config(int H, int W, int *variant, int *k) {
     HMX_REQUIRE(H > 0 && W > 0, "hmx_hs_config: H and W must be positive");
+    // a long solve with the canonical averaging stencil
+    Taps avg;
+    static const float w8[8] = {0};
+    int rc = make_taps(avg, 8, w8, HS_RING_OX, HS_RING_OY);
+    if (rc) return rc;
     int vi, kk;
-    hs_choice(H, W, vi, kk);
+    hs_choice(H, W, 1, kLongSolve, avg, vi, kk);
     if (variant) *variant = vi;
     if (k) *k = kk;
     return HMX_OK;
@@ -723,7 +884,10 @@ extern "C" int hmx_hs_jacobi(const float *Ix, const float *Iy, const float *It,
                              const float *wa, const int *oxa, const int *oya, int iters,
                              float *u, float *v, float *work_u, float *work_v, void *stream) {
     int variant, k;
-    hs_choice(H, W, variant, k);
+    Taps t;
+    int rc = make_taps(t, nda, wa, oxa, oya);
+    if (rc) return rc;
+    hs_choice(H, W, 1, iters, t, variant, k);
     return hmx_hs_jacobi_cfg(Ix, Iy, It, den, alpha2, H, W, nda, wa, oxa, oya, iters, u, v,
                              work_u, work_v, variant, k, stream);
 }
@@ -783,7 +947,7 @@ extern "C" int hmx_hs_tune(const float *Ix, const float *Iy, const float *It, fl
         std::sort(cands.begin(), cands.end(),
                   [](const Cand &a, const Cand &b) { return a.ms < b.ms; });
         int dv, dk;
-        default_choice(H, W, dv, dk);
+        default_choice(H, W, 1, kLongSolve, hs_ring_taps(t), dv, dk);
         float best = 1e30f, dms = -1.0f;
         for (size_t i = 0; i < cands.size() && i < 4 && !rc; ++i) {
             float ms;
@@ -846,7 +1010,8 @@ extern "C" int hmx_hs_solve(const float *I1, const float *I2, int H, int W, floa
     float *wu = workspace + 3 * n, *wv = workspace + 4 * n;
     hipStream_t s = as_stream(stream);
     int variant, k;
-    hs_choice(H, W, variant, k);
+    hs_choice(H, W, 1, iters, av, variant, k);
+    k = hs_effective_k(variant, k, av);
     // an odd launch count starts from the work planes: the setup pass copies
     // (u, v) there as it goes (the persistent form reads u, v itself)
     const bool odd = !hs_runs_persistent(variant, iters, k, 1, nullptr) &&

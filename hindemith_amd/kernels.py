@@ -265,7 +265,8 @@ def hs_tune(Ix, Iy, It, alpha2, Avg):
 
 
 def hs_config(H, W):
-    """(variant, k) the fused Jacobi launches use for an H x W image."""
+    """(variant, k) the fused Jacobi launches of a long solve use for an H x W
+    image and the canonical averaging stencil."""
     vo, ko = ctypes.c_int(), ctypes.c_int()
     check(lib().hmx_hs_config(int(H), int(W), ctypes.byref(vo), ctypes.byref(ko)), "hs_config")
     return vo.value, ko.value
@@ -291,7 +292,8 @@ def hs_variants():
         strip = L.hmx_hs_variant_strip(i)
         out.append(dict(tile_w=tw.value, tile_h=th.value, threads=nt.value, kmax=km.value,
                         strip=strip,
-                        kernel="hs_strip_kernel" if strip > 0 else "hs_tb_kernel"))
+                        kernel="hs_strip_kernel" if strip > 0 else
+                        "hs_rows_kernel" if km.value > 8 else "hs_tb_kernel"))
     return out
 
 

@@ -226,7 +226,7 @@ int hmx_hs_setup(const float *I1, const float *I2, int H, int W,
  *     NULL (else read).  u, v are updated in place; work_u/work_v are H*W
  *     device scratch planes (ping-pong).  Avg taps must lie within radius 1.
  *     Kernel variant and iterations per launch come from the autotuner cache
- *     (hmx_hs_tune) or a size heuristic. */
+ *     (hmx_hs_tune) or a rule on the sizes and iterations. */
 int hmx_hs_jacobi(const float *Ix, const float *Iy, const float *It, const float *den,
                   float alpha2, int H, int W, int nda, const float *wa, const int *oxa,
                   const int *oya, int iters, float *u, float *v, float *work_u,
@@ -239,7 +239,10 @@ int hmx_hs_jacobi_cfg(const float *Ix, const float *Iy, const float *It, const f
                       const int *oya, int iters, float *u, float *v, float *work_u,
                       float *work_v, int variant, int k, void *stream);
 int hmx_hs_variant_count(void);
-/* Tile width/height, threads and max k of a variant. */
+/* Tile width/height, threads and max k of a variant.  (Variants whose tile follows
+ * from the image size and k with the canonical averaging stencil -- the
+ * row-register forms, max k above 8 -- report the tile of their other stencils'
+ * kernels.) */
 int hmx_hs_variant_info(int variant, int *tile_w, int *tile_h, int *threads, int *kmax);
 /* Rows per thread per column of a column-strip variant (hs_strip_kernel), 0 for a
  * rectangular-tile variant (hs_tb_kernel), or a negative HMX_ERR_* code. */
@@ -252,9 +255,10 @@ int hmx_hs_variant_strip(int variant);
  * on stream.  No counterpart in the reference: it pins the bit-exactness of
  * the quotient the reference computes with a division. */
 int hmx_hs_recip_check(int e_lo, int e_hi, unsigned long long *bad, void *stream);
-/* The (variant, k) hmx_hs_jacobi and hmx_hs_solve use for an H x W image:
- * the tuned one if hmx_hs_tune ran for that size in this process, else the
- * default.  No counterpart in the reference. */
+/* The (variant, k) hmx_hs_jacobi and hmx_hs_solve use for an H x W image, the
+ * canonical averaging stencil and a long solve: the tuned one if hmx_hs_tune ran
+ * for that size in this process, else the default (which for other stencils and
+ * for few iterations may be another).  No counterpart in the reference. */
 int hmx_hs_config(int H, int W, int *variant, int *k);
 /* Time every (variant, k) candidate on the given buffers (their contents are
  * overwritten) and cache the best for this H x W; returns the choice.  The
