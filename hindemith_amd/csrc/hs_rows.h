@@ -54,6 +54,18 @@ struct HsRowsLds {
     float2 row[NW][P > 2 ? P - 2 : 1][HS_ROWS_COLS];
 };
 
+// Derivative planes computed by a solve's first launch itself (SETUP builds): the
+// frames, the planes to write, and the weights of Dx, Dy and Dt, whose taps sit
+// at the canonical offsets (hs_cube_taps).
+struct HsSetup {
+    const float *I1, *I2;
+    float *Ix, *Iy, *It;
+    float w[12];
+};
+// the canonical derivative stencils' offsets in their tap order: Dx and Dt, Dy
+constexpr int HS_CUBE_OX[2][4] = {{0, 1, 0, 1}, {0, 0, 1, 1}};
+constexpr int HS_CUBE_OY[2][4] = {{0, 0, 1, 1}, {0, 1, 0, 1}};
+
 // a window row around one column: left neighbour, cell, right neighbour
 struct HsTri {
     float2 l, c, r;
@@ -67,9 +79,15 @@ struct HsTri {
 // more registers per row); otherwise they are read as the row is reached.
 // G: rows computed together (independent fma chains in flight, one range check).
 // LOUT: also store each step's (ubar, vbar) of the output tile (HsImage::lub).
-template <int NW, int P, bool PRE, int G, bool LOUT = false>
+// SETUP: the window's derivatives come from the frames (su), and the tile's are
+// stored for the launches that follow.  A solve then needs no setup pass: that
+// pass is one launch of latency for an image of any ordinary size (135x240 11
+// us, 480x640 14.6 us, against 11 and 20 B/px of traffic) and this is
+// 27 more VALU instructions per cell of one launch.
+template <int NW, int P, bool PRE, int G, bool LOUT = false, bool SETUP = false>
 __device__ __forceinline__ void hs_rows_tile(const HsImage &a, int txi, int tyi, int tw, int th,
-                                             int k, const float (&w)[8], HsRowsLds<NW, P> &lds) {
+                                             int k, const float (&w)[8], HsRowsLds<NW, P> &lds,
+                                             const HsSetup *su = nullptr) {
     static_assert(P >= 2, "a strip has a first and a last row");
     const int lane = threadIdx.x & 63;
     const int wave = __builtin_amdgcn_readfirstlane((int)threadIdx.x >> 6);
@@ -99,10 +117,53 @@ __device__ __forceinline__ void hs_rows_tile(const HsImage &a, int txi, int tyi,
             auto ld = [&](const char *p) { return ld_g(reinterpret_cast<const float *>(p + o)); };
             u[j] = ld(pu);
             v[j] = ld(pv);
+            if (SETUP) continue;
             cx[j] = ld(pIx);
             cy[j] = ld(pIy);
             ct[j] = ld(pIt);
             if (pd) cd[j] = ld(pd);
+        }
+        if constexpr (SETUP) {
+            // the 2 x 2 block of each cell in both frames, its right column and
+            // lower row clamped; a row is the lower row of the one above it
+            const char *const p1 = reinterpret_cast<const char *>(su->I1);
+            const char *const p2 = reinterpret_cast<const char *>(su->I2);
+            const unsigned cr1 = (unsigned)min(clampi(gx, 0, W - 1) + 1, W - 1) * 4u;
+            float f[P + 1][4];
+#pragma unroll
+            for (int j = 0; j <= P; ++j) {
+                const unsigned ro = (unsigned)min(gy0 + r0 + j, H - 1) * rowb;
+                auto ld = [&](const char *p, unsigned o) {
+                    return ld_g(reinterpret_cast<const float *>(p + o));
+                };
+                f[j][0] = ld(p1, ro + co);
+                f[j][1] = ld(p1, ro + cr1);
+                f[j][2] = ld(p2, ro + co);
+                f[j][3] = ld(p2, ro + cr1);
+            }
+#pragma unroll
+            for (int j = 0; j < P; ++j) {
+                // stencil s (0 Dx, 1 Dy, 2 Dt) of frame q: fma in tap order from 0
+                auto cube = [&](int s, int q) {
+                    float acc = 0.0f;
+#pragma unroll
+                    for (int d = 0; d < 4; ++d)
+                        acc = fmaf(su->w[4 * s + d],
+                                   f[j + HS_CUBE_OY[s & 1][d]][2 * q + HS_CUBE_OX[s & 1][d]], acc);
+                    return acc;
+                };
+                cx[j] = cube(0, 0) + cube(0, 1);
+                cy[j] = cube(1, 0) + cube(1, 1);
+                const float t2 = cube(2, 1), t1 = cube(2, 0);
+                ct[j] = t2 - t1;
+                const int gy = gy0 + r0 + j;
+                if (gx >= x0 && gx < x1 && gy >= y0 && gy < y1) {
+                    const unsigned o = (unsigned)gy * (unsigned)W + (unsigned)gx;
+                    ((gfloat *)su->Ix)[o] = cx[j];
+                    ((gfloat *)su->Iy)[o] = cy[j];
+                    ((gfloat *)su->It)[o] = ct[j];
+                }
+            }
         }
 #pragma unroll
         for (int j = 0; j < P; ++j) {
@@ -144,6 +205,14 @@ __device__ __forceinline__ void hs_rows_tile(const HsImage &a, int txi, int tyi,
             R[j] = slot(0, j)[ri];
         }
     }
+    // linearisation output: the strip's offset from the plane's start, and the
+    // strip rows in the output tile
+    const unsigned rowb = (unsigned)W * 4u;
+    unsigned lo0 = (unsigned)(gy0 + r0) * rowb + (unsigned)gx * 4u;
+    unsigned tile_rows = 0;
+    if (LOUT)
+        for (int j = 0; j < P; ++j)
+            if (gy0 + r0 + j >= y0 && gy0 + r0 + j < y1) tile_rows |= 1u << j;
     // BOT: the image's last row is in the strip and not its last row
     auto steps = [&](auto bot_c) {
         constexpr bool BOT = decltype(bot_c)::value;
@@ -156,6 +225,11 @@ __device__ __forceinline__ void hs_rows_tile(const HsImage &a, int txi, int tyi,
             // active strip rows [lo, hi): the tile grown by k - it, inside the image
             const int lo = max(y0 - (k - it), 0) - gy0 - r0;
             const int hi = min(y1 + (k - it), H) - gy0 - r0;
+            // (opaque per step: otherwise every row's output address is kept
+            // across the loop)
+            if (LOUT) asm volatile("" : "+v"(lo0));
+            const float *const lub = LOUT ? a.lub + (int64_t)(it - 1) * a.lstride : nullptr;
+            const float *const lvb = LOUT ? a.lvb + (int64_t)(it - 1) * a.lstride : nullptr;
             if (lo >= P || hi <= 0) continue;
             const float2 *const ra =
                 (gy0 + r0 == 0 || wave == 0) ? lds.edge[buf][wave][0] : lds.edge[buf][wave - 1][1];
@@ -239,14 +313,17 @@ __device__ __forceinline__ void hs_rows_tile(const HsImage &a, int txi, int tyi,
                         u[j] = ub[i] - p1;
                         v[j] = vb[i] - p2;
                         slot(buf ^ 1, j)[lane] = make_float2(u[j], v[j]);
-                        if (LOUT) {
-                            const int gy = gy0 + r0 + j;
-                            if (in && gy >= y0 && gy < y1) {
-                                const int64_t so = (int64_t)(it - 1) * a.lstride + (int64_t)gy * W;
-                                ((gfloat *)(a.lub + so))[gx] = ub[i];
-                                ((gfloat *)(a.lvb + so))[gx] = vb[i];
+                    }
+                    if (LOUT && in) {
+                        const char *const pub = reinterpret_cast<const char *>(lub);
+                        const char *const pvb = reinterpret_cast<const char *>(lvb);
+#pragma unroll
+                        for (int i = 0; i < n; ++i)
+                            if ((tile_rows >> (j0 + i)) & 1) {
+                                const unsigned o = lo0 + (unsigned)(j0 + i) * rowb;
+                                *(gfloat *)(pub + o) = ub[i];
+                                *(gfloat *)(pvb + o) = vb[i];
                             }
-                        }
                     }
                     wave_fence();
                     if (PRE) {

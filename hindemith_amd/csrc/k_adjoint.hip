@@ -28,6 +28,7 @@
 // step needs on the pixel itself -- (ubar, vbar), from which t is recomputed --
 // then walks the segment backwards.
 #include "hmx_common.h"
+#include "hs_rows.h"
 #include "hs_tile.h"
 
 #include <algorithm>
@@ -39,16 +40,18 @@
 
 namespace hmx {
 
-int launch_hs_tb(int variant, const float *Ix, const float *Iy, const float *It,
-                 const float *den, float alpha2, int H, int W, const Taps &taps, int k,
-                 const float *u_in, const float *v_in, float *u_out, float *v_out,
-                 hipStream_t s, int B, const float *alpha2_b, float *lt, float *lub,
-                 float *lvb, int64_t lstride, bool rev);
-int hs_jacobi_run(const float *Ix, const float *Iy, const float *It, const float *den,
-                  float alpha2, int H, int W, const Taps &taps, int iters, float *u, float *v,
-                  float *wu, float *wv, int variant, int k, hipStream_t s, int B,
-                  const float *alpha2_b, bool start_in_work);
-void hs_choice(int H, int W, int B, int iters, const Taps &taps, int &variant, int &k);
+int hs_sweep(const float *Ix, const float *Iy, const float *It, const float *den, float alpha2,
+             int H, int W, const Taps &taps, int iters, const float *su, const float *sv, float *du,
+             float *dv, float *tu, float *tv, int variant, int k, hipStream_t s, int B,
+             const float *alpha2_b, const HsSetup *setup);
+int hs_lin_sweep(const float *Ix, const float *Iy, const float *It, int H, int W, const Taps &taps,
+                 int iters, const float *su, const float *sv, float *du, float *dv, float *tu,
+                 float *tv, float *lin, hipStream_t s, int B, const float *alpha2_b);
+int hs_effective_k(int variant, int k, const Taps &taps);
+bool hs_can_fuse_setup(int variant, const Taps &taps);
+bool hs_cube_taps(const Taps &dx, const Taps &dy, const Taps &dt, HsSetup &su);
+void hs_choice(int H, int W, int B, int iters, bool in_place, const Taps &taps, int &variant,
+               int &k);
 
 __device__ inline void tr_range(int p, int o, int n, int &lo, int &hi) {
     lo = (p == 0) ? 0 : p - o;
@@ -555,44 +558,8 @@ static int64_t adj_tiles(int H, int W) {
     return (int64_t)((W + ADJ_TW - 1) / ADJ_TW) * ((H + ADJ_TH - 1) / ADJ_TH);
 }
 
-// Variant of the forward kernel used to recompute a checkpoint segment: it
-// writes every intermediate state of each k-step launch.
-constexpr int ADJ_RECOMPUTE_VARIANT = 3;  // 1024 threads, 64x32 tiles, k <= 8
-constexpr int ADJ_RECOMPUTE_K = 8;
-
 int launch_hs_copy2(const float *u, const float *v, float *wu, float *wv, int64_t n,
                     hipStream_t s);
-
-// len iterations from the state in (u, v) with the linearisation-output
-// launches (ADJ_RECOMPUTE_K per launch), storing iteration j's (ubar, vbar) at
-// lin + 2*j*n and + n, the state ending in (u, v): the launches ping-pong
-// through (wu, wv), the first reading (wu, wv) after a copy when their count
-// is odd.  The same launches, in the same order, as the adjoint's segment
-// recompute, so the states and the stored values are the same bits.
-static int lin_segment(const float *Ix, const float *Iy, const float *It, int H, int W,
-                       const Taps &av, int len, float *u, float *v, float *wu, float *wv,
-                       float *lin, int64_t n, hipStream_t s, int B, const float *alpha2) {
-    const int nl = (len + ADJ_RECOMPUTE_K - 1) / ADJ_RECOMPUTE_K;
-    float *su = u, *sv = v, *du = wu, *dv = wv;
-    if (nl & 1) {
-        int rc = launch_hs_copy2(u, v, wu, wv, n, s);
-        if (rc) return rc;
-        std::swap(su, du);
-        std::swap(sv, dv);
-    }
-    for (int j0 = 0; j0 < len;) {
-        const int kk = std::min(ADJ_RECOMPUTE_K, len - j0);
-        float *lub = lin + (int64_t)2 * j0 * n;
-        int rc = launch_hs_tb(ADJ_RECOMPUTE_VARIANT, Ix, Iy, It, nullptr, 0.0f, H, W, av, kk, su,
-                              sv, du, dv, s, B, alpha2, nullptr, lub, lub + n, 2 * n,
-                              (j0 / ADJ_RECOMPUTE_K) & 1);
-        if (rc) return rc;
-        std::swap(su, du);
-        std::swap(sv, dv);
-        j0 += kk;
-    }
-    return HMX_OK;
-}
 
 }  // namespace hmx
 
@@ -640,26 +607,44 @@ extern "C" int hmx_hs_forward_ckpt(const float *I1, const float *I2, int B, int 
     float *alpha2 = ws + 5 * n;
     hipLaunchKernelGGL(alpha_sq_kernel, dim3((B + 63) / 64), dim3(64), 0, s, alpha, alpha2, B);
     HMX_LAUNCH_CHECK("alpha_sq");
-    rc = setup_batch(I1, I2, B, H, W, T.dx, T.dy, T.dt, Ix, Iy, It, s);
-    if (rc) return rc;
     int variant, k;
-    hs_choice(H, W, B, std::min(iters, ckpt_every), T.av, variant, k);
+    hs_choice(H, W, B, std::min(iters, ckpt_every), false, T.av, variant, k);
+    k = hs_effective_k(variant, k, T.av);
     const int nck = hmx_hs_ckpt_count(iters, ckpt_every);
-    for (int c = 0; c < nck; ++c) {
-        float *cu = ckpt + (int64_t)(2 * c) * n, *cv = ckpt + (int64_t)(2 * c + 1) * n;
-        HMX_HIP_TRY(hipMemcpyAsync(cu, u, n * 4, hipMemcpyDeviceToDevice, s));
-        HMX_HIP_TRY(hipMemcpyAsync(cv, v, n * 4, hipMemcpyDeviceToDevice, s));
-        const int len = (iters - c * ckpt_every) < ckpt_every ? iters - c * ckpt_every : ckpt_every;
+    // the first launch does the setup, except where it is a linearisation launch
+    HsSetup su;
+    const bool fuse = nck > (lin_last ? 1 : 0) && hs_can_fuse_setup(variant, T.av) &&
+                      hs_cube_taps(T.dx, T.dy, T.dt, su);
+    if (fuse) {
+        su.I1 = I1;
+        su.I2 = I2;
+        su.Ix = Ix;
+        su.Iy = Iy;
+        su.It = It;
+    } else {
+        rc = setup_batch(I1, I2, B, H, W, T.dx, T.dy, T.dt, Ix, Iy, It, s);
+        if (rc) return rc;
+    }
+    // each segment runs from its checkpoint to the next one (the last one to u, v)
+    if (nck > 0) rc = launch_hs_copy2(u, v, ckpt, ckpt + n, n, s);
+    for (int c = 0; c < nck && !rc; ++c) {
+        const float *cu = ckpt + (int64_t)(2 * c) * n, *cv = cu + n;
+        float *du = u, *dv = v;
+        if (c + 1 < nck) {
+            du = ckpt + (int64_t)(2 * c + 2) * n;
+            dv = du + n;
+        }
+        const int len = std::min(iters - c * ckpt_every, ckpt_every);
         if (lin_last && c == nck - 1)
             // the last segment also keeps each iteration's (ubar, vbar): the
             // reverse pass then needs no recompute of it
-            rc = lin_segment(Ix, Iy, It, H, W, T.av, len, u, v, wu, wv, lin_last, n, s, B, alpha2);
+            rc = hs_lin_sweep(Ix, Iy, It, H, W, T.av, len, cu, cv, du, dv, wu, wv, lin_last, s, B,
+                              alpha2);
         else
-            rc = hs_jacobi_run(Ix, Iy, It, nullptr, 0.0f, H, W, T.av, len, u, v, wu, wv, variant,
-                               k, s, B, alpha2, false);
-        if (rc) return rc;
+            rc = hs_sweep(Ix, Iy, It, nullptr, 0.0f, H, W, T.av, len, cu, cv, du, dv, wu, wv,
+                          variant, k, s, B, alpha2, fuse && c == 0 ? &su : nullptr);
     }
-    return HMX_OK;
+    return rc;
 }
 
 extern "C" int hmx_hs_adjoint(const float *I1, const float *I2, int B, int H, int W,
@@ -742,18 +727,10 @@ extern "C" int hmx_hs_adjoint(const float *I1, const float *I2, int B, int H, in
         // the last segment's (ubar, vbar) may come from the forward pass
         const bool kept = lin_last && c == nck - 1;
         float *seg_lin = kept ? const_cast<float *>(lin_last) : lin;
-        int rcur = 0;
-        for (int j0 = 0; j0 < len && !kept;) {
-            const int kk = std::min(ADJ_RECOMPUTE_K, len - j0);
-            float *lub = lin + (int64_t)2 * j0 * n;
-            rc = launch_hs_tb(ADJ_RECOMPUTE_VARIANT, Ix, Iy, It, nullptr, 0.0f, H, W, T.av, kk,
-                              j0 == 0 ? cu : rs[rcur][0], j0 == 0 ? cv : rs[rcur][1],
-                              rs[rcur ^ 1][0], rs[rcur ^ 1][1], s, B, alpha2, nullptr, lub,
-                              lub + n, 2 * n, (j0 / ADJ_RECOMPUTE_K) & 1);
-            if (rc) return rc;
-            rcur ^= 1;
-            j0 += kk;
-        }
+        if (!kept)
+            rc = hs_lin_sweep(Ix, Iy, It, H, W, T.av, len, cu, cv, rs[0][0], rs[0][1], rs[1][0],
+                              rs[1][1], lin, s, B, alpha2);
+        if (rc) return rc;
         // reverse steps len-1 .. 0, up to ADJ_MMAX per launch
         for (int hi = len; hi > 0;) {
             const int mm = std::min(ADJ_MMAX, hi);

@@ -43,7 +43,7 @@ struct HsArgs {
     int H, W, k, tiles_x, ntiles;
     int rev;                // walk each XCD's tiles backwards (see xcd_remap)
     int64_t bstride;        // elements between consecutive pairs (blockIdx.y)
-    float *lt, *lub, *lvb;  // optional per-step linearisation output (see HsImage)
+    float *lub, *lvb;       // optional per-step linearisation output (see HsImage)
     int64_t lstride;
     int tw, th;             // output tile of the row-register kernels (hs_rows_geom)
 };
@@ -51,14 +51,12 @@ struct HsArgs {
 // The linearisation-output form (the adjoint's segment recompute) is compiled
 // for 8 waves per SIMD so its extra stores do not cost a work-group per CU.
 // DB: two LDS windows, one barrier per step (see hs_tile).
-// RING: the canonical 8 taps at compile-time LDS offsets (hs_tile); with LOUT
-// and DB, the one-barrier step storing the linearisation from registers.
 template <int NT, int TW, int TH, int KMAX, int NTAP, bool LOUT = false, bool DB = false,
-          bool FDIV = false, bool RING = false>
+          bool FDIV = false>
 __global__ __launch_bounds__(NT, LOUT ? 8 : 1) void hs_tb_kernel(HsArgs a, Taps taps) {
     using Win = HsWindow<NT, TW, TH, KMAX, DB>;
     __shared__ float2 uvm[Win::SIZE];
-    __shared__ float lin[LOUT && !DB ? 3 * TW * TH : 1];
+    __shared__ float lin[LOUT ? 2 * TW * TH : 1];
     const int64_t off = (int64_t)blockIdx.y * a.bstride;  // pair of a batch
     HsImage im;
     im.Ix = a.Ix + off;
@@ -74,20 +72,14 @@ __global__ __launch_bounds__(NT, LOUT ? 8 : 1) void hs_tb_kernel(HsArgs a, Taps 
     im.W = a.W;
     im.tiles_x = a.tiles_x;
     if (LOUT) {
-        im.lt = a.lt ? a.lt + off : nullptr;
         im.lub = a.lub + off;
         im.lvb = a.lvb + off;
         im.lstride = a.lstride;
     }
     const HsTapTable<TW + 2 * KMAX> tp(taps, NTAP);
     const int t = xcd_remap(blockIdx.x, a.ntiles, a.rev);
-    if constexpr (RING)
-        // shared tap addresses cost no registers here: one base plus constants
-        hs_tile<NT, TW, TH, KMAX, NTAP, LOUT, DB, FDIV, true, DB && !LOUT, false, true>(
-            im, t, a.k, tp, uvm + Win::PAD, nullptr);
-    else
-        hs_tile<NT, TW, TH, KMAX, NTAP, LOUT, DB, FDIV>(im, t, a.k, tp, uvm + Win::PAD,
-                                                        LOUT ? lin : nullptr);
+    hs_tile<NT, TW, TH, KMAX, NTAP, LOUT, DB, FDIV>(im, t, a.k, tp, uvm + Win::PAD,
+                                                    LOUT ? lin : nullptr);
 }
 
 // Ring-ordered form (hs_tile_ring): 64 x 32 tiles, k <= 8, double-buffered,
@@ -137,8 +129,8 @@ __global__ __launch_bounds__(NT) void hs_strip_kernel(HsArgs a, Taps taps) {
 
 // Row-register form (hs_rows.h): a window of 64 columns x NW * P rows, the canonical
 // 8-tap averaging offsets.  WPE: waves per SIMD the build is held to.
-template <int NW, int P, bool PRE, int G, int WPE, bool LOUT = false>
-__global__ __launch_bounds__(64 * NW, WPE) void hs_rows_kernel(HsArgs a, Taps taps) {
+template <int NW, int P, bool PRE, int G, bool LOUT, bool SETUP>
+__device__ __forceinline__ void hs_rows_body(const HsArgs &a, const Taps &taps, const HsSetup *su) {
     __shared__ HsRowsLds<NW, P> lds;
     const int64_t off = (int64_t)blockIdx.y * a.bstride;
     HsImage im;
@@ -158,12 +150,33 @@ __global__ __launch_bounds__(64 * NW, WPE) void hs_rows_kernel(HsArgs a, Taps ta
         im.lvb = a.lvb + off;
         im.lstride = a.lstride;
     }
+    HsSetup so;
+    if (SETUP) {
+        so = *su;
+        so.I1 += off;
+        so.I2 += off;
+        so.Ix += off;
+        so.Iy += off;
+        so.It += off;
+    }
     float w[8];
 #pragma unroll
     for (int d = 0; d < 8; ++d) w[d] = taps.w[d];
     const int t = xcd_remap(blockIdx.x, a.ntiles, a.rev);
     const int tyi = t / a.tiles_x, txi = t - tyi * a.tiles_x;
-    hs_rows_tile<NW, P, PRE, G, LOUT>(im, txi, tyi, a.tw, a.th, a.k, w, lds);
+    hs_rows_tile<NW, P, PRE, G, LOUT, SETUP>(im, txi, tyi, a.tw, a.th, a.k, w, lds, &so);
+}
+
+template <int NW, int P, bool PRE, int G, int WPE, bool LOUT = false>
+__global__ __launch_bounds__(64 * NW, WPE) void hs_rows_kernel(HsArgs a, Taps taps) {
+    hs_rows_body<NW, P, PRE, G, LOUT, false>(a, taps, nullptr);
+}
+
+// a solve's first launch, computing the derivative planes as well (HsSetup)
+template <int NW, int P, bool PRE, int G, int WPE>
+__global__ __launch_bounds__(64 * NW, WPE) void hs_rows_first_kernel(HsArgs a, Taps taps,
+                                                                     HsSetup su) {
+    hs_rows_body<NW, P, PRE, G, false, true>(a, taps, &su);
 }
 
 // ---------------------------------------------------------------------------
@@ -288,6 +301,8 @@ struct HsVariant {
     // takes.  Zero for the others.
     int nw, rows, wgs;
     float us0, us_row;
+    void (*first)(HsArgs, Taps, HsSetup);  // a solve's first launch, with its setup
+    void (*lin)(HsArgs, Taps);             // with the linearisation output, or null
 };
 
 // tap count -> kernel slot (straight-line kernels for the common stencils)
@@ -327,14 +342,15 @@ static int tap_class(int nd) {
       hs_strip_kernel<NT, TW, TH, K, S, 8>, hs_strip_kernel<NT, TW, TH, K, S, 9>,      \
       hs_strip_kernel<NT, TW, TH, K, S, 0>}, nullptr}
 // row-register forms: the canonical stencil's kernel, and variant 24's for others
-#define HS_R(NW, P, PRE, G, WPE, WGS, KMAX, US0, USROW)                                 \
+#define HS_R(NW, P, PRE, G, WPE, WGS, KMAX, US0, USROW, LIN)                            \
     {1024, 64, 32, KMAX, 0,                                                             \
      {hs_tb_kernel<1024, 64, 32, 8, 4, false, true, true>,                              \
       hs_tb_kernel<1024, 64, 32, 8, 5, false, true, true>,                              \
       hs_tb_kernel<1024, 64, 32, 8, 8, false, true, true>,                              \
       hs_tb_kernel<1024, 64, 32, 8, 9, false, true, true>,                              \
       hs_tb_kernel<1024, 64, 32, 8, 0, false, true, true>},                             \
-     hs_rows_kernel<NW, P, PRE, G, WPE>, false, NW, P, WGS, US0, USROW}
+     hs_rows_kernel<NW, P, PRE, G, WPE>, false, NW, P, WGS, US0, USROW,                 \
+     hs_rows_first_kernel<NW, P, PRE, G, WPE>, LIN}
 static const HsVariant kVariants[] = {
     HS_V(256, 64, 16, 1),     // 0: one iteration per launch (plain sweep)
     HS_V(256, 64, 32, 4),     // 1
@@ -387,15 +403,23 @@ static const HsVariant kVariants[] = {
     // height sets how many pixels a CU takes (neighbours prefetched; 56 to 110
     // VGPRs).  Two work-groups per CU for larger images, so that one's loads
     // and barriers overlap the other's steps: 8 waves at up to 128 VGPRs, or 16 at
-    // 61 (one row at a time).
-    HS_R(16, 2, true, 2, 4, 1, 12, 4.39f, 0.0183f),   // 29: window 64 x 32
-    HS_R(16, 3, true, 3, 4, 1, 16, 3.22f, 0.0422f),   // 30: 64 x 48
-    HS_R(16, 4, true, 4, 4, 1, 16, 3.09f, 0.0437f),   // 31: 64 x 64
-    HS_R(16, 5, true, 5, 4, 1, 16, 2.89f, 0.0445f),   // 32: 64 x 80
-    HS_R(8, 7, false, 4, 4, 2, 16, 6.22f, 0.0077f),   // 33: 64 x 56
-    HS_R(8, 9, false, 3, 4, 2, 16, 7.28f, 0.0092f),   // 34: 64 x 72
-    HS_R(8, 10, false, 2, 4, 2, 16, 8.32f, 0.0099f),  // 35: 64 x 80
-    HS_R(16, 4, false, 1, 8, 2, 16, 5.80f, 0.0201f),  // 36: 64 x 64
+    // 61 (one row at a time; its linearisation build would spill).
+    HS_R(16, 2, true, 2, 4, 1, 12, 4.39f, 0.0183f,
+         (hs_rows_kernel<16, 2, true, 2, 4, true>)),   // 29: window 64 x 32
+    HS_R(16, 3, true, 3, 4, 1, 16, 3.22f, 0.0422f,
+         (hs_rows_kernel<16, 3, true, 3, 4, true>)),   // 30: 64 x 48
+    HS_R(16, 4, true, 4, 4, 1, 16, 3.09f, 0.0437f,
+         (hs_rows_kernel<16, 4, true, 4, 4, true>)),   // 31: 64 x 64
+    HS_R(16, 5, true, 5, 4, 1, 16, 2.89f, 0.0445f,
+         (hs_rows_kernel<16, 5, true, 5, 4, true>)),   // 32: 64 x 80
+    HS_R(8, 7, false, 4, 4, 2, 16, 6.22f, 0.0077f,
+         (hs_rows_kernel<8, 7, false, 4, 4, true>)),   // 33: 64 x 56
+    HS_R(8, 9, false, 3, 4, 2, 16, 7.28f, 0.0092f,
+         (hs_rows_kernel<8, 9, false, 3, 4, true>)),   // 34: 64 x 72
+    HS_R(8, 10, false, 2, 4, 2, 16, 8.32f, 0.0099f,
+         (hs_rows_kernel<8, 10, false, 2, 4, true>)),  // 35: 64 x 80
+    HS_R(16, 4, false, 1, 8, 2, 16, 5.80f, 0.0201f,
+         nullptr),  // 36: 64 x 64
 };
 #undef HS_R
 #undef HS_V
@@ -415,9 +439,29 @@ static bool hs_runs_rows(const HsVariant &V, const Taps &taps) {
     return V.nw > 0 && hs_ring_taps(taps);
 }
 
+// Whether a solve's first launch can compute the derivative planes (V.first).
+bool hs_can_fuse_setup(int variant, const Taps &taps) {
+    return hs_runs_rows(kVariants[variant], taps);
+}
+
+// Whether (dx, dy, dt) have the canonical derivative stencils' offsets, in their
+// tap order; fills su's weights.
+bool hs_cube_taps(const Taps &dx, const Taps &dy, const Taps &dt, HsSetup &su) {
+    const Taps *const t[3] = {&dx, &dy, &dt};
+    for (int q = 0; q < 3; ++q) {
+        if (t[q]->nd != 4) return false;
+        for (int d = 0; d < 4; ++d) {
+            if (t[q]->ox[d] != HS_CUBE_OX[q & 1][d] || t[q]->oy[d] != HS_CUBE_OY[q & 1][d])
+                return false;
+            su.w[4 * q + d] = t[q]->w[d];
+        }
+    }
+    return true;
+}
+
 // Iterations per launch as the launches of a solve take them: a row-register
 // variant's other stencils run variant 24's kernels, 8 at most.
-static int hs_effective_k(int variant, int k, const Taps &taps) {
+int hs_effective_k(int variant, int k, const Taps &taps) {
     const HsVariant &V = kVariants[variant];
     return V.nw > 0 && !hs_ring_taps(taps) ? std::min(k, 8) : k;
 }
@@ -465,22 +509,27 @@ static float rows_launch_us(const HsVariant &V, int H, int W, int k, int B) {
 
 // The row-register variant and iterations per launch with the least cost for
 // iters iterations of B images (the iterations split evenly over the launches).
-static void hs_rows_choice(int H, int W, int B, int iters, int &variant, int &k) {
+// in_place: the sweep ends in the planes it starts from, so an odd launch count
+// costs a copy of the start state (16 B per pixel and a launch).  lin: of the
+// variants with a linearisation build.
+static void hs_rows_choice(int H, int W, int B, int iters, bool in_place, bool lin, int &variant,
+                           int &k) {
     float best = 1e30f;
+    const float copy_us = in_place ? 3.0f + 16e-6f / 4.0f * (float)H * (float)W * (float)B : 0.0f;
     for (int vi = 0; vi < kNumVariants; ++vi) {
         const HsVariant &V = kVariants[vi];
-        if (!V.nw) continue;
+        if (!V.nw || (lin && !V.lin)) continue;
         const int k_lo = std::min(iters, 5), k_hi = std::min(iters, V.kmax);
         for (int n = (iters + k_hi - 1) / k_hi; n <= (iters + k_lo - 1) / k_lo; ++n) {
             const int kk = (iters + n - 1) / n;
-            const float us = (float)n * rows_launch_us(V, H, W, kk, B);
+            const float us = (float)n * rows_launch_us(V, H, W, kk, B) + (n & 1 ? copy_us : 0.0f);
             if (us < best) {
                 best = us;
                 variant = vi;
                 k = kk;
             }
-            // longer solves: the next launch count that changes k
-            if (kk > k_lo) n = std::max(n, (iters + kk - 2) / (kk - 1) - 1);
+            // longer solves: the next launch counts (an even and an odd one) that change k
+            if (kk > k_lo && (n & 1) == 0) n = std::max(n, (iters + kk - 2) / (kk - 1) - 2);
         }
     }
 }
@@ -488,23 +537,23 @@ static void hs_rows_choice(int H, int W, int B, int iters, int &variant, int &k)
 // Untuned sizes.  The canonical averaging stencil: a row-register variant.  Other
 // stencils: double-buffered window with the reciprocal quotient, k = 8 (the
 // fastest variant at 512^2 .. 3840x2160 in the sweeps).
-static void default_choice(int H, int W, int B, int iters, bool canonical, int &variant, int &k) {
+static void default_choice(int H, int W, int B, int iters, bool in_place, bool canonical,
+                           int &variant, int &k) {
     variant = 24;
     k = 8;
-    if (canonical) hs_rows_choice(H, W, B, std::max(iters, 1), variant, k);
+    if (canonical) hs_rows_choice(H, W, B, std::max(iters, 1), in_place, false, variant, k);
 }
 
 int launch_hs_tb(int variant, const float *Ix, const float *Iy, const float *It,
                  const float *den, float alpha2, int H, int W, const Taps &taps, int k,
                  const float *u_in, const float *v_in, float *u_out, float *v_out,
                  hipStream_t s, int B = 1, const float *alpha2_b = nullptr,
-                 float *lt = nullptr, float *lub = nullptr, float *lvb = nullptr,
-                 int64_t lstride = 0, bool rev = false) {
+                 float *lub = nullptr, float *lvb = nullptr, int64_t lstride = 0,
+                 bool rev = false, const HsSetup *setup = nullptr) {
     const HsVariant &V = kVariants[variant];
     HsArgs a;
     a.rev = rev ? 1 : 0;
     a.alpha2_b = alpha2_b;
-    a.lt = lt;
     a.lub = lub;
     a.lvb = lvb;
     a.lstride = lstride;
@@ -537,27 +586,27 @@ int launch_hs_tb(int variant, const float *Ix, const float *Iy, const float *It,
         a.ntiles = g.ntiles;
         nt = 64 * V.nw;
     }
-    if (lt || lub) {
-        // linearisation output exists only for the 1024-thread 64x32 k<=8 shape
-        // (with the reciprocal quotient: the same bits as the division, fewer
-        // VALU per step; 59 VGPRs at most, within the 8 waves per SIMD)
+    if (lub && hs_runs_rows(V, taps)) {
+        kern = V.lin;
+    } else if (lub) {
+        // other linearisation outputs exist only for the 1024-thread 64x32 k<=8
+        // shape (with the reciprocal quotient: the same bits as the division,
+        // fewer VALU per step; 59 VGPRs at most, within the 8 waves per SIMD)
         static void (*const kLinKernels[5])(HsArgs, Taps) = {
             hs_tb_kernel<1024, 64, 32, 8, 4, true, false, true>,
             hs_tb_kernel<1024, 64, 32, 8, 5, true, false, true>,
             hs_tb_kernel<1024, 64, 32, 8, 8, true, false, true>,
             hs_tb_kernel<1024, 64, 32, 8, 9, true, false, true>,
             hs_tb_kernel<1024, 64, 32, 8, 0, true, false, true>};
-        if (V.strip || V.nt != 1024 || V.tw != 64 || V.th != 32 || V.kmax != 8)
+        if (V.strip || V.nt != 1024 || V.tw != 64 || V.th != 32 || V.nw || V.kmax != 8)
             return fail(HMX_ERR_UNSUPPORTED,
                         "hs_tb: linearisation output needs the 1024x64x32x8 variant");
         kern = kLinKernels[tap_class(taps.nd)];
-        // the canonical stencil: one barrier per step, the linearisation
-        // stored from registers (HMX_LIN_STAGED=1 keeps the staged form)
-        const char *staged = std::getenv("HMX_LIN_STAGED");
-        if (hs_ring_taps(taps) && !(staged && staged[0] == '1'))
-            kern = hs_tb_kernel<1024, 64, 32, 8, 8, true, true, true, true>;
     }
-    hipLaunchKernelGGL(kern, dim3(a.ntiles, B), dim3(nt), 0, s, a, taps);
+    if (setup)
+        hipLaunchKernelGGL(V.first, dim3(a.ntiles, B), dim3(nt), 0, s, a, taps, *setup);
+    else
+        hipLaunchKernelGGL(kern, dim3(a.ntiles, B), dim3(nt), 0, s, a, taps);
     HMX_LAUNCH_CHECK("hs_tb");
     return HMX_OK;
 }
@@ -595,11 +644,6 @@ int launch_hs_copy2(const float *u, const float *v, float *wu, float *wv, int64_
 // Launches of a solve of iters iterations at k per launch.
 int hs_launch_count(int iters, int k) { return iters <= 0 ? 0 : (iters + k - 1) / k; }
 
-// iters Jacobi steps, ping-ponging between (u,v) and (wu,wv); the result ends
-// in (u,v).  Launches alternate direction, so with an odd launch count the
-// start state is first copied into (wu,wv) (one pass over both planes) and
-// the first launch reads it from there; start_in_work: the caller has already
-// put the start state there (hmx_hs_solve's setup does it in the same pass).
 // Uncached ping-pong planes and tile counters of the persistent form, one set
 // per device, grown on demand.  Uncached memory is never freed: a buffer
 // freed after a kernel has read it has corrupted later allocations on this
@@ -728,56 +772,99 @@ static int hs_persist_run(const float *Ix, const float *Iy, const float *It, con
     return HMX_OK;
 }
 
+// iters Jacobi steps from the state (su, sv) to (du, dv), k per launch: launches
+// alternate between (du, dv) and the scratch planes (tu, tv) so that the last one
+// writes (du, dv).  The state must not be in the planes the first launch
+// writes: (tu, tv) for an even launch count, (du, dv) for an odd one.  setup
+// (row-register variants): the first launch computes the derivative planes too.
+int hs_sweep(const float *Ix, const float *Iy, const float *It, const float *den, float alpha2,
+             int H, int W, const Taps &taps, int iters, const float *su, const float *sv, float *du,
+             float *dv, float *tu, float *tv, int variant, int k, hipStream_t s, int B,
+             const float *alpha2_b, const HsSetup *setup) {
+    const int n = hs_launch_count(iters, k);
+    for (int i = 0; i < n; ++i) {
+        const int kk = std::min(k, iters - i * k);
+        const bool to_dst = ((n - 1 - i) & 1) == 0;
+        float *const ou = to_dst ? du : tu, *const ov = to_dst ? dv : tv;
+        // alternate launches walk the tiles backwards (xcd_remap)
+        int rc = launch_hs_tb(variant, Ix, Iy, It, den, alpha2, H, W, taps, kk, su, sv, ou, ov, s,
+                              B, alpha2_b, nullptr, nullptr, 0, i & 1,
+                              i == 0 ? setup : nullptr);
+        if (rc) return rc;
+        su = ou;
+        sv = ov;
+    }
+    return HMX_OK;
+}
+
+// As hs_sweep for the adjoint's segments: every step also stores what it linearises
+// about, step j's (ubar, vbar) at lin + 2*j*plane and one plane further (plane =
+// the B images' pixels).  The canonical averaging stencil takes the row-register
+// launches (52 -> 38 us per 8 steps of 8 x 512 x 512); other stencils, and
+// HMX_LIN_STAGED=1, the two-barrier tile that stages them through LDS.
+int hs_lin_sweep(const float *Ix, const float *Iy, const float *It, int H, int W, const Taps &taps,
+                 int iters, const float *su, const float *sv, float *du, float *dv, float *tu,
+                 float *tv, float *lin, hipStream_t s, int B, const float *alpha2_b) {
+    int variant = 3, k = 8;  // 1024 threads, 64x32 tiles
+    const char *staged = std::getenv("HMX_LIN_STAGED");
+    if (hs_ring_taps(taps) && !(staged && staged[0] == '1'))
+        hs_rows_choice(H, W, B, iters, false, true, variant, k);
+    const int64_t plane = (int64_t)B * H * W;
+    const int n = hs_launch_count(iters, k);
+    for (int i = 0; i < n; ++i) {
+        const int kk = std::min(k, iters - i * k);
+        const bool to_dst = ((n - 1 - i) & 1) == 0;
+        float *const ou = to_dst ? du : tu, *const ov = to_dst ? dv : tv;
+        float *const lub = lin + (int64_t)2 * i * k * plane;
+        int rc = launch_hs_tb(variant, Ix, Iy, It, nullptr, 0.0f, H, W, taps, kk, su, sv, ou, ov,
+                              s, B, alpha2_b, lub, lub + plane, 2 * plane, i & 1);
+        if (rc) return rc;
+        su = ou;
+        sv = ov;
+    }
+    return HMX_OK;
+}
+
+// iters Jacobi steps in place: the state starts and ends in (u, v), with
+// (wu, wv) as scratch.  With an odd launch count the start state is first
+// copied into (wu, wv) (one pass over both planes) and the first launch reads
+// it from there; start_in_work: the caller has already put it there
+// (hmx_hs_solve's setup does it in the same pass).  setup: see hs_sweep.
 int hs_jacobi_run(const float *Ix, const float *Iy, const float *It, const float *den,
                   float alpha2, int H, int W, const Taps &taps, int iters, float *u, float *v,
                   float *wu, float *wv, int variant, int k, hipStream_t s, int B,
-                  const float *alpha2_b, bool start_in_work) {
+                  const float *alpha2_b, bool start_in_work, const HsSetup *setup) {
     if (iters <= 0) return HMX_OK;
     k = hs_effective_k(variant, k, taps);
     if (hs_runs_persistent(variant, iters, k, B, alpha2_b))
         return hs_persist_run(Ix, Iy, It, den, alpha2, H, W, taps, iters, u, v, k, s);
     const bool odd = hs_launch_count(iters, k) & 1;
-    float *src_u = u, *src_v = v, *dst_u = wu, *dst_v = wv;
-    if (odd) {
-        if (!start_in_work) {
-            int rc = launch_hs_copy2(u, v, wu, wv, (int64_t)H * W * B, s);
-            if (rc) return rc;
-        }
-        std::swap(src_u, dst_u);
-        std::swap(src_v, dst_v);
-    }
-    int done = 0;
-    bool rev = false;  // alternate launches walk the tiles backwards (xcd_remap)
-    while (done < iters) {
-        const int kk = (iters - done) < k ? (iters - done) : k;
-        int rc = launch_hs_tb(variant, Ix, Iy, It, den, alpha2, H, W, taps, kk, src_u, src_v,
-                              dst_u, dst_v, s, B, alpha2_b, nullptr, nullptr, nullptr, 0, rev);
-        rev = !rev;
+    if (odd && !start_in_work) {
+        int rc = launch_hs_copy2(u, v, wu, wv, (int64_t)H * W * B, s);
         if (rc) return rc;
-        std::swap(src_u, dst_u);
-        std::swap(src_v, dst_v);
-        done += kk;
     }
-    return HMX_OK;
+    return hs_sweep(Ix, Iy, It, den, alpha2, H, W, taps, iters, odd ? wu : u, odd ? wv : v, u, v, wu,
+                    wv, variant, k, s, B, alpha2_b, setup);
 }
 
 int hs_jacobi_run(const float *Ix, const float *Iy, const float *It, const float *den,
                   float alpha2, int H, int W, const Taps &taps, int iters, float *u, float *v,
                   float *wu, float *wv, int variant, int k, hipStream_t s) {
     return hs_jacobi_run(Ix, Iy, It, den, alpha2, H, W, taps, iters, u, v, wu, wv, variant, k,
-                         s, 1, nullptr, false);
+                         s, 1, nullptr, false, nullptr);
 }
 
 // (variant, k) for iters iterations of B images of one size: the tuned choice, if
 // hs_tune ran for the size, else the default.
-void hs_choice(int H, int W, int B, int iters, const Taps &taps, int &variant, int &k) {
+void hs_choice(int H, int W, int B, int iters, bool in_place, const Taps &taps, int &variant,
+               int &k) {
     std::lock_guard<std::mutex> lk(g_tune_mu);
     auto it = g_tuned.find({H, W});
     if (it != g_tuned.end()) {
         variant = it->second.first;
         k = it->second.second;
     } else {
-        default_choice(H, W, B, iters, hs_ring_taps(taps), variant, k);
+        default_choice(H, W, B, iters, in_place, hs_ring_taps(taps), variant, k);
     }
 }
 
@@ -849,7 +936,7 @@ extern "C" int hmx_hs_config(int H, int W, int *variant, int *k) {
     int rc = make_taps(avg, 8, w8, HS_RING_OX, HS_RING_OY);
     if (rc) return rc;
     int vi, kk;
-    hs_choice(H, W, 1, kLongSolve, avg, vi, kk);
+    hs_choice(H, W, 1, kLongSolve, true, avg, vi, kk);
     if (variant) *variant = vi;
     if (k) *k = kk;
     return HMX_OK;
@@ -887,7 +974,7 @@ extern "C" int hmx_hs_jacobi(const float *Ix, const float *Iy, const float *It,
     Taps t;
     int rc = make_taps(t, nda, wa, oxa, oya);
     if (rc) return rc;
-    hs_choice(H, W, 1, iters, t, variant, k);
+    hs_choice(H, W, 1, iters, true, t, variant, k);
     return hmx_hs_jacobi_cfg(Ix, Iy, It, den, alpha2, H, W, nda, wa, oxa, oya, iters, u, v,
                              work_u, work_v, variant, k, stream);
 }
@@ -947,7 +1034,7 @@ extern "C" int hmx_hs_tune(const float *Ix, const float *Iy, const float *It, fl
         std::sort(cands.begin(), cands.end(),
                   [](const Cand &a, const Cand &b) { return a.ms < b.ms; });
         int dv, dk;
-        default_choice(H, W, 1, kLongSolve, hs_ring_taps(t), dv, dk);
+        default_choice(H, W, 1, kLongSolve, true, hs_ring_taps(t), dv, dk);
         float best = 1e30f, dms = -1.0f;
         for (size_t i = 0; i < cands.size() && i < 4 && !rc; ++i) {
             float ms;
@@ -1010,8 +1097,19 @@ extern "C" int hmx_hs_solve(const float *I1, const float *I2, int H, int W, floa
     float *wu = workspace + 3 * n, *wv = workspace + 4 * n;
     hipStream_t s = as_stream(stream);
     int variant, k;
-    hs_choice(H, W, 1, iters, av, variant, k);
+    hs_choice(H, W, 1, iters, true, av, variant, k);
     k = hs_effective_k(variant, k, av);
+    // the canonical stencils: the first row-register launch does the setup
+    HsSetup su;
+    if (iters > 0 && hs_can_fuse_setup(variant, av) && hs_cube_taps(dx, dy, dt, su)) {
+        su.I1 = I1;
+        su.I2 = I2;
+        su.Ix = Ix;
+        su.Iy = Iy;
+        su.It = It;
+        return hs_jacobi_run(Ix, Iy, It, nullptr, alpha2, H, W, av, iters, u, v, wu, wv, variant,
+                             k, s, 1, nullptr, false, &su);
+    }
     // an odd launch count starts from the work planes: the setup pass copies
     // (u, v) there as it goes (the persistent form reads u, v itself)
     const bool odd = !hs_runs_persistent(variant, iters, k, 1, nullptr) &&
@@ -1020,5 +1118,5 @@ extern "C" int hmx_hs_solve(const float *I1, const float *I2, int H, int W, floa
                          odd ? v : nullptr, wu, wv);
     if (rc) return rc;
     return hs_jacobi_run(Ix, Iy, It, nullptr, alpha2, H, W, av, iters, u, v, wu, wv, variant, k,
-                         s, 1, nullptr, odd);
+                         s, 1, nullptr, odd, nullptr);
 }

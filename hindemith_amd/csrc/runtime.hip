@@ -40,7 +40,8 @@ int launch_csr(int M, int64_t nnz, const int *indptr, const int *indices, const 
 int hs_jacobi_run(const float *Ix, const float *Iy, const float *It, const float *den,
                   float alpha2, int H, int W, const Taps &taps, int iters, float *u, float *v,
                   float *wu, float *wv, int variant, int k, hipStream_t s);
-void hs_choice(int H, int W, int B, int iters, const Taps &taps, int &variant, int &k);
+void hs_choice(int H, int W, int B, int iters, bool in_place, const Taps &taps, int &variant,
+               int &k);
 int launch_hs_precond(const float *diag0, const float *diag1, const float *offdiag,
                       const float *x0, const float *x1, float *y0, float *y1, int H, int W,
                       const float *w_dev, float w_val, hipStream_t s);
@@ -1357,7 +1358,7 @@ static int exec_node(Record &R, Node &n) {
                 return rc;
             }
             int variant, k;
-            hs_choice(U.H, U.W, 1, n.ub, t, variant, k);
+            hs_choice(U.H, U.W, 1, n.ub, true, t, variant, k);
             const int64_t np = (int64_t)U.H * U.W;
             return hs_jacobi_run(R.syms[n.syms[2]].cur_buf(), R.syms[n.syms[3]].cur_buf(),
                                  R.syms[n.syms[4]].cur_buf(), R.syms[n.syms[5]].cur_buf(), 0.0f,
