@@ -3,12 +3,14 @@
 ``horn_schunck(I1, I2, alpha, iters=200, ckpt_every=20)`` takes B x H x W
 frame stacks and per-pair ``alpha`` (B,) on the GPU and returns the flow
 ``(u, v)``.  The forward pass runs the fused, temporally blocked Jacobi kernel
-and keeps the state every ``ckpt_every`` iterations; the backward pass
-(hand-written adjoint kernel, libhmx ``hmx_hs_adjoint``) recomputes one
-segment at a time and walks it backwards, so memory is
-(iters/ckpt_every + ckpt_every) state pairs instead of iters.  The forward
-keeps the last segment's linearisation (up to ckpt_every more pairs of
-planes), so the backward recomputes every segment but that one.
+and keeps the state every ``ckpt_every`` iterations (every 8 for the canonical
+averaging stencil, where that takes no more memory); the backward pass
+(hand-written adjoint kernels, libhmx ``hmx_hs_adjoint``) recomputes one segment
+at a time and walks it backwards, so memory is at most
+(iters/ckpt_every + ckpt_every) state pairs instead of iters.  For stencils
+other than the canonical one the forward keeps the last segment's linearisation
+(up to ckpt_every more pairs of planes), so the backward recomputes every
+segment but that one.
 Gradients flow to I1, I2, alpha and, when given, the initial flow u0, v0.
 """
 from __future__ import annotations
@@ -36,6 +38,24 @@ def _tap_args(taps):
     return ts, args
 
 
+_RING_OX = (-1, 1, 0, 0, -1, 1, -1, 1)
+_RING_OY = (0, 0, -1, 1, -1, -1, 1, 1)
+_BLOCK = 8  # steps a fused reverse block takes
+
+
+def _canonical(avg):
+    t = _Taps(avg)
+    return tuple(t.ox.tolist()) == _RING_OX and tuple(t.oy.tolist()) == _RING_OY
+
+
+def _segment(iters, every):
+    """Checkpoint interval of the canonical stencil's passes.  Its backward works in
+    blocks of 8 steps from the state before each: a checkpoint per block saves it
+    the recompute of those states, where that keeps no more pairs of planes than
+    one checkpoint per interval and one pair per step of an interval would."""
+    return _BLOCK if -(-iters // _BLOCK) <= -(-iters // every) + every else every
+
+
 class HornSchunckFunction(torch.autograd.Function):
     @staticmethod
     def forward(ctx, I1, I2, alpha, u0, v0, iters, ckpt_every, taps):
@@ -47,29 +67,34 @@ class HornSchunckFunction(torch.autograd.Function):
         u = torch.zeros_like(I1) if u0 is None else _dev(u0, "u0").clone()
         v = torch.zeros_like(I1) if v0 is None else _dev(v0, "v0").clone()
         L = lib()
-        nck = L.hmx_hs_ckpt_count(int(iters), int(ckpt_every))
+        iters, ckpt_every = int(iters), int(ckpt_every)
+        want = any(ctx.needs_input_grad[:5]) and iters > 0
+        fused = _canonical(taps["Avg"]) and ckpt_every > 0
+        if fused and want:
+            ckpt_every = _segment(iters, ckpt_every)
+        nck = L.hmx_hs_ckpt_count(iters, ckpt_every)
         ckpt = torch.empty((max(nck, 1), 2, B, H, W), device=I1.device, dtype=torch.float32)
         ws = torch.empty(int(L.hmx_hs_forward_workspace(B, H, W)) // 4 + 1, device=I1.device,
                          dtype=torch.float32)
         keep, targs = _tap_args(taps)
-        # With a gradient to come, the forward also keeps its last checkpoint
-        # segment's linearisation (the backward then recomputes one segment
-        # fewer) and its derivative planes (in ws); the gradients are the same
-        # bits as without them.
-        want = any(ctx.needs_input_grad[:5]) and int(iters) > 0
-        last = int(iters) - (nck - 1) * int(ckpt_every) if want else 0
+        # With a gradient to come, the forward also keeps its derivative planes (in
+        # ws) and, for a stencil whose backward recomputes whole segments, its last
+        # checkpoint segment's linearisation (the backward then recomputes one
+        # segment fewer); the gradients are the same bits as without them.
+        last = iters - (nck - 1) * ckpt_every if want else 0
         lin = (torch.empty((2 * last, B, H, W), device=I1.device, dtype=torch.float32)
-               if want else None)
+               if want and not fused else None)
         check(L.hmx_hs_forward_ckpt(_ptr(I1), _ptr(I2), B, H, W, _ptr(alpha), *targs,
-                                    int(iters), int(ckpt_every), _ptr(u), _ptr(v), _ptr(ckpt),
+                                    iters, ckpt_every, _ptr(u), _ptr(v), _ptr(ckpt),
                                     _ptr(lin) if lin is not None else ctypes.c_void_p(0),
                                     _ptr(ws), stream_ptr()), "hs_forward_ckpt")
         if lin is None:
             lin = torch.empty(0, device=I1.device)
         ctx.save_for_backward(I1, I2, alpha, ckpt, lin, ws)
-        ctx.iters, ctx.ckpt_every, ctx.taps = int(iters), int(ckpt_every), taps
+        ctx.iters, ctx.ckpt_every, ctx.taps = iters, ckpt_every, taps
         ctx.has_u0 = u0 is not None
         ctx.kept = want
+        ctx.lin = want and not fused
         return u, v
 
     @staticmethod
@@ -89,7 +114,7 @@ class HornSchunckFunction(torch.autograd.Function):
         keep, targs = _tap_args(ctx.taps)
         null = ctypes.c_void_p(0)
         check(L.hmx_hs_adjoint(_ptr(I1), _ptr(I2), B, H, W, _ptr(alpha), *targs, ctx.iters,
-                               ctx.ckpt_every, _ptr(ckpt), _ptr(lin) if ctx.kept else null,
+                               ctx.ckpt_every, _ptr(ckpt), _ptr(lin) if ctx.lin else null,
                                _ptr(fws) if ctx.kept else null, _ptr(gu), _ptr(gv), _ptr(gI1),
                                _ptr(gI2), _ptr(ga), _ptr(gu0) if gu0 is not None else null,
                                _ptr(gv0) if gv0 is not None else null, _ptr(ws), stream_ptr()),

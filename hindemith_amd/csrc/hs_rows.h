@@ -34,6 +34,7 @@
 // chain, NaN propagating); a lane that fails it divides all of them.
 #pragma once
 
+#include <algorithm>
 #include <type_traits>
 
 #include "hmx_common.h"
@@ -45,6 +46,33 @@
 namespace hmx {
 
 constexpr int HS_ROWS_COLS = 64;  // window columns: one per lane
+
+// Tile grid of a row-register launch of k steps of B images (windows of win rows, wgs
+// work-groups per CU): as few columns and rows of
+// tiles as the window allows, then as many rows of tiles as the same number of
+// rounds of work-groups takes, each shorter: a round lasts as long as one tile,
+// so 3600 tiles on 512 places (8 rounds, the last of 16 tiles) cost 8 rounds
+// of 48 rows and 4080 tiles cost 8 of 43 (3840x2160: 107 and 98 us).
+struct RowsGeom {
+    int tw, th, tiles_x, ntiles;  // ntiles: of one image
+};
+constexpr int kCus = 256;
+inline RowsGeom hs_rows_geom(int win, int wgs, int H, int W, int k, int B) {
+    RowsGeom g;
+    const int mw = HS_ROWS_COLS - 2 * k, mh = win - 2 * k;
+    int nx = (W + mw - 1) / mw;
+    g.tw = (W + nx - 1) / nx;
+    nx = (W + g.tw - 1) / g.tw;
+    int ny = (H + mh - 1) / mh;
+    const int64_t slots = (int64_t)wgs * kCus, col = (int64_t)nx * B;
+    const int64_t rounds = (col * ny + slots - 1) / slots;
+    ny = (int)std::max<int64_t>(ny, std::min<int64_t>(rounds * slots / col, H));
+    g.th = (H + ny - 1) / ny;
+    ny = (H + g.th - 1) / g.th;
+    g.tiles_x = nx;
+    g.ntiles = nx * ny;
+    return g;
+}
 
 // LDS of one work-group: the first and last row of every wave's strip, double
 // buffered (another wave reads them), and its other rows (read by the wave alone).

@@ -28,6 +28,7 @@
 // step needs on the pixel itself -- (ubar, vbar), from which t is recomputed --
 // then walks the segment backwards.
 #include "hmx_common.h"
+#include "hs_adj_rows.h"
 #include "hs_rows.h"
 #include "hs_tile.h"
 
@@ -139,14 +140,10 @@ __device__ __forceinline__ float adj_recip(float d) {
 // offset is a constant.
 // NTAP > 0: the averaging stencil has exactly NTAP taps (straight-line
 // gather, its reads issued in groups of four so the latency of a group is
-// paid once); 0: any count up to HS_MAX_TAPS.  RING: the 8 taps sit at the
-// canonical offsets HS_RING_OX/OY in that order (weights at run time), so
-// every tap of a gather is a constant LDS offset from the cell's own address:
-// no address arithmetic per tap.  Same arithmetic in the same order either
-// way.
-template <int NT, int TW, int TH, int MMAX, int NTAP, bool RING>
+// paid once); 0: any count up to HS_MAX_TAPS.  (The canonical averaging stencil
+// runs hs_adj_rows_kernel instead, the same arithmetic in the same order.)
+template <int NT, int TW, int TH, int MMAX, int NTAP>
 __global__ __launch_bounds__(NT, 8) void hs_adj_tb_kernel(AdjTbArgs a, Taps taps) {
-    static_assert(!RING || NTAP == 8, "the ring build has the 8 canonical taps");
     // LDS window: the tile grown by MMAX, plus one column and one row, so the
     // ghost gathers of pass B (up to two pixels past the image) stay inside
     // it on every side
@@ -332,10 +329,7 @@ __global__ __launch_bounds__(NT, 8) void hs_adj_tb_kernel(AdjTbArgs a, Taps taps
 #pragma unroll
                 for (int i = 0; i < G; ++i)
                     if (d0 + i < NTAP) {
-                        const int dl = RING ? HS_RING_OY[(d0 + i) & 7] * PITCH +
-                                                  HS_RING_OX[(d0 + i) & 7]
-                                            : tp.dl[d0 + i];
-                        q[i] = cell(A, c0 - dl);
+                        q[i] = cell(A, c0 - tp.dl[d0 + i]);
                     }
 #pragma unroll
                 for (int i = 0; i < G; ++i)
@@ -539,6 +533,47 @@ struct AdjTaps {
     Taps dx, dy, dt, av;
 };
 
+// The fused reverse block's builds by window height (16 waves of P rows, one
+// work-group per CU), with the constants of their launch cost in us.
+struct AdjRowsBuild {
+    int rows;  // window rows
+    float launch, tile, step, row;
+    void (*kernel)(AdjRowsArgs);
+};
+static const AdjRowsBuild kAdjRows[] = {
+    {32, 1.33f, 3.77f, 0.218f, 0.0350f, hs_adj_rows_kernel<16, 2, 0, 4>},
+    {48, 0.66f, 5.65f, 0.391f, 0.0336f, hs_adj_rows_kernel<16, 3, 0, 4>},
+    {64, 0.0f, 7.47f, 0.512f, 0.0352f, hs_adj_rows_kernel<16, 4, 3, 4>},
+};
+
+// One fused reverse block of a.m steps of B images, by the build with the least
+// cost: the busiest CU's tiles, each its window's loads and stores, and per step
+// its barriers and active rows.  The constants are a fit to 14 sizes from 64^2 to
+// 1920x1080 and 8 x 512^2 at m = 2 .. 8 (rms error 6-7 %); the build it picks was
+// within 2.6 % of the fastest one at every size and m.
+static int launch_adj_rows(AdjRowsArgs &a, int B, hipStream_t s) {
+    const AdjRowsBuild *best = nullptr;
+    float best_us = 1e30f;
+    for (const AdjRowsBuild &K : kAdjRows) {
+        const RowsGeom g = hs_rows_geom(K.rows, 1, a.H, a.W, a.m, B);
+        const int tiles = (int)(((int64_t)g.ntiles * B + kCus - 1) / kCus);
+        const int active = std::min(std::min(g.th + a.m + 2, K.rows), a.H);
+        const float us = K.launch + (float)tiles * (K.tile + (float)a.m * (K.step + K.row *
+                                                                           (float)active));
+        if (us < best_us) {
+            best_us = us;
+            best = &K;
+            a.tw = g.tw;
+            a.th = g.th;
+            a.tiles_x = g.tiles_x;
+            a.ntiles = g.ntiles;
+        }
+    }
+    hipLaunchKernelGGL(best->kernel, dim3((unsigned)a.ntiles, B), dim3(1024), 0, s, a);
+    HMX_LAUNCH_CHECK("hs_adj_rows");
+    return HMX_OK;
+}
+
 static int make_all_taps(AdjTaps &T, int ndx, const float *wx, const int *oxx, const int *oyx,
                          int ndy, const float *wy, const int *oxy, const int *oyy, int ndt,
                          const float *wt, const int *oxt, const int *oyt, int nda,
@@ -689,9 +724,20 @@ extern "C" int hmx_hs_adjoint(const float *I1, const float *I2, int B, int H, in
     hipLaunchKernelGGL(alpha_sq_kernel, dim3((B + 63) / 64), dim3(64), 0, s, alpha, alpha2, B);
     HMX_LAUNCH_CHECK("alpha_sq");
     rc = fwd_workspace ? HMX_OK : setup_batch(I1, I2, B, H, W, T.dx, T.dy, T.dt, Ix, Iy, It, s);
-    if (!rc) rc = launch_fill_f32(gIx, 0.0f, 3 * n, s);
-    if (!rc) rc = launch_fill_f32(ga2, 0.0f, n, s);
     if (rc) return rc;
+    // The canonical averaging stencil runs fused reverse blocks (hs_adj_rows.h);
+    // HMX_ADJ_GENERIC=1 and HMX_LIN_STAGED=1 take the two-launch form, same
+    // results bit for bit.
+    auto set = [](const char *name) {
+        const char *e = std::getenv(name);
+        return e && e[0] == '1';
+    };
+    const bool fused = hs_ring_taps(T.av) && !set("HMX_ADJ_GENERIC") && !set("HMX_LIN_STAGED");
+    if (!fused || iters == 0) {  // (a fused block starts them at zero itself)
+        rc = launch_fill_f32(gIx, 0.0f, 3 * n, s);
+        if (!rc) rc = launch_fill_f32(ga2, 0.0f, n, s);
+        if (rc) return rc;
+    }
     // the gradient in: dL/dx_N itself for the first reverse launch, then the
     // ping-pong pair g[0], g[1] (the launch writing g[cur ^ 1] reads the other)
     const float *gin_u = gu_N, *gin_v = gv_N;
@@ -713,13 +759,57 @@ extern "C" int hmx_hs_adjoint(const float *I1, const float *I2, int B, int H, in
     a.ntiles = (int)ntiles;
     a.bstride = (int64_t)H * W;
 
-    // the reverse sweep's ring build for the canonical 8-neighbour stencil
-    // (HMX_ADJ_GENERIC=1 takes the generic build, same results bit for bit)
-    const char *gen = std::getenv("HMX_ADJ_GENERIC");
-    const bool ring = hs_ring_taps(T.av) && !(gen && gen[0] == '1');
     const int nck = hmx_hs_ckpt_count(iters, ckpt_every);
     for (int c = nck - 1; c >= 0; --c) {
         const int len = (iters - c * ckpt_every) < ckpt_every ? iters - c * ckpt_every : ckpt_every;
+        if (fused) {
+            // blocks of at most ADJR_MMAX steps: each one's first state, then the
+            // blocks from the last to the first
+            const float *cu = ckpt + (int64_t)(2 * c) * n, *cv = cu + n;
+            const int nb = (len + ADJR_MMAX - 1) / ADJR_MMAX, bs = (len + nb - 1) / nb;
+            int variant, k;
+            hs_choice(H, W, B, bs, false, T.av, variant, k);
+            const float *su = cu, *sv = cv;
+            for (int b = 1; b < nb && !rc; ++b) {
+                float *du = lin + (int64_t)2 * (b - 1) * n, *dv = du + n;
+                rc = hs_sweep(Ix, Iy, It, nullptr, 0.0f, H, W, T.av, bs, su, sv, du, dv, rs[0][0],
+                              rs[0][1], variant, hs_effective_k(variant, k, T.av), s, B, alpha2,
+                              nullptr);
+                su = du;
+                sv = dv;
+            }
+            if (rc) return rc;
+            for (int b = nb - 1; b >= 0; --b) {
+                AdjRowsArgs r;
+                std::memset(&r, 0, sizeof(r));
+                r.Ix = Ix;
+                r.Iy = Iy;
+                r.It = It;
+                r.u = b ? lin + (int64_t)2 * (b - 1) * n : cu;
+                r.v = b ? lin + (int64_t)(2 * (b - 1) + 1) * n : cv;
+                r.gu_in = gin_u;
+                r.gv_in = gin_v;
+                r.gu_out = g[cur][0];
+                r.gv_out = g[cur][1];
+                r.gIx = gIx;
+                r.gIy = gIy;
+                r.gIt = gIt;
+                r.ga2 = ga2;
+                r.alpha2_b = alpha2;
+                r.first = c == nck - 1 && b == nb - 1;
+                r.H = H;
+                r.W = W;
+                r.m = std::min(bs, len - b * bs);
+                r.bstride = (int64_t)H * W;
+                for (int d = 0; d < 8; ++d) r.w[d] = T.av.w[d];
+                rc = launch_adj_rows(r, B, s);
+                if (rc) return rc;
+                gin_u = g[cur][0];
+                gin_v = g[cur][1];
+                cur ^= 1;
+            }
+            continue;
+        }
         // recompute the segment's len steps from its checkpoint, k steps per
         // launch, keeping each step's (ubar, vbar); the states themselves
         // are bit-identical to the forward pass and only ping-pong here
@@ -743,15 +833,12 @@ extern "C" int hmx_hs_adjoint(const float *I1, const float *I2, int B, int H, in
             a.gu_out = g[cur][0];
             a.gv_out = g[cur][1];
             const dim3 grid((unsigned)ntiles, B);
-            if (ring)
-                hipLaunchKernelGGL((hs_adj_tb_kernel<ADJ_NT, ADJ_TW, ADJ_TH, ADJ_MMAX, 8, true>),
-                                   grid, dim3(ADJ_NT), 0, s, a, T.av);
-            else if (T.av.nd == 8)
-                hipLaunchKernelGGL((hs_adj_tb_kernel<ADJ_NT, ADJ_TW, ADJ_TH, ADJ_MMAX, 8, false>),
-                                   grid, dim3(ADJ_NT), 0, s, a, T.av);
+            if (T.av.nd == 8)
+                hipLaunchKernelGGL((hs_adj_tb_kernel<ADJ_NT, ADJ_TW, ADJ_TH, ADJ_MMAX, 8>), grid,
+                                   dim3(ADJ_NT), 0, s, a, T.av);
             else
-                hipLaunchKernelGGL((hs_adj_tb_kernel<ADJ_NT, ADJ_TW, ADJ_TH, ADJ_MMAX, 0, false>),
-                                   grid, dim3(ADJ_NT), 0, s, a, T.av);
+                hipLaunchKernelGGL((hs_adj_tb_kernel<ADJ_NT, ADJ_TW, ADJ_TH, ADJ_MMAX, 0>), grid,
+                                   dim3(ADJ_NT), 0, s, a, T.av);
             HMX_LAUNCH_CHECK("hs_adj_tb");
             gin_u = g[cur][0];
             gin_v = g[cur][1];

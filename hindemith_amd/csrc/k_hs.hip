@@ -466,32 +466,6 @@ int hs_effective_k(int variant, int k, const Taps &taps) {
     return V.nw > 0 && !hs_ring_taps(taps) ? std::min(k, 8) : k;
 }
 
-// Tile grid of a row-register launch of B images: as few columns and rows of
-// tiles as the window allows, then as many rows of tiles as the same number of
-// rounds of work-groups takes, each shorter: a round lasts as long as one tile,
-// so 3600 tiles on 512 places (8 rounds, the last of 16 tiles) cost 8 rounds
-// of 48 rows and 4080 tiles cost 8 of 43 (3840x2160: 107 and 98 us).
-struct RowsGeom {
-    int tw, th, tiles_x, ntiles;  // ntiles: of one image
-};
-constexpr int kCus = 256;
-static RowsGeom hs_rows_geom(const HsVariant &V, int H, int W, int k, int B) {
-    RowsGeom g;
-    const int mw = HS_ROWS_COLS - 2 * k, mh = V.nw * V.rows - 2 * k;
-    int nx = (W + mw - 1) / mw;
-    g.tw = (W + nx - 1) / nx;
-    nx = (W + g.tw - 1) / g.tw;
-    int ny = (H + mh - 1) / mh;
-    const int64_t slots = (int64_t)V.wgs * kCus, col = (int64_t)nx * B;
-    const int64_t rounds = (col * ny + slots - 1) / slots;
-    ny = (int)std::max<int64_t>(ny, std::min<int64_t>(rounds * slots / col, H));
-    g.th = (H + ny - 1) / ny;
-    ny = (H + g.th - 1) / g.th;
-    g.tiles_x = nx;
-    g.ntiles = nx * ny;
-    return g;
-}
-
 // Cost of a row-register launch of k steps in us, from what bounds it: the
 // busiest CU takes m tiles, each of which loads its window and updates its
 // active rows (th + k - 1 on average over the steps) at 31 VALU instructions
@@ -500,7 +474,7 @@ static RowsGeom hs_rows_geom(const HsVariant &V, int H, int W, int k, int B) {
 // was within 2.6 % of the fastest measured one at every size.
 constexpr float kRowsStepUs = 0.0150f;
 static float rows_launch_us(const HsVariant &V, int H, int W, int k, int B) {
-    const RowsGeom g = hs_rows_geom(V, H, W, k, B);
+    const RowsGeom g = hs_rows_geom(V.nw * V.rows, V.wgs, H, W, k, B);
     const int m = (int)(((int64_t)g.ntiles * B + kCus - 1) / kCus);
     const int win = V.nw * V.rows;
     const int active = std::min(std::min(g.th + k - 1, win), H);
@@ -579,7 +553,7 @@ int launch_hs_tb(int variant, const float *Ix, const float *Iy, const float *It,
     a.th = V.th;
     if (V.ring && hs_ring_taps(taps)) kern = V.ring;
     if (hs_runs_rows(V, taps)) {
-        const RowsGeom g = hs_rows_geom(V, H, W, k, B);
+        const RowsGeom g = hs_rows_geom(V.nw * V.rows, V.wgs, H, W, k, B);
         a.tw = g.tw;
         a.th = g.th;
         a.tiles_x = g.tiles_x;

@@ -309,8 +309,10 @@ int hmx_hs_forward_ckpt(const float *I1, const float *I2, int B, int H, int W,
  * dL/dalpha (B, device) and, if non-null, dL/du_0, dL/dv_0.  Recomputes one
  * checkpoint segment at a time; averaging stencil within radius 1.  Optional
  * (null: recomputed here), from the hmx_hs_forward_ckpt call that wrote ckpt:
- * lin_last, its last segment's linearisation, and fwd_workspace, its
- * workspace (derivative planes).  The gradients are the same bits either way. */
+ * lin_last, its last segment's linearisation (not read for the canonical averaging
+ * stencil, whose segments run in fused blocks of at most 8 steps; segments of 8
+ * or fewer need no state recomputed), and fwd_workspace, its workspace (derivative
+ * planes).  The gradients are the same bits either way. */
 int hmx_hs_adjoint(const float *I1, const float *I2, int B, int H, int W, const float *alpha,
                    int ndx, const float *wx, const int *oxx, const int *oyx,
                    int ndy, const float *wy, const int *oxy, const int *oyy,
