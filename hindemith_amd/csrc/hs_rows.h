@@ -74,6 +74,29 @@ inline RowsGeom hs_rows_geom(int win, int wgs, int H, int W, int k, int B) {
     return g;
 }
 
+// Cost in us of a row-register launch of k steps, from what bounds it: the busiest CU
+// takes m tiles, each of which loads its window (load per window row) and in each
+// step pays its barrier (step) and updates its active rows (row each; tile rows
+// + k - 1 on average over the steps) at 31 VALU instructions per wave-row.  Fitted
+// per build to 21 image sizes from 64^2 to 3840x2160 at k = 4 .. 16 (rms error 3-8
+// %): the (build, k) of least cost was the fastest measured one at 17 of them, and
+// within 3.8 % of it at the others.
+struct RowsCost {
+    float launch, load, row, step;
+    float us(int win, int m, int k, float active) const {
+        return launch + (float)m * (load * (float)win +
+                                    (float)k * (row * std::min(active, (float)win) + step));
+    }
+};
+constexpr RowsCost kRowsCost16x2 = {4.33f, 0.0071f, 0.0145f, 0.0925f};   // waves x rows
+constexpr RowsCost kRowsCost16x3 = {2.67f, 0.0383f, 0.0120f, 0.2019f};
+constexpr RowsCost kRowsCost16x4 = {2.59f, 0.0353f, 0.0121f, 0.2527f};
+constexpr RowsCost kRowsCost16x5 = {2.17f, 0.0447f, 0.0117f, 0.2558f};
+constexpr RowsCost kRowsCost8x7 = {4.85f, 0.0218f, 0.0099f, 0.1674f};
+constexpr RowsCost kRowsCost8x9 = {5.50f, 0.0240f, 0.0094f, 0.1741f};
+constexpr RowsCost kRowsCost8x10 = {5.72f, 0.0223f, 0.0098f, 0.2204f};
+constexpr RowsCost kRowsCost16x4two = {5.07f, 0.0216f, 0.0110f, 0.0754f};  // two per CU
+
 // LDS of one work-group: the first and last row of every wave's strip, double
 // buffered (another wave reads them), and its other rows (read by the wave alone).
 template <int NW, int P>

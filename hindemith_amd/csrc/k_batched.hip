@@ -23,6 +23,7 @@
 // work-group has given up, it sets *status and every work-group returns, so
 // the grid always drains.  The launch is captured in a hipGraph (counter and
 // status reset by a fill kernel, never a memset node) and replayed.
+#include "hs_rows.h"
 #include "hs_tile.h"
 
 #include <algorithm>
@@ -42,6 +43,7 @@ struct PairDesc {
     float *zu, *zv;  // stepped form: third plane pair (see phase_image_stepped)
     float alpha2;
     int H, W, tiles_x, tile_base, ntiles;
+    int tw, th;  // output tile
 };
 
 struct BatchArgs {
@@ -378,6 +380,53 @@ __global__ __launch_bounds__(NT) __attribute__((amdgpu_num_sgpr(74))) void hs_mu
                                                       uvm + Win::PAD);
 }
 
+// Stepped form on the row-register tile (hs_rows.h) for the canonical stencils: every
+// pair has a tile grid of its own, as few tiles as the window allows and all of one
+// size, and phase 0 computes the derivatives (no setup launch).  Against the 64 x 32
+// tiles of variant 8, 200 iterations: 32 pairs of 64 .. 1024 pixels a side 3.80 ->
+// 3.17 ms, 64 of them 7.23 -> 6.36; 100 iterations: 6 pairs up to 300 pixels 204 ->
+// 151 us.
+struct MultiRowsArgs {
+    const PairDesc *tiles;
+    int total_tiles, nph;
+    float w[8];       // averaging weights
+    float cube[12];   // Dx, Dy, Dt weights (HsSetup)
+};
+
+template <int NW, int P, bool PRE, int G, bool FIRST>
+__device__ __forceinline__ void multi_rows_body(const MultiRowsArgs &b, int ph, int kk) {
+    __shared__ HsRowsLds<NW, P> lds;
+    // phases alternate the walk over each XCD's share of the list
+    const int w = xcd_remap(blockIdx.x, b.total_tiles, (ph & 1) == 0);
+    const PairDesc &D = b.tiles[w];
+    const HsImage im = phase_image_stepped(D, ph, b.nph, 0);
+    HsSetup su;
+    if (FIRST) {
+        su.I1 = D.I1;
+        su.I2 = D.I2;
+        su.Ix = D.Ix;
+        su.Iy = D.Iy;
+        su.It = D.It;
+#pragma unroll
+        for (int d = 0; d < 12; ++d) su.w[d] = b.cube[d];
+    }
+    const int t = w - D.tile_base;
+    const int tyi = t / D.tiles_x, txi = t - tyi * D.tiles_x;
+    hs_rows_tile<NW, P, PRE, G, false, FIRST>(im, txi, tyi, D.tw, D.th, kk, b.w, lds, &su);
+}
+
+template <int NW, int P, bool PRE, int G, int WPE>
+__global__ __launch_bounds__(64 * NW, WPE) void hs_multi_rows_kernel(MultiRowsArgs b, int ph,
+                                                                     int kk) {
+    multi_rows_body<NW, P, PRE, G, false>(b, ph, kk);
+}
+
+template <int NW, int P, bool PRE, int G, int WPE>
+__global__ __launch_bounds__(64 * NW, WPE) void hs_multi_rows_first_kernel(MultiRowsArgs b, int ph,
+                                                                           int kk) {
+    multi_rows_body<NW, P, PRE, G, true>(b, ph, kk);
+}
+
 // ---------------------------------------------------------------------------
 struct BVariant {
     int nt, tw, th, kmax, wpe;
@@ -385,6 +434,12 @@ struct BVariant {
     // stepped form (kernel[] null): setup, phase (8 taps, any count)
     void (*setup)(BatchArgs, SetupTaps);
     void (*phase[2])(BatchArgs, Taps, int, int);
+    // row-register stepped form (else zero): waves and rows per wave, work-groups per
+    // CU, its launch cost, phase and first phase
+    int nw, rows, wgs;
+    RowsCost cost;
+    void (*rphase)(MultiRowsArgs, int, int);
+    void (*rfirst)(MultiRowsArgs, int, int);
 };
 
 #define HB_V(NT, TW, TH, K, WPE)                                                          \
@@ -406,6 +461,11 @@ struct BVariant {
     {NT, TW, TH, K, 0, {nullptr, nullptr}, hs_multi_setup_kernel<kSetupNT, TW, TH>,      \
      {hs_multi_phase_kernel<NT, TW, TH, K, 8, DB, FDIV>,                                  \
       hs_multi_phase_kernel<NT, TW, TH, K, 0, DB, FDIV>}}
+// row-register stepped form
+#define HB_R(NW, P, PRE, G, WPE, WGS, KMAX, COST)                                         \
+    {64 * NW, 48, NW * P - 16, KMAX, 0, {nullptr, nullptr}, nullptr, {nullptr, nullptr},  \
+     NW, P, WGS, COST, hs_multi_rows_kernel<NW, P, PRE, G, WPE>,                    \
+     hs_multi_rows_first_kernel<NW, P, PRE, G, WPE>}
 static const BVariant kBVariants[] = {
     HB_V(1024, 64, 32, 4, 8),   // 0: two work-groups per CU
     HB_V(1024, 64, 32, 8, 8),   // 1: two work-groups per CU
@@ -419,11 +479,21 @@ static const BVariant kBVariants[] = {
     HB_S(1024, 64, 32, 4, true, true),   // 9: stepped, as variant 25
     HB_S(1024, 64, 32, 8, true, false),  // 10: stepped, as variant 17
     HB_S(512, 64, 32, 4, true, true),    // 11: stepped, as variant 26
+    // 12-18: stepped, row-register tiles (tile at k = 8), as the single-image
+    // variants 29, 30, 32, 33, 34, 35 and 36
+    HB_R(16, 2, true, 2, 4, 1, 12, kRowsCost16x2),
+    HB_R(16, 3, true, 3, 4, 1, 16, kRowsCost16x3),
+    HB_R(16, 5, true, 5, 4, 1, 16, kRowsCost16x5),
+    HB_R(8, 7, false, 4, 4, 2, 16, kRowsCost8x7),
+    HB_R(8, 9, false, 3, 4, 2, 16, kRowsCost8x9),
+    HB_R(8, 10, false, 2, 4, 2, 16, kRowsCost8x10),
+    HB_R(16, 4, false, 1, 8, 2, 16, kRowsCost16x4two),
 };
 #undef HB_V
 #undef HB_D
 #undef HB_F
 #undef HB_S
+#undef HB_R
 static constexpr int kNumBVariants = sizeof(kBVariants) / sizeof(kBVariants[0]);
 
 // A cached launch: device descriptors, barrier words and (optionally) the
@@ -460,6 +530,54 @@ static void append(std::vector<char> &k, const T &v) {
     k.insert(k.end(), c, c + sizeof(T));
 }
 
+bool hs_cube_taps(const Taps &dx, const Taps &dy, const Taps &dt, HsSetup &su);
+
+// A pair's tile grid: of a row-register variant as few tiles of at most the window's
+// reach as fit and all of one size, else the variant's own tile.
+static void pair_tiles(const BVariant &V, int k, int H, int W, int &tw, int &th, int &nx, int &ny) {
+    tw = V.tw;
+    th = V.th;
+    if (V.nw) {
+        const int mw = HS_ROWS_COLS - 2 * k, mh = V.nw * V.rows - 2 * k;
+        const int cx = (W + mw - 1) / mw, cy = (H + mh - 1) / mh;
+        tw = (W + cx - 1) / cx;
+        th = (H + cy - 1) / cy;
+    }
+    nx = (W + tw - 1) / tw;
+    ny = (H + th - 1) / th;
+}
+
+// The row-register variant and iterations per phase with the least cost for these
+// pairs, as hs_rows_choice for one image: the busiest CU's tiles times the mean
+// tile's rows.  At least two phases (a single one would read the planes it writes);
+// an odd phase count needs no copy (the third plane pair).
+static void batched_rows_choice(const hmx_pair *pairs, int npairs, int iters, int &variant,
+                                int &k) {
+    float best = 1e30f;
+    for (int vi = 0; vi < kNumBVariants; ++vi) {
+        const BVariant &V = kBVariants[vi];
+        if (!V.nw) continue;
+        for (int kk = std::min(5, (iters + 1) / 2); kk <= std::min(V.kmax, (iters + 1) / 2); ++kk) {
+            int64_t tiles = 0, active = 0;
+            for (int i = 0; i < npairs; ++i) {
+                int tw, th, nx, ny;
+                pair_tiles(V, kk, pairs[i].H, pairs[i].W, tw, th, nx, ny);
+                tiles += (int64_t)nx * ny;
+                active += (int64_t)nx * ny * std::min(th + kk - 1, pairs[i].H);
+            }
+            const int m = (int)((tiles + kCus - 1) / kCus);
+            const int nph = (iters + kk - 1) / kk;
+            const float us = (float)nph * V.cost.us(V.nw * V.rows, m, kk,
+                                               (float)active / (float)tiles);
+            if (us < best) {
+                best = us;
+                variant = vi;
+                k = kk;
+            }
+        }
+    }
+}
+
 static int launch_batch(const BatchPlan &P, const SetupTaps &st, const Taps &av, int npairs,
                         int iters, long long spin_limit, hipStream_t s) {
     int rc = launch_fill_u32(P.d_sync, 0u, P.sync_words, s);
@@ -476,6 +594,24 @@ static int launch_batch(const BatchPlan &P, const SetupTaps &st, const Taps &av,
     a.k = P.k;
     const int nph = (iters + P.k - 1) / P.k;
     const BVariant &V = kBVariants[P.variant];
+    if (V.nw) {
+        MultiRowsArgs r;
+        r.tiles = P.d_pairs;
+        r.total_tiles = P.total_tiles;
+        r.nph = nph;
+        for (int d = 0; d < 8; ++d) r.w[d] = av.w[d];
+        HsSetup su;
+        if (!hs_cube_taps(st.dx, st.dy, st.dt, su))  // (the variant is chosen for them)
+            return fail(HMX_ERR_UNSUPPORTED, "hmx_hs_batched: not the canonical stencils");
+        std::copy(su.w, su.w + 12, r.cube);
+        for (int ph = 0; ph < nph; ++ph) {
+            const int kk = std::min(P.k, iters - ph * P.k);
+            hipLaunchKernelGGL(ph == 0 ? V.rfirst : V.rphase, dim3(P.total_tiles), dim3(V.nt), 0,
+                               s, r, ph, kk);
+            HMX_LAUNCH_CHECK("hs_multi_rows");
+        }
+        return HMX_OK;
+    }
     a.nph = nph;
     a.phase0 = V.kernel[0] ? nph & 1 : nph == 1;
     if (V.kernel[0]) {
@@ -503,6 +639,7 @@ static int launch_batch(const BatchPlan &P, const SetupTaps &st, const Taps &av,
 static int resident_per_cu(int variant, int nd, int device, int &api, int &own, int &cus) {
     const BVariant &V = kBVariants[variant];
     const void *kern = V.kernel[0] ? reinterpret_cast<const void *>(V.kernel[nd == 8 ? 0 : 1])
+                       : V.nw      ? reinterpret_cast<const void *>(V.rphase)
                                    : reinterpret_cast<const void *>(V.phase[nd == 8 ? 0 : 1]);
     HMX_HIP_TRY(hipOccupancyMaxActiveBlocksPerMultiprocessor(&api, kern, V.nt, 0));
     if (!V.kernel[0]) {  // stepped form: no residency requirement
@@ -644,6 +781,11 @@ static int batched_impl(const hmx_pair *pairs, int npairs, const SetupTaps &st, 
     HMX_REQUIRE(iters >= 0, "hmx_hs_batched: iters must be >= 0");
     HMX_REQUIRE(av.rx <= 1 && av.ry <= 1 && av.nd <= HS_MAX_TAPS,
                 "hmx_hs_batched: averaging stencil must lie within radius 1 with <= 9 taps");
+    HsSetup su;
+    const bool canonical = hs_ring_taps(av) && hs_cube_taps(st.dx, st.dy, st.dt, su);
+    for (int i = 0; i < npairs; ++i)
+        HMX_REQUIRE(pairs[i].H > 0 && pairs[i].W > 0 && pairs[i].H < 32768 && pairs[i].W < 32768,
+                    "hmx_hs_batched: pair sizes must be in 1..32767");
     if (variant < 0) {  // autotuned choice for this size signature, else default
         variant = 8;  // stepped, double-buffered, reciprocal quotient
         k = 8;
@@ -653,22 +795,29 @@ static int batched_impl(const hmx_pair *pairs, int npairs, const SetupTaps &st, 
             sig.push_back(pairs[i].W);
         }
         std::lock_guard<std::mutex> lk(g_bmu);
+        bool tuned = false;
         for (auto &e : g_btuned)
             if (e.first == sig) {
                 variant = e.second.first;
                 k = e.second.second;
+                tuned = true;
             }
+        if (!tuned && iters >= 2 && canonical) batched_rows_choice(pairs, npairs, iters, variant, k);
     }
     HMX_REQUIRE(variant < kNumBVariants, "hmx_hs_batched: unknown variant");
     HMX_REQUIRE(k >= 1 && k <= kBVariants[variant].kmax, "hmx_hs_batched: k out of range");
+    // the row-register variants take the canonical stencils and two phases or more;
+    // for anything else they stand for variant 8
+    if (kBVariants[variant].nw && (!canonical || iters <= k)) {
+        variant = 8;
+        k = std::min(k, kBVariants[8].kmax);
+    }
     const BVariant &V = kBVariants[variant];
     std::vector<PairDesc> desc(npairs);
     int tiles = 0;
     for (int i = 0; i < npairs; ++i) {
         const hmx_pair &p = pairs[i];
         HMX_REQUIRE(p.I1 && p.I2 && p.u && p.v && p.work, "hmx_hs_batched: null pair buffer");
-        HMX_REQUIRE(p.H > 0 && p.W > 0 && p.H < 32768 && p.W < 32768,
-                    "hmx_hs_batched: pair sizes must be in 1..32767");
         const int64_t n = (int64_t)p.H * p.W;
         PairDesc &d = desc[i];
         d.I1 = p.I1;
@@ -685,8 +834,9 @@ static int batched_impl(const hmx_pair *pairs, int npairs, const SetupTaps &st, 
         d.alpha2 = p.alpha * p.alpha;
         d.H = p.H;
         d.W = p.W;
-        d.tiles_x = (p.W + V.tw - 1) / V.tw;
-        d.ntiles = d.tiles_x * ((p.H + V.th - 1) / V.th);
+        int ny;
+        pair_tiles(V, k, p.H, p.W, d.tw, d.th, d.tiles_x, ny);
+        d.ntiles = d.tiles_x * ny;
         d.tile_base = tiles;
         HMX_REQUIRE((int64_t)tiles + d.ntiles < (1 << 30), "hmx_hs_batched: too many tiles");
         tiles += d.ntiles;

@@ -296,11 +296,9 @@ struct HsVariant {
     bool persist;                     // whole solve in one persistent launch (hs_persist_run)
     // Row-register forms: waves per work-group and rows per wave of the canonical
     // stencil's kernel (in `ring`; other stencils run variant 24's kernels), the
-    // work-groups of it a CU holds, and its launch cost (rows_launch_us): us
-    // of a launch besides the steps, and per window row of each work-group a CU
-    // takes.  Zero for the others.
+    // work-groups of it a CU holds, and its launch cost.  Zero for the others.
     int nw, rows, wgs;
-    float us0, us_row;
+    RowsCost cost;
     void (*first)(HsArgs, Taps, HsSetup);  // a solve's first launch, with its setup
     void (*lin)(HsArgs, Taps);             // with the linearisation output, or null
 };
@@ -342,14 +340,14 @@ static int tap_class(int nd) {
       hs_strip_kernel<NT, TW, TH, K, S, 8>, hs_strip_kernel<NT, TW, TH, K, S, 9>,      \
       hs_strip_kernel<NT, TW, TH, K, S, 0>}, nullptr}
 // row-register forms: the canonical stencil's kernel, and variant 24's for others
-#define HS_R(NW, P, PRE, G, WPE, WGS, KMAX, US0, USROW, LIN)                            \
+#define HS_R(NW, P, PRE, G, WPE, WGS, KMAX, COST, LIN)                                  \
     {1024, 64, 32, KMAX, 0,                                                             \
      {hs_tb_kernel<1024, 64, 32, 8, 4, false, true, true>,                              \
       hs_tb_kernel<1024, 64, 32, 8, 5, false, true, true>,                              \
       hs_tb_kernel<1024, 64, 32, 8, 8, false, true, true>,                              \
       hs_tb_kernel<1024, 64, 32, 8, 9, false, true, true>,                              \
       hs_tb_kernel<1024, 64, 32, 8, 0, false, true, true>},                             \
-     hs_rows_kernel<NW, P, PRE, G, WPE>, false, NW, P, WGS, US0, USROW,                 \
+     hs_rows_kernel<NW, P, PRE, G, WPE>, false, NW, P, WGS, COST,                 \
      hs_rows_first_kernel<NW, P, PRE, G, WPE>, LIN}
 static const HsVariant kVariants[] = {
     HS_V(256, 64, 16, 1),     // 0: one iteration per launch (plain sweep)
@@ -404,21 +402,21 @@ static const HsVariant kVariants[] = {
     // VGPRs).  Two work-groups per CU for larger images, so that one's loads
     // and barriers overlap the other's steps: 8 waves at up to 128 VGPRs, or 16 at
     // 61 (one row at a time; its linearisation build would spill).
-    HS_R(16, 2, true, 2, 4, 1, 12, 4.39f, 0.0183f,
+    HS_R(16, 2, true, 2, 4, 1, 12, kRowsCost16x2,
          (hs_rows_kernel<16, 2, true, 2, 4, true>)),   // 29: window 64 x 32
-    HS_R(16, 3, true, 3, 4, 1, 16, 3.22f, 0.0422f,
+    HS_R(16, 3, true, 3, 4, 1, 16, kRowsCost16x3,
          (hs_rows_kernel<16, 3, true, 3, 4, true>)),   // 30: 64 x 48
-    HS_R(16, 4, true, 4, 4, 1, 16, 3.09f, 0.0437f,
+    HS_R(16, 4, true, 4, 4, 1, 16, kRowsCost16x4,
          (hs_rows_kernel<16, 4, true, 4, 4, true>)),   // 31: 64 x 64
-    HS_R(16, 5, true, 5, 4, 1, 16, 2.89f, 0.0445f,
+    HS_R(16, 5, true, 5, 4, 1, 16, kRowsCost16x5,
          (hs_rows_kernel<16, 5, true, 5, 4, true>)),   // 32: 64 x 80
-    HS_R(8, 7, false, 4, 4, 2, 16, 6.22f, 0.0077f,
+    HS_R(8, 7, false, 4, 4, 2, 16, kRowsCost8x7,
          (hs_rows_kernel<8, 7, false, 4, 4, true>)),   // 33: 64 x 56
-    HS_R(8, 9, false, 3, 4, 2, 16, 7.28f, 0.0092f,
+    HS_R(8, 9, false, 3, 4, 2, 16, kRowsCost8x9,
          (hs_rows_kernel<8, 9, false, 3, 4, true>)),   // 34: 64 x 72
-    HS_R(8, 10, false, 2, 4, 2, 16, 8.32f, 0.0099f,
+    HS_R(8, 10, false, 2, 4, 2, 16, kRowsCost8x10,
          (hs_rows_kernel<8, 10, false, 2, 4, true>)),  // 35: 64 x 80
-    HS_R(16, 4, false, 1, 8, 2, 16, 5.80f, 0.0201f,
+    HS_R(16, 4, false, 1, 8, 2, 16, kRowsCost16x4two,
          nullptr),  // 36: 64 x 64
 };
 #undef HS_R
@@ -466,19 +464,10 @@ int hs_effective_k(int variant, int k, const Taps &taps) {
     return V.nw > 0 && !hs_ring_taps(taps) ? std::min(k, 8) : k;
 }
 
-// Cost of a row-register launch of k steps in us, from what bounds it: the
-// busiest CU takes m tiles, each of which loads its window and updates its
-// active rows (th + k - 1 on average over the steps) at 31 VALU instructions
-// per wave-row.  The constants are a fit to 15 image sizes from 64^2 to
-// 3840x2160 at k = 5 .. 12, every variant (rms error 3-8 %); the choice it makes
-// was within 2.6 % of the fastest measured one at every size.
-constexpr float kRowsStepUs = 0.0150f;
 static float rows_launch_us(const HsVariant &V, int H, int W, int k, int B) {
     const RowsGeom g = hs_rows_geom(V.nw * V.rows, V.wgs, H, W, k, B);
     const int m = (int)(((int64_t)g.ntiles * B + kCus - 1) / kCus);
-    const int win = V.nw * V.rows;
-    const int active = std::min(std::min(g.th + k - 1, win), H);
-    return V.us0 + (float)m * (V.us_row * (float)win + kRowsStepUs * (float)(k * active));
+    return V.cost.us(V.nw * V.rows, m, k, (float)std::min(g.th + k - 1, H));
 }
 
 // The row-register variant and iterations per launch with the least cost for

@@ -355,8 +355,10 @@ struct hmx_pair {
 
 /* Setup + iters Jacobi iterations of every pair over one list of all pairs'
  * tiles, in phases of k iterations.  Two forms:
- *   stepped (variants 8-11, the default): one launch per phase over every
- *     tile, plus a setup launch.  Phases alternate (u, v) with the work
+ *   stepped (variants 8 and up, the default): one launch per phase over every
+ *     tile, plus a setup launch (variants 8-11) or the setup in the first phase
+ *     (12 and up: row-register tiles for the canonical stencils and two phases or
+ *     more; anything else runs variant 8 instead).  Phases alternate (u, v) with the work
  *     planes; an odd number of phases above one also uses a plane pair the
  *     launch state owns (2 x H x W floats per pair), so the last phase writes
  *     (u, v) and nothing is copied; a single phase reads a copy of (u, v)
@@ -369,7 +371,8 @@ struct hmx_pair {
  *     every work-group exits.  A persistent call always synchronises its
  *     stream and returns HMX_ERR_TIMEOUT in that case (so a partial result
  *     is never silent); HMX_BATCH_SYNC makes a stepped call synchronise too.
- * variant = -1 uses the autotuned (or default) variant and k.
+ * variant = -1 uses the autotuned variant and k, or those a rule on the sizes and
+ * iterations picks.
  * Launch state (descriptors, barrier words, graph, the stepped form's extra
  * plane pairs) is cached per signature, up to 8 signatures;
  * a graph call on a signature first run eagerly captures the graph then.

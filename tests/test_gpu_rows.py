@@ -73,3 +73,26 @@ def test_default_choice_bitexact(shape, iters):
     u, v = u0.clone(), v0.clone()
     K.hs_jacobi(Ix, Iy, It, 0.7, AVG, iters, u, v)
     assert torch.equal(u, ru) and torch.equal(v, rv)
+
+
+@pytest.mark.parametrize("taps9", [False, True])
+def test_batched_rows_variants_match_single_solves(taps9):
+    """The batched row-register variants on uneven pairs, and what they stand for
+    with another averaging stencil (variant 8), at even and odd phase counts."""
+    from hindemith_amd import batched
+    taps = dict(TAPS, Avg=AVG)
+    if taps9:
+        taps["Avg"] = (np.full(9, 1.0 / 9.0, np.float32), np.array([-1, 0, 1] * 3, np.int32),
+                       np.repeat(np.array([-1, 0, 1], np.int32), 3))
+    rng = np.random.default_rng(2)
+    f = lambda s: torch.from_numpy(rng.normal(size=s).astype(np.float32)).cuda()  # noqa: E731
+    shapes = [(1, 70), (33, 47), (90, 131), (64, 49), (257, 3)]
+    B = batched.BatchedHS([f(s) for s in shapes], [f(s) for s in shapes], [0.5, 1.0, 1.5, 2.0, 0.75],
+                          iters=17, taps=taps)
+    ref = [(u.clone(), v.clone()) for u, v in B.solve_each(variant=0, k=1)]
+    n = len(batched.batched_variants())
+    for vi, k in [(-1, 0)] + [(vi, k) for vi in range(8, n) if vi == 8 or vi >= 12
+                              for k in (3, 6, 8)]:
+        out = B.run(graph=False, variant=vi, k=k)
+        for (u, v), (ru, rv) in zip(out, ref):
+            assert torch.equal(u, ru) and torch.equal(v, rv), (vi, k, tuple(u.shape))
