@@ -13,7 +13,7 @@
 
 namespace hmx {
 
-constexpr int RED_NT = 256;
+constexpr int RED_NT = 256, SUM_U = 8;
 
 __device__ inline double wave_sum(double v) {
 #pragma unroll
@@ -37,8 +37,17 @@ __global__ __launch_bounds__(RED_NT) void sum_pass1_kernel(const float *__restri
                                                            double *__restrict__ partials) {
     double acc = 0.0;
     const int64_t stride = (int64_t)gridDim.x * RED_NT;
-    for (int64_t i = (int64_t)blockIdx.x * RED_NT + threadIdx.x; i < n; i += stride)
-        acc += (double)x[i];
+    // SUM_U reads in flight per thread, added in the order of a plain loop (the
+    // same bits): one read at a time left a 3840x2160 plane at 1.5 TB/s (22 us)
+    int64_t i = (int64_t)blockIdx.x * RED_NT + threadIdx.x;
+    for (; i + (SUM_U - 1) * stride < n; i += SUM_U * stride) {
+        float v[SUM_U];
+#pragma unroll
+        for (int q = 0; q < SUM_U; ++q) v[q] = x[i + q * stride];
+#pragma unroll
+        for (int q = 0; q < SUM_U; ++q) acc += (double)v[q];
+    }
+    for (; i < n; i += stride) acc += (double)x[i];
     const double r = block_sum(acc);
     if (threadIdx.x == 0) partials[blockIdx.x] = r;
 }
