@@ -13,6 +13,7 @@
 // rounding per operator, the "y += p * q" accumulations of HSMatrixPowers as
 // fmas (as the stencil accumulation elsewhere), correctly rounded division.
 #include "hmx_common.h"
+#include "hs_rows.h"
 
 #include <algorithm>
 
@@ -61,19 +62,32 @@ __global__ __launch_bounds__(256) void hs_precond_kernel(
 // ---------------------------------------------------------------------------
 // a16: V[0] = r, V[s] = A V[s-1] for s = 1..steps-1, all powers stored.
 //
-// Temporally blocked like the Jacobi sweep: a work-group loads r on its tile
-// grown by m = (powers this launch) pixels, Ix and Iy into registers, and
-// computes the m powers on chip; power j is valid on the tile grown by m - j.
-// Two LDS windows: power j reads one and writes the other, one barrier per
-// power.  Each power's tile is stored as it is made, so HBM traffic per launch
-// is 16 B/px read + 8 B/px per power written (the per-power launches of the
-// reference move 24 B/px per power).
+// Temporally blocked like the Jacobi sweep, in its row-register layout
+// (hs_rows_tile): a work-group loads r, Ix and Iy on its tile grown by m =
+// (powers this launch) pixels and computes the m powers on chip; power j is valid
+// on the tile grown by m - j.  A lane is a window column, a wave owns POW_P
+// window rows in registers, and only left and right neighbours (a wave's own
+// rows) and the rows where two waves meet go through LDS: 3 LDS operations per
+// cell and power, one barrier per power.  Each power's tile is stored as it is
+// made, so HBM traffic per launch is 16 B/px read + 8 B/px per power written (the
+// per-power launches of the reference move 24 B/px per power).
+//
+// What bounds it: the stores.  8 powers and r of 3840x2160 are 597 MB out and 133 MB
+// in, 119 us at the rates of a fill (6.9 TB/s) and a read (4.2); without its stores
+// the kernel takes 100 us.  Measured, 8 powers: 3840x2160 161 us (a 64x32 tile with
+// every cell's neighbours read from LDS: 239, 183 with non-temporal stores),
+// 1920x1080 35 (43.5), 135x240 11 (13.7).  Tiles are POW_TW = 48 columns, three
+// 64-byte sectors a row: 32-column tiles in whole cache lines cost 214 us in redundant
+// columns; windows of 48 to 96 rows and 8 to 16 waves lie within 155 - 177.
+constexpr int POW_MMAX = 8, POW_TW = HS_ROWS_COLS - 2 * POW_MMAX;
+constexpr int POW_NW = 16, POW_P = 4;  // waves, window rows per wave
+
 struct PowArgs {
     const float *Ix, *Iy;
     const float *u0, *v0;  // power s0 - 1 (V[0] = r on the first launch)
     float *V0, *V1;        // steps x H x W
     int s0, m;             // this launch makes powers s0 .. s0+m-1
-    int H, W, tiles_x, ntiles;
+    int H, W, th, tiles_x, ntiles;
     int64_t plane;         // H * W
     const void *lam_dev;   // device scalar of dtype lam_dtype, or null: lam_val
     int lam_dtype;
@@ -81,19 +95,36 @@ struct PowArgs {
     int copy_r;            // also store V[0] = r (the Array2D -> Array3D copy)
 };
 
-template <int NT, int TW, int TH, int MMAX>
-__global__ __launch_bounds__(NT) void hs_powers_kernel(PowArgs a) {
-    constexpr int PITCH = TW + 2 * MMAX, RHM = TH + 2 * MMAX, NPX = PITCH * RHM;
-    constexpr int P = (NPX + NT - 1) / NT;
-    __shared__ float2 win[2][NPX];
+template <int NW, int P, bool NTS>
+__global__ __launch_bounds__(NW * 64, 8) void hs_powers_kernel(PowArgs a) {
+    __shared__ HsRowsLds<NW, P> lds;
+    const int lane = threadIdx.x & 63;
+    const int wave = __builtin_amdgcn_readfirstlane((int)threadIdx.x >> 6);
     const int H = a.H, W = a.W, m = a.m;
     const int t = xcd_remap(blockIdx.x, a.ntiles);
     const int tyi = t / a.tiles_x, txi = t - tyi * a.tiles_x;
-    const int x0 = txi * TW, y0 = tyi * TH;
-    const int x1 = min(x0 + TW, W), y1 = min(y0 + TH, H);
-    const int gx0 = max(x0 - m, 0), gy0 = max(y0 - m, 0);
-    const int gx1 = min(x1 + m, W), gy1 = min(y1 + m, H);
-    const int RW = gx1 - gx0, RH = gy1 - gy0;
+    const int x0 = txi * POW_TW, y0 = tyi * a.th;
+    const int x1 = min(x0 + POW_TW, W), y1 = min(y0 + a.th, H);
+    // window: columns x0 - m .., rows from y0 - m, or from the image's first
+    const int gx0 = x0 - m, gy0 = max(y0 - m, 0);
+    const int gx = gx0 + lane;
+    const int r0 = wave * P;  // the strip's first window row
+    // a row's address is uniform over its wave (64-bit offsets, for planes of any
+    // size); a lane adds its column's distance from the window's first
+    const unsigned co = (unsigned)(clampi(gx, 0, W - 1) - gx0) * 4u;
+    const unsigned lane4 = (unsigned)lane * 4u;
+    float cx[P], cy[P], u[P], v[P];
+#pragma unroll
+    for (int j = 0; j < P; ++j) {
+        const int64_t o = (int64_t)min(gy0 + r0 + j, H - 1) * W + gx0;
+        auto ld = [&](const float *p) {
+            return ld_g(reinterpret_cast<const float *>(reinterpret_cast<const char *>(p + o) + co));
+        };
+        u[j] = ld(a.u0);
+        v[j] = ld(a.v0);
+        cx[j] = ld(a.Ix);
+        cy[j] = ld(a.Iy);
+    }
     // a scalar of another dtype is rounded to float32 first
     float lam = a.lam_val;
     if (a.lam_dev) {
@@ -105,126 +136,108 @@ __global__ __launch_bounds__(NT) void hs_powers_kernel(PowArgs a) {
         }
     }
     const float nlam = -lam;
-
-    // Thread tid owns window cells c = tid + j*NT (the pitch-PITCH grid), so a
-    // neighbour of cell c is c +- 1 or c +- PITCH: constant LDS offsets.  pk
-    // packs L << 27 | ry << 16 | rx for a cell in the region, L = m - (its
-    // distance outside the tile) = the last power that updates it (the
-    // region of power j is the tile grown by m - j, clipped to the image);
-    // -1 for cells outside the region.
-    const bool clipped = (x0 - m < 0) || (y0 - m < 0) || (x1 + m > W) || (y1 + m > H);
-    int pk[P];
-    float cx[P], cy[P];
+    const int li = max(lane - 1, 0), ri = min(lane + 1, HS_ROWS_COLS - 1);
+    const bool in = gx >= x0 && gx < x1;
+    const bool has_l = gx > 0, has_r = gx < W - 1;
+    // the strip's rows in the output tile
+    unsigned tile_rows = 0;
+    for (int j = 0; j < P; ++j)
+        if (gy0 + r0 + j >= y0 && gy0 + r0 + j < y1) tile_rows |= 1u << j;
+    // rows of power s: uniform row addresses plus the lane's offset (opaque, so that
+    // it is added by the store and not before, in 64-bit vector additions)
+    auto store = [&](int s, const float (&p)[P], const float (&q)[P]) {
+        const int64_t o = (int64_t)s * a.plane + (int64_t)(gy0 + r0) * W + gx0;
+        float *row0 = a.V0 + o, *row1 = a.V1 + o;
 #pragma unroll
-    for (int j = 0; j < P; ++j) {
-        const int c = threadIdx.x + j * NT;
-        const int ry = c / PITCH, rx = c - ry * PITCH;
-        pk[j] = -1;
-        cx[j] = cy[j] = 0.0f;
-        if (c < NPX && rx < RW && ry < RH) {
-            const int gx = gx0 + rx, gy = gy0 + ry;
-            const int dx = max(max(x0 - gx, gx - x1 + 1), 0);
-            const int dy = max(max(y0 - gy, gy - y1 + 1), 0);
-            pk[j] = ((m - max(dx, dy)) << 27) | (ry << 16) | rx;
-            const int64_t g = (int64_t)gy * W + gx;
-            cx[j] = a.Ix[g];
-            cy[j] = a.Iy[g];
-            const float u = a.u0[g], v = a.v0[g];
-            win[0][c] = make_float2(u, v);
-            if (a.copy_r && gx >= x0 && gx < x1 && gy >= y0 && gy < y1) {
-                st_out(a.V0 + g, u, rows_whole_lines(a.W));
-                st_out(a.V1 + g, v, rows_whole_lines(a.W));
-            }
+        for (int j = 0; j < P; ++j, row0 += W, row1 += W) {
+            if (!((tile_rows >> j) & 1)) continue;
+            auto st = [&](float *row, float x) {
+                unsigned l4 = lane4;
+                asm volatile("" : "+v"(l4));
+                gfloat *const g = (gfloat *)(reinterpret_cast<char *>(row) + l4);
+                if (NTS)
+                    __builtin_nontemporal_store(x, g);
+                else
+                    *g = x;
+            };
+            st(row0, p[j]);
+            st(row1, q[j]);
         }
-    }
-    __syncthreads();
-
-    for (int j = 1; j <= m; ++j) {
-        const float2 *rd = win[(j - 1) & 1];
-        float2 *wr = win[j & 1];
-        const int act_min = j << 27, tile_min = m << 27;
-        float *V0s = a.V0 + (int64_t)(a.s0 + j - 1) * a.plane;
-        float *V1s = a.V1 + (int64_t)(a.s0 + j - 1) * a.plane;
+    };
+    if (a.copy_r && in) store(0, u, v);
+    auto slot = [&](int buf, int j) -> float2 * {
+        if (j == 0) return lds.edge[buf][wave][0];
+        if (j == P - 1) return lds.edge[buf][wave][1];
+        return lds.row[wave][j - 1];
+    };
+    // a wave's LDS writes before its reads of the same row (a wavefront's LDS
+    // accesses are performed in order; this keeps the compiler's order)
+    auto wave_fence = []() {
+        __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+        __builtin_amdgcn_wave_barrier();
+        __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+    };
 #pragma unroll
-        for (int q = 0; q < P; ++q) {
-            const int pkq = pk[q];
-            if (pkq < act_min) continue;
-            const int c = threadIdx.x + q * NT;
-            const float2 mid = rd[c];
-            const float ix = cx[q], iy = cy[q];
-            const float p1 = ix * mid.x, p2 = iy * mid.y;
-            const float dot = p1 + p2;
-            float ur = ix * dot, vr = iy * dot;
-            if (!clipped) {
-                // an updated cell is at least one cell inside the region on
-                // every side and the region inside the image: all four
-                // neighbours exist; reads issued together
-                const float2 nl = rd[c - 1], nr = rd[c + 1], nu = rd[c - PITCH],
-                             nd = rd[c + PITCH];
-                ur = fmaf(nlam, nl.x, ur);
-                vr = fmaf(nlam, nl.y, vr);
-                ur = fmaf(lam, mid.x, ur);
-                vr = fmaf(lam, mid.y, vr);
-                ur = fmaf(nlam, nr.x, ur);
-                vr = fmaf(nlam, nr.y, vr);
-                ur = fmaf(lam, mid.x, ur);
-                vr = fmaf(lam, mid.y, vr);
-                ur = fmaf(nlam, nu.x, ur);
-                vr = fmaf(nlam, nu.y, vr);
-                ur = fmaf(lam, mid.x, ur);
-                vr = fmaf(lam, mid.y, vr);
-                ur = fmaf(nlam, nd.x, ur);
-                vr = fmaf(nlam, nd.y, vr);
-                ur = fmaf(lam, mid.x, ur);
-                vr = fmaf(lam, mid.y, vr);
-            } else {
-                int pkc = pkq;
-                asm volatile("" : "+v"(pkc));  // keep per-cell values out of registers
-                const int gx = gx0 + (pkc & 0xffff), gy = gy0 + ((pkc >> 16) & 0x7ff);
-                if (gx > 0) {
-                    const float2 nb = rd[c - 1];
-                    ur = fmaf(nlam, nb.x, ur);
-                    vr = fmaf(nlam, nb.y, vr);
-                    ur = fmaf(lam, mid.x, ur);
-                    vr = fmaf(lam, mid.y, vr);
-                }
-                if (gx < W - 1) {
-                    const float2 nb = rd[c + 1];
-                    ur = fmaf(nlam, nb.x, ur);
-                    vr = fmaf(nlam, nb.y, vr);
-                    ur = fmaf(lam, mid.x, ur);
-                    vr = fmaf(lam, mid.y, vr);
-                }
-                if (gy > 0) {
-                    const float2 nb = rd[c - PITCH];
-                    ur = fmaf(nlam, nb.x, ur);
-                    vr = fmaf(nlam, nb.y, vr);
-                    ur = fmaf(lam, mid.x, ur);
-                    vr = fmaf(lam, mid.y, vr);
-                }
-                if (gy < H - 1) {
-                    const float2 nb = rd[c + PITCH];
-                    ur = fmaf(nlam, nb.x, ur);
-                    vr = fmaf(nlam, nb.y, vr);
-                    ur = fmaf(lam, mid.x, ur);
-                    vr = fmaf(lam, mid.y, vr);
-                }
+    for (int j = 0; j < P; ++j) slot(0, j)[lane] = make_float2(u[j], v[j]);
+    wave_fence();
+
+    auto steps = [&](auto clip_c) {
+        constexpr bool CLIP = decltype(clip_c)::value;
+        for (int it = 1; it <= m; ++it) {
+            // power it reads edge buffer (it - 1) & 1 and writes the other, which was
+            // last read for power it - 1, before this barrier
+            __syncthreads();
+            const int buf = (it - 1) & 1;
+            // active strip rows [lo, hi): the tile grown by m - it, inside the image
+            const int lo = max(y0 - (m - it), 0) - gy0 - r0;
+            const int hi = min(y1 + (m - it), H) - gy0 - r0;
+            if (lo >= P || hi <= 0) continue;
+            const float2 *const ra =
+                wave == 0 ? lds.edge[buf][wave][0] : lds.edge[buf][wave - 1][1];
+            const float2 *const rb =
+                wave == NW - 1 ? lds.edge[buf][wave][1] : lds.edge[buf][wave + 1][0];
+            const float2 above = ra[lane], below = rb[lane];
+            float nu[P], nv[P];
+#pragma unroll
+            for (int j = 0; j < P; ++j) {
+                const float2 l = slot(buf, j)[li], r = slot(buf, j)[ri];
+                const float2 up = j == 0 ? above : make_float2(u[j > 0 ? j - 1 : 0],
+                                                               v[j > 0 ? j - 1 : 0]);
+                const float2 dn = j == P - 1 ? below : make_float2(u[j < P - 1 ? j + 1 : j],
+                                                                   v[j < P - 1 ? j + 1 : j]);
+                const float p1 = cx[j] * u[j], p2 = cy[j] * v[j];
+                const float dot = p1 + p2;
+                float x = cx[j] * dot, y = cy[j] * dot;
+                auto nb = [&](float2 q, bool has) {
+                    float xn = fmaf(nlam, q.x, x), yn = fmaf(nlam, q.y, y);
+                    xn = fmaf(lam, u[j], xn);
+                    yn = fmaf(lam, v[j], yn);
+                    x = !CLIP || has ? xn : x;
+                    y = !CLIP || has ? yn : y;
+                };
+                const int gy = gy0 + r0 + j;
+                nb(l, has_l);
+                nb(r, has_r);
+                nb(up, gy > 0);
+                nb(dn, gy < H - 1);
+                nu[j] = x;
+                nv[j] = y;
             }
-            wr[c] = make_float2(ur, vr);
-            if (pkq >= tile_min) {  // a tile cell (L = m): this power's output
-                const int64_t g =
-                    (int64_t)(gy0 + ((pkq >> 16) & 0x7ff)) * W + gx0 + (pkq & 0xffff);
-                V0s[g] = ur;
-                V1s[g] = vr;
+#pragma unroll
+            for (int j = 0; j < P; ++j) {
+                u[j] = nu[j];
+                v[j] = nv[j];
+                slot(buf ^ 1, j)[lane] = make_float2(nu[j], nv[j]);
             }
+            if (in) store(a.s0 + it - 1, u, v);
+            wave_fence();
         }
-        // the window written here was last read by power j-1, before the
-        // previous barrier
-        __syncthreads();
-    }
+    };
+    if (gx0 <= 0 || y0 - m <= 0 || x1 + m >= W || y1 + m >= H)
+        steps(std::true_type());
+    else
+        steps(std::false_type());
 }
-
-constexpr int POW_NT = 1024, POW_TW = 64, POW_TH = 32, POW_MMAX = 8;
 
 int launch_hs_precond(const float *diag0, const float *diag1, const float *offdiag,
                       const float *x0, const float *x1, float *y0, float *y1, int H, int W,
@@ -251,7 +264,6 @@ int launch_hs_powers(const float *Ix, const float *Iy, const float *r0, const fl
     a.W = W;
     a.plane = (int64_t)H * W;
     a.tiles_x = (W + POW_TW - 1) / POW_TW;
-    a.ntiles = a.tiles_x * ((H + POW_TH - 1) / POW_TH);
     a.lam_dev = lam_dev;
     a.lam_dtype = lam_dtype;
     a.lam_val = lam_val;
@@ -260,14 +272,26 @@ int launch_hs_powers(const float *Ix, const float *Iy, const float *r0, const fl
         HMX_HIP_TRY(hipMemcpyAsync(V1, r1, a.plane * 4, hipMemcpyDeviceToDevice, s));
         return HMX_OK;
     }
+    // Non-temporal stores pay where the powers outgrow the 256 MB memory-side cache
+    // anyway and a row starts on a 64-byte sector, so that a tile row's 192 bytes are
+    // whole ones.  us for 8 powers, plain / non-temporal: 3840x2160 205 / 155, 2560x1440
+    // (265 MB) 94 / 71, 1920x1080 (149 MB) 37 / 35; 2100x1200, rows off the sectors, 44
+    // / 87; smaller ones alike, and a consumer then finds plain ones cached.
+    const bool nts = (W & 15) == 0 && 2 * (int64_t)steps * a.plane * 4 >= ((int64_t)128 << 20);
     for (int s0 = 1; s0 < steps; s0 += POW_MMAX) {
         a.s0 = s0;
         a.m = std::min(POW_MMAX, steps - s0);
+        a.th = POW_NW * POW_P - 2 * a.m;
+        a.ntiles = a.tiles_x * ((H + a.th - 1) / a.th);
         a.copy_r = s0 == 1;
         a.u0 = s0 == 1 ? r0 : V0 + (int64_t)(s0 - 1) * a.plane;
         a.v0 = s0 == 1 ? r1 : V1 + (int64_t)(s0 - 1) * a.plane;
-        hipLaunchKernelGGL((hs_powers_kernel<POW_NT, POW_TW, POW_TH, POW_MMAX>),
-                           dim3(a.ntiles), dim3(POW_NT), 0, s, a);
+        if (nts)
+            hipLaunchKernelGGL((hs_powers_kernel<POW_NW, POW_P, true>), dim3(a.ntiles),
+                               dim3(POW_NW * 64), 0, s, a);
+        else
+            hipLaunchKernelGGL((hs_powers_kernel<POW_NW, POW_P, false>), dim3(a.ntiles),
+                               dim3(POW_NW * 64), 0, s, a);
         HMX_LAUNCH_CHECK("hs_powers");
     }
     return HMX_OK;
