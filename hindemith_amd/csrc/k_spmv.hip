@@ -234,7 +234,16 @@ __global__ __launch_bounds__(RB_NT) void csr_rowblock_kernel(const int *__restri
 // pass adds a row's 8 partials in slice order.  Within a slice a row's
 // products are added in entry order, so results are deterministic and within
 // the multi-lane bound of the fp64 product.
-constexpr int SL_N = 8, SL_RB = 256, SL_CAP = 2048;
+//
+// What bounds it: gathers through the L1.  73 million of them (2048^2 rows, 17
+// entries a row) miss it and fetch a line from the L2 each (92 % hits there), 0.33
+// per CU and clock, two thirds of what the line width allows; every other phase
+// (row pointers, entries, sums) hides behind them only with all 32 waves of a CU
+// resident.  Both passes: 430 us with 512 rows a work-group and SL_U entries per
+// thread in flight, 485 with 256 rows and one entry at a time; 2 to 4 rows per thread
+// take 421 - 540, fewer resident waves 478 - 625, and a persistent form that
+// prefetches the next rows' entries 550 - 590.
+constexpr int SL_N = 8, SL_RB = 512, SL_U = 4, SL_CAP = SL_RB * SL_U;
 
 __global__ __launch_bounds__(SL_RB) void csr_slice_kernel(int M, const int *__restrict__ sptr,
                                                           const int *__restrict__ sidx,
@@ -257,11 +266,22 @@ __global__ __launch_bounds__(SL_RB) void csr_slice_kernel(int M, const int *__re
     float acc = 0.0f;
     for (int cb = beg; cb < end; cb += SL_CAP) {
         const int m = min(SL_CAP, end - cb);
-        for (int k = tid; k < m; k += SL_RB) {
-            const float d = __builtin_nontemporal_load(sdata + cb + k);
-            const int c = __builtin_nontemporal_load(sidx + cb + k);
-            prod[k] = d * x[c];
+        int c[SL_U];
+        float d[SL_U], xv[SL_U];
+#pragma unroll
+        for (int q = 0; q < SL_U; ++q) {
+            const int k = tid + q * SL_RB;
+            if (k < m) {
+                c[q] = __builtin_nontemporal_load(sidx + cb + k);
+                d[q] = __builtin_nontemporal_load(sdata + cb + k);
+            }
         }
+#pragma unroll
+        for (int q = 0; q < SL_U; ++q)
+            if (tid + q * SL_RB < m) xv[q] = x[c[q]];
+#pragma unroll
+        for (int q = 0; q < SL_U; ++q)
+            if (tid + q * SL_RB < m) prod[tid + q * SL_RB] = d[q] * xv[q];
         __syncthreads();
         const int lo = max(a, cb) - cb, hi = min(e, cb + m) - cb;
         for (int k = lo; k < hi; ++k) acc += prod[k];

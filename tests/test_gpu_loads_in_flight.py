@@ -41,3 +41,31 @@ def test_sum_unroll_edges(n):
     x[-1] = 5.0
     got = K.sum2d(dev(x)).cpu().numpy()
     assert got[0] == np.float32(x.sum(dtype=np.float64))
+
+
+@pytest.mark.parametrize("n", [0, 1, 511, 512, 513, 1535, 2047, 2048, 2049, 4097])
+@pytest.mark.parametrize("rows", [1, 512, 515])
+def test_csr_sliced_chunk_edges_bitexact(n, rows):
+    """n entries of one column slice in the first 512 rows, around the entries a
+    work-group takes at once (one row holds a third of them), one entry per row in
+    another slice: products rounded, then added in entry order, slices in order."""
+    rng = np.random.default_rng(n * 7 + rows)
+    N = 8000  # slices of 1000 columns
+    near = min(rows, 512)
+    lens = np.bincount(rng.integers(0, near, n - n // 3), minlength=rows)
+    lens[near // 2] += n // 3
+    cols, vals, ref = [], [], np.zeros(rows, np.float32)
+    x = rng.normal(size=N).astype(np.float32)
+    for i in range(rows):
+        c = np.concatenate([rng.integers(3000, 4000, lens[i]), rng.integers(7000, N, 1)])
+        v = rng.normal(size=len(c)).astype(np.float32)
+        part = np.float32(0)
+        for p in v[:-1] * x[c[:-1]]:
+            part = np.float32(part + p)
+        ref[i] = np.float32(part + np.float32(v[-1] * x[c[-1]]))
+        cols.append(c)
+        vals.append(v)
+    indptr = np.concatenate([[0], np.cumsum(lens + 1)]).astype(np.int32)
+    sl = K.CSRSlices(indptr, np.concatenate(cols).astype(np.int32), N, "cuda")
+    y = K.csr_spmv_sliced(sl, sl.values(dev(np.concatenate(vals))), dev(x))
+    assert np.array_equal(y.cpu().numpy(), ref)
