@@ -2,7 +2,7 @@
 // stencil: one launch takes the state (u, v) m <= 8 steps before and the gradient
 // after them, recomputes the m forward steps on chip and walks them backwards.
 //
-// What bounds it: vector issue, about 31 VALU instructions per cell and forward
+// What bounds it: vector issue, about 28 VALU instructions per cell and forward
 // step, 22 per reverse step and 14 more on the tile's own rows, and, with one
 // work-group per CU, the loads before the first step.  The two-launch form
 // (hs_adj_tb_kernel after a recompute that stores each step's (ubar, vbar)) is
@@ -69,10 +69,20 @@ __device__ __forceinline__ float adj_recip_of(float r, float d) {
     return r;
 }
 
-template <int NW, int P, int HL, int WPE>
+// Averaging weights held in vector registers, as kRowsVgprWeights; TWO builds: for two
+// weights (hs_two_weights), where eight do not fit.
+template <int P>
+constexpr int kAdjVgprWeights = P == 2 ? 8 : 0;
+
+template <int NW, int P, int HL, int WPE, bool TWO>
 __global__ __launch_bounds__(64 * NW, WPE) void hs_adj_rows_kernel(AdjRowsArgs a) {
     static_assert(P >= 2 && P <= 4, "one group of rows per strip");
     __shared__ AdjRowsLds<NW, P, HL> lds;
+    float w[8];
+#pragma unroll
+    for (int d = 0; d < 8; ++d)
+        w[d] = TWO ? (d % 4 == 0 ? in_vgpr(a.w[d]) : w[d / 4 * 4])
+                   : d < kAdjVgprWeights<P> ? in_vgpr(a.w[d]) : a.w[d];
     const int lane = threadIdx.x & 63;
     const int wave = __builtin_amdgcn_readfirstlane((int)threadIdx.x >> 6);
     const int64_t off = (int64_t)blockIdx.y * a.bstride;
@@ -168,8 +178,8 @@ __global__ __launch_bounds__(64 * NW, WPE) void hs_adj_rows_kernel(AdjRowsArgs a
             const HsTri &up = rows[j], &me = rows[j + 1], &dn = rows[j + 2];
             float x = 0.0f, y = 0.0f;
             auto tap = [&](int d, float2 z) {
-                x = fmaf(a.w[d], z.x, x);
-                y = fmaf(a.w[d], z.y, y);
+                x = fmaf(w[d], z.x, x);
+                y = fmaf(w[d], z.y, y);
             };
             tap(0, me.l);  // HS_RING_OX/OY order
             tap(1, me.r);
@@ -185,11 +195,7 @@ __global__ __launch_bounds__(64 * NW, WPE) void hs_adj_rows_kernel(AdjRowsArgs a
             const float m2 = cy[j] * y;
             const float s1 = m1 + m2;
             s2[j] = s1 + ct[j];
-            const float q0 = s2[j] * cr[j];
-            const float e0 = fmaf(-q0, cd[j], s2[j]);
-            const float q1 = fmaf(e0, cr[j], q0);
-            const float e1 = fmaf(-q1, cd[j], s2[j]);
-            q[j] = fmaf(e1, cr[j], q1);
+            q[j] = hs_quotient(s2[j], cd[j], cr[j]);
         }
         float mx = fabsf(q[0]), mn = mx;
 #pragma unroll
@@ -362,8 +368,8 @@ __global__ __launch_bounds__(64 * NW, WPE) void hs_adj_rows_kernel(AdjRowsArgs a
                 const HsTri &up = rows[j], &me = rows[j + 1], &dn = rows[j + 2];
                 float x = 0.0f, y = 0.0f;
                 auto tap = [&](int d, float2 z) {
-                    x = fmaf(a.w[d], z.x, x);
-                    y = fmaf(a.w[d], z.y, y);
+                    x = fmaf(w[d], z.x, x);
+                    y = fmaf(w[d], z.y, y);
                 };
                 tap(0, me.r);  // the source of tap d lies at -(ox, oy)
                 tap(1, me.l);

@@ -2,19 +2,25 @@
 //
 // The Jacobi step divides a new numerator by the same per-pixel denominator
 // every iteration.  With y = RN(1/b) computed once (an IEEE division), each
-// step takes the quotient from three corrections instead of a full division:
+// step takes the quotient from one correction instead of a full division:
 //
 //   q0 = RN(a*y)                  within 1.5 ulp of a/b
-//   q1 = RN(q0 + RN(a - b*q0)*y)  within 1/2 ulp + 2^-22 ulp of a/b: faithful
-//   q  = RN(q1 + (a - b*q1)*y)    = RN(a/b)
+//   q  = RN(q0 + RN(a - b*q0)*y)  = RN(a/b)
 //
-// The last line is Markstein's theorem (Markstein, "Computation of elementary
-// functions on the IBM RISC System/6000 processor", IBM J. Res. Dev. 34(1),
+// With x, d the significands of a, b in [1, 2): if x >= d then |q0 - a/b| < 1 ulp,
+// and the second line is Markstein's theorem (Markstein, "Computation of
+// elementary functions on the IBM RISC System/6000 processor", IBM J. Res. Dev. 34(1),
 // 1990; restated as Theorem 4.10 of Muller et al., Handbook of
-// Floating-Point Arithmetic): if y is within 1/2 ulp of 1/b, q within one ulp
-// of a/b and r = a - b*q is computed exactly (an fma, exact because q is
-// faithful), then RN(q + r*y) is the correctly rounded quotient.  Its
-// no-overflow / no-underflow conditions hold when |b| lies in [2^-24, 2^24]
+// Floating-Point Arithmetic): if y is within 1/2 ulp of 1/b, q0 within one ulp
+// of a/b and the residual exact, q is the correctly rounded quotient.  If x < d, q0
+// may be 1.5 ulp off; the value rounded to q is then within 7 * 2^-49 of x/d (2^-47
+// from the residual's rounding, 3 * 2^-49 from y's), and x/d is r/(2^25 D) away
+// from the nearest midpoint of two floats, D < 2^24 the divisor's integer
+// significand and r a whole number other than 0: RN(x/d) whenever |r| >= 7.
+// The quotients with smaller |r| are few enough to be enumerated, and
+// fast_div_hard_cases.cpp checks all of them (46.5 M with |r| <= 8, in both
+// halves), so the second correction that a proof for all of them would need is not made.
+// The no-overflow / no-underflow conditions hold when |b| lies in [2^-24, 2^24]
 // and |a/b| in [2^-76, 2^76]: every residual then lies on a grid no finer
 // than 2^-147.  hs_recip gives NaN for any other b, so the quotient is NaN
 // and hs_div_fast reports failure; a failed lane (also a zero, tiny, huge or
@@ -54,14 +60,17 @@ HS_DIV_HD inline float hs_recip(float b) {
     return (ab >= 0x1p-24f && ab <= 0x1p24f) ? y : __builtin_nanf("");
 }
 
+// RN(a / b) if its magnitude lies in [2^-76, 2^76]; the caller checks that.
+HS_DIV_HD inline float hs_quotient(float a, float b, float y) {
+    const float q0 = a * y;
+    const float r = std::fma(-q0, b, a);
+    return std::fma(r, y, q0);
+}
+
 // q = RN(a / b) when the result is true; otherwise q is unspecified and the
 // caller must divide.
 HS_DIV_HD inline bool hs_div_fast(float a, float b, float y, float &q) {
-    const float q0 = a * y;
-    const float r0 = std::fma(-q0, b, a);
-    const float q1 = std::fma(r0, y, q0);
-    const float r1 = std::fma(-q1, b, a);
-    q = std::fma(r1, y, q1);
+    q = hs_quotient(a, b, y);
     const float aq = std::fabs(q);
     return aq >= 0x1p-76f && aq <= 0x1p76f;
 }

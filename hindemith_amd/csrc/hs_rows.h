@@ -10,15 +10,18 @@
 // left and right ones go through LDS, and those are a wave's own rows, so a
 // step has one barrier, for the rows where two waves meet.
 //
-// What bounds it: vector issue.  hs_tile reads 8 neighbours per cell from LDS
+// What bounds it: vector issue, and, where a CU holds one or two tiles, the loads
+// before the first step.  hs_tile reads 8 neighbours per cell from LDS
 // (9 LDS operations of 4 cycles per wave-cell against 33 VALU instructions: the
 // two units are equally loaded and neither hides the other's latency); this
-// body does 3 LDS operations and 31 VALU instructions per cell, no activity
+// body does 3 LDS operations and 28 VALU instructions per cell, no activity
 // test (a row's activity is uniform over its wave) and no per-cell address
 // arithmetic, and its prologue takes ~20 instructions per cell instead of ~47.
-// Measured, us per 8 iterations, hs_tile's variant 24 / this body as
-// hs_rows_choice picks it: 135x240 12.5 / 5.8, 480x640 12.9 / 9.1, 613x977
-// 19.4 / 13.0, 1920x1080 33.6 / 31.2, 3840x2160 112 / 98.
+// Its operands are vector registers (in_vgpr), which two waves issue together.
+// Measured, us per 8 iterations, hs_tile's variant 24 / this body with scalar
+// weights and two corrections per quotient / as it is: 135x240 12.5 / 5.8 / 5.4,
+// 480x640 12.9 / 9.1 / 8.4, 613x977 19.4 / 12.3 / 12.0, 1920x1080 33.6 / 32.3 / 28.2,
+// 3840x2160 112 / 98 / 91.
 //
 // Replicated borders cost nothing per step: the lane a cell takes its left (right)
 // neighbour from is clamped to the image once per tile, a window never starts
@@ -35,6 +38,7 @@
 #pragma once
 
 #include <algorithm>
+#include <cstring>
 #include <type_traits>
 
 #include "hmx_common.h"
@@ -77,10 +81,10 @@ inline RowsGeom hs_rows_geom(int win, int wgs, int H, int W, int k, int B) {
 // Cost in us of a row-register launch of k steps, from what bounds it: the busiest CU
 // takes m tiles, each of which loads its window (load per window row) and in each
 // step pays its barrier (step) and updates its active rows (row each; tile rows
-// + k - 1 on average over the steps) at 31 VALU instructions per wave-row.  Fitted
-// per build to 21 image sizes from 64^2 to 3840x2160 at k = 4 .. 16 (rms error 3-8
-// %): the (build, k) of least cost was the fastest measured one at 17 of them, and
-// within 3.8 % of it at the others.
+// + k - 1 on average over the steps) at 28 VALU instructions per wave-row.  Fitted
+// per build to 21 image sizes from 64^2 to 3840x2160 at k = 4 .. 16, the (build, k)
+// within 10 % of a size's fastest weighing most: the pair of least cost was the
+// fastest measured one at 18 of them, and within 3.5 % of it at the others.
 struct RowsCost {
     float launch, load, row, step;
     float us(int win, int m, int k, float active) const {
@@ -88,14 +92,14 @@ struct RowsCost {
                                     (float)k * (row * std::min(active, (float)win) + step));
     }
 };
-constexpr RowsCost kRowsCost16x2 = {4.33f, 0.0071f, 0.0145f, 0.0925f};   // waves x rows
-constexpr RowsCost kRowsCost16x3 = {2.67f, 0.0383f, 0.0120f, 0.2019f};
-constexpr RowsCost kRowsCost16x4 = {2.59f, 0.0353f, 0.0121f, 0.2527f};
-constexpr RowsCost kRowsCost16x5 = {2.17f, 0.0447f, 0.0117f, 0.2558f};
-constexpr RowsCost kRowsCost8x7 = {4.85f, 0.0218f, 0.0099f, 0.1674f};
-constexpr RowsCost kRowsCost8x9 = {5.50f, 0.0240f, 0.0094f, 0.1741f};
-constexpr RowsCost kRowsCost8x10 = {5.72f, 0.0223f, 0.0098f, 0.2204f};
-constexpr RowsCost kRowsCost16x4two = {5.07f, 0.0216f, 0.0110f, 0.0754f};  // two per CU
+constexpr RowsCost kRowsCost16x2 = {3.95f, 0.0153f, 0.0096f, 0.1289f};   // waves x rows
+constexpr RowsCost kRowsCost16x3 = {2.03f, 0.0484f, 0.0084f, 0.2240f};
+constexpr RowsCost kRowsCost16x4 = {1.88f, 0.0481f, 0.0116f, 0.1789f};
+constexpr RowsCost kRowsCost16x5 = {1.54f, 0.0493f, 0.0117f, 0.2021f};
+constexpr RowsCost kRowsCost8x7 = {4.42f, 0.0186f, 0.0097f, 0.1270f};
+constexpr RowsCost kRowsCost8x9 = {4.99f, 0.0210f, 0.0090f, 0.1318f};
+constexpr RowsCost kRowsCost8x10 = {5.49f, 0.0180f, 0.0092f, 0.1958f};
+constexpr RowsCost kRowsCost16x4two = {4.14f, 0.0225f, 0.0083f, 0.1409f};  // two per CU
 
 // LDS of one work-group: the first and last row of every wave's strip, double
 // buffered (another wave reads them), and its other rows (read by the wave alone).
@@ -117,6 +121,23 @@ struct HsSetup {
 constexpr int HS_CUBE_OX[2][4] = {{0, 1, 0, 1}, {0, 0, 1, 1}};
 constexpr int HS_CUBE_OY[2][4] = {{0, 0, 1, 1}, {0, 1, 0, 1}};
 
+// 16 of a cell's 28 VALU instructions take a weight, and run at up to twice the rate
+// when it is in a vector register (in_vgpr).  A build holds as many of the eight
+// there as its register budget leaves; the tall and the two-per-CU ones, which
+// have room for 2 to 6, also come as TWO builds for stencils whose first four and last
+// four weights are equal (Horn and Schunck's own), which need two registers.
+// Per 8 iterations, scalar weights / as many as fit / TWO: 1920x1080 (16 x 4 rows) 32.3 /
+// 29.7 / 27.8 us, 2560x1440 (8 x 9) 50.4 / 47.2 / 45.2.
+template <int NW, int P, bool PRE>
+constexpr int kRowsVgprWeights = NW == 16 && !PRE ? 2 : P == 10 ? 2 : P == 9 ? 6 : 8;
+template <int NW, int P, bool PRE>
+constexpr bool kRowsTwoBuild = kRowsVgprWeights<NW, P, PRE> < 8;
+inline bool hs_two_weights(const float *w) {
+    for (int d = 1; d < 4; ++d)
+        if (std::memcmp(w + d, w, 4) || std::memcmp(w + 4 + d, w + 4, 4)) return false;
+    return true;
+}
+
 // a window row around one column: left neighbour, cell, right neighbour
 struct HsTri {
     float2 l, c, r;
@@ -135,11 +156,20 @@ struct HsTri {
 // pass is one launch of latency for an image of any ordinary size (135x240 11
 // us, 480x640 14.6 us, against 11 and 20 B/px of traffic) and this is
 // 27 more VALU instructions per cell of one launch.
-template <int NW, int P, bool PRE, int G, bool LOUT = false, bool SETUP = false>
+template <int NW, int P, bool PRE, int G, bool TWO, bool LOUT = false, bool SETUP = false>
 __device__ __forceinline__ void hs_rows_tile(const HsImage &a, int txi, int tyi, int tw, int th,
-                                             int k, const float (&w)[8], HsRowsLds<NW, P> &lds,
-                                             const HsSetup *su = nullptr) {
+                                             int k, const float (&weights)[8],
+                                             HsRowsLds<NW, P> &lds, const HsSetup *su = nullptr) {
     static_assert(P >= 2, "a strip has a first and a last row");
+    constexpr int WV = kRowsVgprWeights<NW, P, PRE>;
+    float w[8];
+#pragma unroll
+    for (int d = 0; d < 8; ++d) {
+        if (TWO)
+            w[d] = d % 4 == 0 ? in_vgpr(weights[d]) : w[d / 4 * 4];
+        else
+            w[d] = d < WV ? in_vgpr(weights[d]) : weights[d];
+    }
     const int lane = threadIdx.x & 63;
     const int wave = __builtin_amdgcn_readfirstlane((int)threadIdx.x >> 6);
     const int H = a.H, W = a.W;
@@ -336,11 +366,7 @@ __device__ __forceinline__ void hs_rows_tile(const HsImage &a, int txi, int tyi,
                         const float s1 = m1 + m2;
                         s2[i] = s1 + ct[j];
                         // hs_div_fast's quotient; its range check follows
-                        const float q0 = s2[i] * cr[j];
-                        const float e0 = fmaf(-q0, cd[j], s2[i]);
-                        const float q1 = fmaf(e0, cr[j], q0);
-                        const float e1 = fmaf(-q1, cd[j], s2[i]);
-                        q[i] = fmaf(e1, cr[j], q1);
+                        q[i] = hs_quotient(s2[i], cd[j], cr[j]);
                     }
                     float mx = fabsf(q[0]), mn = mx;
 #pragma unroll

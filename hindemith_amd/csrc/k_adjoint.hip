@@ -538,12 +538,12 @@ struct AdjTaps {
 struct AdjRowsBuild {
     int rows;  // window rows
     float launch, tile, step, row;
-    void (*kernel)(AdjRowsArgs);
+    void (*kernel[2])(AdjRowsArgs);  // for any eight weights, and for two (hs_two_weights)
 };
 static const AdjRowsBuild kAdjRows[] = {
-    {32, 1.33f, 3.77f, 0.218f, 0.0350f, hs_adj_rows_kernel<16, 2, 0, 4>},
-    {48, 0.66f, 5.65f, 0.391f, 0.0336f, hs_adj_rows_kernel<16, 3, 0, 4>},
-    {64, 0.0f, 7.47f, 0.512f, 0.0352f, hs_adj_rows_kernel<16, 4, 3, 4>},
+    {32, 1.33f, 3.77f, 0.218f, 0.0350f, {hs_adj_rows_kernel<16, 2, 0, 4, false>, hs_adj_rows_kernel<16, 2, 0, 4, false>}},
+    {48, 0.66f, 5.65f, 0.391f, 0.0336f, {hs_adj_rows_kernel<16, 3, 0, 4, false>, hs_adj_rows_kernel<16, 3, 0, 4, true>}},
+    {64, 0.0f, 7.47f, 0.512f, 0.0352f, {hs_adj_rows_kernel<16, 4, 3, 4, false>, hs_adj_rows_kernel<16, 4, 3, 4, true>}},
 };
 
 // One fused reverse block of a.m steps of B images, by the build with the least
@@ -569,7 +569,7 @@ static int launch_adj_rows(AdjRowsArgs &a, int B, hipStream_t s) {
             a.ntiles = g.ntiles;
         }
     }
-    hipLaunchKernelGGL(best->kernel, dim3((unsigned)a.ntiles, B), dim3(1024), 0, s, a);
+    hipLaunchKernelGGL(best->kernel[hs_two_weights(a.w) ? 1 : 0], dim3((unsigned)a.ntiles, B), dim3(1024), 0, s, a);
     HMX_LAUNCH_CHECK("hs_adj_rows");
     return HMX_OK;
 }

@@ -393,7 +393,7 @@ struct MultiRowsArgs {
     float cube[12];   // Dx, Dy, Dt weights (HsSetup)
 };
 
-template <int NW, int P, bool PRE, int G, bool FIRST>
+template <int NW, int P, bool PRE, int G, bool TWO, bool FIRST>
 __device__ __forceinline__ void multi_rows_body(const MultiRowsArgs &b, int ph, int kk) {
     __shared__ HsRowsLds<NW, P> lds;
     // phases alternate the walk over each XCD's share of the list
@@ -412,19 +412,19 @@ __device__ __forceinline__ void multi_rows_body(const MultiRowsArgs &b, int ph, 
     }
     const int t = w - D.tile_base;
     const int tyi = t / D.tiles_x, txi = t - tyi * D.tiles_x;
-    hs_rows_tile<NW, P, PRE, G, false, FIRST>(im, txi, tyi, D.tw, D.th, kk, b.w, lds, &su);
+    hs_rows_tile<NW, P, PRE, G, TWO, false, FIRST>(im, txi, tyi, D.tw, D.th, kk, b.w, lds, &su);
 }
 
-template <int NW, int P, bool PRE, int G, int WPE>
+template <int NW, int P, bool PRE, int G, int WPE, bool TWO>
 __global__ __launch_bounds__(64 * NW, WPE) void hs_multi_rows_kernel(MultiRowsArgs b, int ph,
                                                                      int kk) {
-    multi_rows_body<NW, P, PRE, G, false>(b, ph, kk);
+    multi_rows_body<NW, P, PRE, G, TWO, false>(b, ph, kk);
 }
 
-template <int NW, int P, bool PRE, int G, int WPE>
+template <int NW, int P, bool PRE, int G, int WPE, bool TWO>
 __global__ __launch_bounds__(64 * NW, WPE) void hs_multi_rows_first_kernel(MultiRowsArgs b, int ph,
                                                                            int kk) {
-    multi_rows_body<NW, P, PRE, G, true>(b, ph, kk);
+    multi_rows_body<NW, P, PRE, G, TWO, true>(b, ph, kk);
 }
 
 // ---------------------------------------------------------------------------
@@ -438,8 +438,9 @@ struct BVariant {
     // CU, its launch cost, phase and first phase
     int nw, rows, wgs;
     RowsCost cost;
-    void (*rphase)(MultiRowsArgs, int, int);
-    void (*rfirst)(MultiRowsArgs, int, int);
+    // (each for any eight weights, and for two: hs_two_weights)
+    void (*rphase[2])(MultiRowsArgs, int, int);
+    void (*rfirst[2])(MultiRowsArgs, int, int);
 };
 
 #define HB_V(NT, TW, TH, K, WPE)                                                          \
@@ -464,8 +465,11 @@ struct BVariant {
 // row-register stepped form
 #define HB_R(NW, P, PRE, G, WPE, WGS, KMAX, COST)                                         \
     {64 * NW, 48, NW * P - 16, KMAX, 0, {nullptr, nullptr}, nullptr, {nullptr, nullptr},  \
-     NW, P, WGS, COST, hs_multi_rows_kernel<NW, P, PRE, G, WPE>,                    \
-     hs_multi_rows_first_kernel<NW, P, PRE, G, WPE>}
+     NW, P, WGS, COST,                                                                    \
+     {hs_multi_rows_kernel<NW, P, PRE, G, WPE, false>,                                    \
+      hs_multi_rows_kernel<NW, P, PRE, G, WPE, kRowsTwoBuild<NW, P, PRE>>},               \
+     {hs_multi_rows_first_kernel<NW, P, PRE, G, WPE, false>,                              \
+      hs_multi_rows_first_kernel<NW, P, PRE, G, WPE, kRowsTwoBuild<NW, P, PRE>>}}
 static const BVariant kBVariants[] = {
     HB_V(1024, 64, 32, 4, 8),   // 0: two work-groups per CU
     HB_V(1024, 64, 32, 8, 8),   // 1: two work-groups per CU
@@ -604,10 +608,11 @@ static int launch_batch(const BatchPlan &P, const SetupTaps &st, const Taps &av,
         if (!hs_cube_taps(st.dx, st.dy, st.dt, su))  // (the variant is chosen for them)
             return fail(HMX_ERR_UNSUPPORTED, "hmx_hs_batched: not the canonical stencils");
         std::copy(su.w, su.w + 12, r.cube);
+        const int two = hs_two_weights(r.w) ? 1 : 0;
         for (int ph = 0; ph < nph; ++ph) {
             const int kk = std::min(P.k, iters - ph * P.k);
-            hipLaunchKernelGGL(ph == 0 ? V.rfirst : V.rphase, dim3(P.total_tiles), dim3(V.nt), 0,
-                               s, r, ph, kk);
+            hipLaunchKernelGGL(ph == 0 ? V.rfirst[two] : V.rphase[two], dim3(P.total_tiles),
+                               dim3(V.nt), 0, s, r, ph, kk);
             HMX_LAUNCH_CHECK("hs_multi_rows");
         }
         return HMX_OK;
@@ -639,7 +644,7 @@ static int launch_batch(const BatchPlan &P, const SetupTaps &st, const Taps &av,
 static int resident_per_cu(int variant, int nd, int device, int &api, int &own, int &cus) {
     const BVariant &V = kBVariants[variant];
     const void *kern = V.kernel[0] ? reinterpret_cast<const void *>(V.kernel[nd == 8 ? 0 : 1])
-                       : V.nw      ? reinterpret_cast<const void *>(V.rphase)
+                       : V.nw      ? reinterpret_cast<const void *>(V.rphase[0])
                                    : reinterpret_cast<const void *>(V.phase[nd == 8 ? 0 : 1]);
     HMX_HIP_TRY(hipOccupancyMaxActiveBlocksPerMultiprocessor(&api, kern, V.nt, 0));
     if (!V.kernel[0]) {  // stepped form: no residency requirement

@@ -129,7 +129,7 @@ __global__ __launch_bounds__(NT) void hs_strip_kernel(HsArgs a, Taps taps) {
 
 // Row-register form (hs_rows.h): a window of 64 columns x NW * P rows, the canonical
 // 8-tap averaging offsets.  WPE: waves per SIMD the build is held to.
-template <int NW, int P, bool PRE, int G, bool LOUT, bool SETUP>
+template <int NW, int P, bool PRE, int G, bool TWO, bool LOUT, bool SETUP>
 __device__ __forceinline__ void hs_rows_body(const HsArgs &a, const Taps &taps, const HsSetup *su) {
     __shared__ HsRowsLds<NW, P> lds;
     const int64_t off = (int64_t)blockIdx.y * a.bstride;
@@ -164,19 +164,19 @@ __device__ __forceinline__ void hs_rows_body(const HsArgs &a, const Taps &taps, 
     for (int d = 0; d < 8; ++d) w[d] = taps.w[d];
     const int t = xcd_remap(blockIdx.x, a.ntiles, a.rev);
     const int tyi = t / a.tiles_x, txi = t - tyi * a.tiles_x;
-    hs_rows_tile<NW, P, PRE, G, LOUT, SETUP>(im, txi, tyi, a.tw, a.th, a.k, w, lds, &so);
+    hs_rows_tile<NW, P, PRE, G, TWO, LOUT, SETUP>(im, txi, tyi, a.tw, a.th, a.k, w, lds, &so);
 }
 
-template <int NW, int P, bool PRE, int G, int WPE, bool LOUT = false>
+template <int NW, int P, bool PRE, int G, int WPE, bool TWO, bool LOUT = false>
 __global__ __launch_bounds__(64 * NW, WPE) void hs_rows_kernel(HsArgs a, Taps taps) {
-    hs_rows_body<NW, P, PRE, G, LOUT, false>(a, taps, nullptr);
+    hs_rows_body<NW, P, PRE, G, TWO, LOUT, false>(a, taps, nullptr);
 }
 
 // a solve's first launch, computing the derivative planes as well (HsSetup)
-template <int NW, int P, bool PRE, int G, int WPE>
+template <int NW, int P, bool PRE, int G, int WPE, bool TWO>
 __global__ __launch_bounds__(64 * NW, WPE) void hs_rows_first_kernel(HsArgs a, Taps taps,
                                                                      HsSetup su) {
-    hs_rows_body<NW, P, PRE, G, false, true>(a, taps, &su);
+    hs_rows_body<NW, P, PRE, G, TWO, false, true>(a, taps, &su);
 }
 
 // ---------------------------------------------------------------------------
@@ -295,12 +295,14 @@ struct HsVariant {
     void (*ring)(HsArgs, Taps);       // ring-ordered kernel for the canonical 8 taps, or null
     bool persist;                     // whole solve in one persistent launch (hs_persist_run)
     // Row-register forms: waves per work-group and rows per wave of the canonical
-    // stencil's kernel (in `ring`; other stencils run variant 24's kernels), the
+    // stencil's kernels (other stencils run variant 24's), the
     // work-groups of it a CU holds, and its launch cost.  Zero for the others.
     int nw, rows, wgs;
     RowsCost cost;
-    void (*first)(HsArgs, Taps, HsSetup);  // a solve's first launch, with its setup
-    void (*lin)(HsArgs, Taps);             // with the linearisation output, or null
+    // each for any eight weights, and for two (hs_two_weights)
+    void (*step[2])(HsArgs, Taps);
+    void (*first[2])(HsArgs, Taps, HsSetup);  // a solve's first launch, with its setup
+    void (*lin[2])(HsArgs, Taps);             // with the linearisation output, or null
 };
 
 // tap count -> kernel slot (straight-line kernels for the common stencils)
@@ -340,15 +342,22 @@ static int tap_class(int nd) {
       hs_strip_kernel<NT, TW, TH, K, S, 8>, hs_strip_kernel<NT, TW, TH, K, S, 9>,      \
       hs_strip_kernel<NT, TW, TH, K, S, 0>}, nullptr}
 // row-register forms: the canonical stencil's kernel, and variant 24's for others
-#define HS_R(NW, P, PRE, G, WPE, WGS, KMAX, COST, LIN)                                  \
+#define HS_R(NW, P, PRE, G, WPE, WGS, KMAX, COST, ...)                                  \
     {1024, 64, 32, KMAX, 0,                                                             \
      {hs_tb_kernel<1024, 64, 32, 8, 4, false, true, true>,                              \
       hs_tb_kernel<1024, 64, 32, 8, 5, false, true, true>,                              \
       hs_tb_kernel<1024, 64, 32, 8, 8, false, true, true>,                              \
       hs_tb_kernel<1024, 64, 32, 8, 9, false, true, true>,                              \
       hs_tb_kernel<1024, 64, 32, 8, 0, false, true, true>},                             \
-     hs_rows_kernel<NW, P, PRE, G, WPE>, false, NW, P, WGS, COST,                 \
-     hs_rows_first_kernel<NW, P, PRE, G, WPE>, LIN}
+     nullptr, false, NW, P, WGS, COST,                                                  \
+     {hs_rows_kernel<NW, P, PRE, G, WPE, false>,                                        \
+      hs_rows_kernel<NW, P, PRE, G, WPE, kRowsTwoBuild<NW, P, PRE>>},                   \
+     {hs_rows_first_kernel<NW, P, PRE, G, WPE, false>,                                  \
+      hs_rows_first_kernel<NW, P, PRE, G, WPE, kRowsTwoBuild<NW, P, PRE>>},             \
+     {__VA_ARGS__}}
+#define HS_RL(NW, P, PRE, G, WPE)                                                       \
+    hs_rows_kernel<NW, P, PRE, G, WPE, false, true>,                                    \
+        hs_rows_kernel<NW, P, PRE, G, WPE, kRowsTwoBuild<NW, P, PRE>, true>
 static const HsVariant kVariants[] = {
     HS_V(256, 64, 16, 1),     // 0: one iteration per launch (plain sweep)
     HS_V(256, 64, 32, 4),     // 1
@@ -398,28 +407,29 @@ static const HsVariant kVariants[] = {
      nullptr, true},
     // 29-36: row-register forms, chosen by hs_rows_choice.  One work-group of 16
     // waves per CU, for images that give a CU at most one tile: the window's
-    // height sets how many pixels a CU takes (neighbours prefetched; 56 to 110
+    // height sets how many pixels a CU takes (neighbours prefetched; 64 to 118
     // VGPRs).  Two work-groups per CU for larger images, so that one's loads
     // and barriers overlap the other's steps: 8 waves at up to 128 VGPRs, or 16 at
-    // 61 (one row at a time; its linearisation build would spill).
+    // 63 (one row at a time).  The linearisation builds of the last two would spill.
     HS_R(16, 2, true, 2, 4, 1, 12, kRowsCost16x2,
-         (hs_rows_kernel<16, 2, true, 2, 4, true>)),   // 29: window 64 x 32
+         HS_RL(16, 2, true, 2, 4)),   // 29: window 64 x 32
     HS_R(16, 3, true, 3, 4, 1, 16, kRowsCost16x3,
-         (hs_rows_kernel<16, 3, true, 3, 4, true>)),   // 30: 64 x 48
+         HS_RL(16, 3, true, 3, 4)),   // 30: 64 x 48
     HS_R(16, 4, true, 4, 4, 1, 16, kRowsCost16x4,
-         (hs_rows_kernel<16, 4, true, 4, 4, true>)),   // 31: 64 x 64
+         HS_RL(16, 4, true, 4, 4)),   // 31: 64 x 64
     HS_R(16, 5, true, 5, 4, 1, 16, kRowsCost16x5,
-         (hs_rows_kernel<16, 5, true, 5, 4, true>)),   // 32: 64 x 80
+         HS_RL(16, 5, true, 5, 4)),   // 32: 64 x 80
     HS_R(8, 7, false, 4, 4, 2, 16, kRowsCost8x7,
-         (hs_rows_kernel<8, 7, false, 4, 4, true>)),   // 33: 64 x 56
+         HS_RL(8, 7, false, 4, 4)),   // 33: 64 x 56
     HS_R(8, 9, false, 3, 4, 2, 16, kRowsCost8x9,
-         (hs_rows_kernel<8, 9, false, 3, 4, true>)),   // 34: 64 x 72
+         HS_RL(8, 9, false, 3, 4)),   // 34: 64 x 72
     HS_R(8, 10, false, 2, 4, 2, 16, kRowsCost8x10,
-         (hs_rows_kernel<8, 10, false, 2, 4, true>)),  // 35: 64 x 80
+         nullptr, nullptr),  // 35: 64 x 80
     HS_R(16, 4, false, 1, 8, 2, 16, kRowsCost16x4two,
-         nullptr),  // 36: 64 x 64
+         nullptr, nullptr),  // 36: 64 x 64
 };
 #undef HS_R
+#undef HS_RL
 #undef HS_V
 #undef HS_D
 #undef HS_S
@@ -481,7 +491,7 @@ static void hs_rows_choice(int H, int W, int B, int iters, bool in_place, bool l
     const float copy_us = in_place ? 3.0f + 16e-6f / 4.0f * (float)H * (float)W * (float)B : 0.0f;
     for (int vi = 0; vi < kNumVariants; ++vi) {
         const HsVariant &V = kVariants[vi];
-        if (!V.nw || (lin && !V.lin)) continue;
+        if (!V.nw || (lin && !V.lin[0])) continue;
         const int k_lo = std::min(iters, 5), k_hi = std::min(iters, V.kmax);
         for (int n = (iters + k_hi - 1) / k_hi; n <= (iters + k_lo - 1) / k_lo; ++n) {
             const int kk = (iters + n - 1) / n;
@@ -541,7 +551,9 @@ int launch_hs_tb(int variant, const float *Ix, const float *Iy, const float *It,
     a.tw = V.tw;
     a.th = V.th;
     if (V.ring && hs_ring_taps(taps)) kern = V.ring;
+    const int two = V.nw && hs_two_weights(taps.w) ? 1 : 0;
     if (hs_runs_rows(V, taps)) {
+        kern = V.step[two];
         const RowsGeom g = hs_rows_geom(V.nw * V.rows, V.wgs, H, W, k, B);
         a.tw = g.tw;
         a.th = g.th;
@@ -550,7 +562,7 @@ int launch_hs_tb(int variant, const float *Ix, const float *Iy, const float *It,
         nt = 64 * V.nw;
     }
     if (lub && hs_runs_rows(V, taps)) {
-        kern = V.lin;
+        kern = V.lin[two];
     } else if (lub) {
         // other linearisation outputs exist only for the 1024-thread 64x32 k<=8
         // shape (with the reciprocal quotient: the same bits as the division,
@@ -567,7 +579,7 @@ int launch_hs_tb(int variant, const float *Ix, const float *Iy, const float *It,
         kern = kLinKernels[tap_class(taps.nd)];
     }
     if (setup)
-        hipLaunchKernelGGL(V.first, dim3(a.ntiles, B), dim3(nt), 0, s, a, taps, *setup);
+        hipLaunchKernelGGL(V.first[two], dim3(a.ntiles, B), dim3(nt), 0, s, a, taps, *setup);
     else
         hipLaunchKernelGGL(kern, dim3(a.ntiles, B), dim3(nt), 0, s, a, taps);
     HMX_LAUNCH_CHECK("hs_tb");
