@@ -297,6 +297,14 @@ struct ScalarStmt {
     int op, dst, a, b;  // symbol ids (b = -1 for unary/copy)
 };
 
+// A result's host copy.  Pinned, and kept while the record lives: a fresh pageable one per
+// run costs a page fault and a clearing pass per page besides a staged copy
+// (1080p, two planes of flow: see hmx_run).
+struct HostResult {
+    char *p = nullptr;
+    int64_t cap = 0, bytes = 0;
+};
+
 struct Record {
     int id = 0, device = 0;
     hipStream_t stream = nullptr;
@@ -308,7 +316,8 @@ struct Record {
     std::vector<std::vector<ScalarStmt>> sprogs;
     std::vector<Node> plan;
     std::vector<int> returns;
-    std::vector<std::vector<char>> results;
+    std::vector<HostResult> results;  // kept from run to run
+    int nresults = 0;                 // results of the last run
     std::map<int, std::vector<int>> reads;  // sym -> statement indices reading it
     std::set<int> renamed;
     float *hs_work = nullptr;
@@ -1172,10 +1181,35 @@ static int allocate(Record &R) {
     return HMX_OK;
 }
 
+// The host copies that the plan's RETURN nodes need.
+static int allocate_results(Record &R, const std::vector<Node> &nodes) {
+    for (const Node &n : nodes) {
+        if (n.t == Node::RETURN) {
+            if (R.results.size() < n.syms.size()) R.results.resize(n.syms.size());
+            for (size_t i = 0; i < n.syms.size(); ++i) {
+                HostResult &h = R.results[i];
+                const int64_t bytes = R.syms[n.syms[i]].bytes[0];
+                if (h.cap >= bytes) continue;
+                if (h.p) (void)hipHostFree(h.p);
+                h = HostResult();
+                HMX_HIP_TRY(hipHostMalloc((void **)&h.p, (size_t)bytes, hipHostMallocDefault));
+                h.cap = bytes;
+            }
+        }
+        int rc = allocate_results(R, n.body);
+        if (rc) return rc;
+    }
+    return HMX_OK;
+}
+
 static void release_record(Record &R) {
     if (R.stream) (void)hipStreamSynchronize(R.stream);
     for (void *p : R.allocs) (void)hipFree(p);
     R.allocs.clear();
+    for (HostResult &h : R.results)
+        if (h.p) (void)hipHostFree(h.p);
+    R.results.clear();
+    R.nresults = 0;
     for (Group &g : R.groups) g.partials = nullptr;
     if (R.stream) (void)hipStreamDestroy(R.stream);
     R.stream = nullptr;
@@ -1374,13 +1408,16 @@ static int exec_node(Record &R, Node &n) {
                     s.kind != HMX_KIND_SCALAR && s.kind != HMX_KIND_ARRAY3D)
                     return fail(HMX_ERR_UNSUPPORTED, "returning " + s.name +
                                                          " (a matrix/stencil) is not supported");
-                R.results[i].resize((size_t)s.bytes[0]);
+                HostResult &h = R.results[i];
+                h.bytes = s.bytes[0];
                 const void *src = (s.kind == HMX_KIND_SCALAR || s.kind == HMX_KIND_ARRAY3D)
                                       ? s.dev[0]
                                       : (void *)s.cur_buf();
-                HMX_HIP_TRY(hipMemcpyAsync(R.results[i].data(), src, (size_t)s.bytes[0],
-                                           hipMemcpyDeviceToHost, R.stream));
+                if (s.bytes[0] > 0)
+                    HMX_HIP_TRY(hipMemcpyAsync(h.p, src, (size_t)s.bytes[0],
+                                               hipMemcpyDeviceToHost, R.stream));
             }
+            R.nresults = (int)n.syms.size();
             return HMX_OK;
         }
     }
@@ -1576,6 +1613,7 @@ extern "C" int hmx_compile(int rec, const char *symtab_xml, const char *sm_xml,
     HMX_HIP_TRY(hipStreamCreateWithFlags(&R->stream, hipStreamNonBlocking));
     mark_buffers(*R, R->plan);
     rc = allocate(*R);
+    if (!rc) rc = allocate_results(*R, R->plan);
     const bool jit = program_jit_enabled();
     for (Group &g : R->groups) {
         if (rc) break;
@@ -1676,7 +1714,7 @@ extern "C" int hmx_run(int rec) {
         s.cur = 0;
     }
     for (Sym &s : R->syms) s.cur = 0;
-    R->results.clear();
+    R->nresults = 0;
     R->returns.clear();
     int rc = exec_nodes(*R, R->plan);
     hipError_t e = hipStreamSynchronize(R->stream);
@@ -1693,7 +1731,7 @@ extern "C" int hmx_result_count(int rec, int *n) {
     Record *R = find_record(rec);
     if (!R) return fail(HMX_ERR_NOT_FOUND, "no record " + std::to_string(rec));
     if (!n) return fail(HMX_ERR_INVALID, "null n");
-    *n = (int)R->results.size();
+    *n = R->nresults;
     return HMX_OK;
 }
 
@@ -1721,12 +1759,12 @@ extern "C" int hmx_result_info(int rec, int i, int *kind, int *dtype, int *ndim,
 extern "C" int hmx_result_read(int rec, int i, void *host, int64_t nbytes) {
     Record *R = find_record(rec);
     if (!R) return fail(HMX_ERR_NOT_FOUND, "no record " + std::to_string(rec));
-    if (i < 0 || i >= (int)R->results.size()) return fail(HMX_ERR_NOT_FOUND, "no such result");
-    if (nbytes != (int64_t)R->results[i].size())
+    if (i < 0 || i >= R->nresults) return fail(HMX_ERR_NOT_FOUND, "no such result");
+    if (nbytes != R->results[i].bytes)
         return fail(HMX_ERR_INVALID, "result " + std::to_string(i) + ": expected " +
-                                         std::to_string(R->results[i].size()) + " bytes");
+                                         std::to_string(R->results[i].bytes) + " bytes");
     if (!host) return fail(HMX_ERR_INVALID, "null destination");
-    std::memcpy(host, R->results[i].data(), (size_t)nbytes);
+    std::memcpy(host, R->results[i].p, (size_t)nbytes);
     return HMX_OK;
 }
 
