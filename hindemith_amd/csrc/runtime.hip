@@ -1401,7 +1401,6 @@ static int exec_node(Record &R, Node &n) {
         }
         case Node::RETURN: {
             R.returns = n.syms;
-            R.results.assign(n.syms.size(), {});
             for (size_t i = 0; i < n.syms.size(); ++i) {
                 Sym &s = R.syms[n.syms[i]];
                 if (s.kind != HMX_KIND_ARRAY2D && s.kind != HMX_KIND_ARRAY &&
