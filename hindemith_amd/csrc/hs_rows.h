@@ -14,14 +14,14 @@
 // before the first step.  hs_tile reads 8 neighbours per cell from LDS
 // (9 LDS operations of 4 cycles per wave-cell against 33 VALU instructions: the
 // two units are equally loaded and neither hides the other's latency); this
-// body does 3 LDS operations and 28 VALU instructions per cell, no activity
-// test (a row's activity is uniform over its wave) and no per-cell address
-// arithmetic, and its prologue takes ~20 instructions per cell instead of ~47.
+// body does 3 LDS operations and 29 VALU instructions per cell, no activity
+// test (a wave's strip is active in its first steps and not after them) and no
+// address arithmetic (every LDS access is one of three registers plus a constant), and its prologue takes ~20 instructions per cell instead of ~47.
 // Its operands are vector registers (in_vgpr), which two waves issue together.
 // Measured, us per 8 iterations, hs_tile's variant 24 / this body with scalar
-// weights and two corrections per quotient / as it is: 135x240 12.5 / 5.8 / 5.4,
-// 480x640 12.9 / 9.1 / 8.4, 613x977 19.4 / 12.3 / 12.0, 1920x1080 33.6 / 32.3 / 28.2,
-// 3840x2160 112 / 98 / 91.
+// weights, two corrections per quotient and a branch per row / as it is: 135x240
+// 12.5 / 5.8 / 5.1, 480x640 12.9 / 9.1 / 7.8, 613x977 19.4 / 12.3 / 10.8, 1920x1080
+// 33.6 / 32.3 / 26.7, 3840x2160 112 / 98 / 90.
 //
 // Replicated borders cost nothing per step: the lane a cell takes its left (right)
 // neighbour from is clamped to the image once per tile, a window never starts
@@ -81,10 +81,10 @@ inline RowsGeom hs_rows_geom(int win, int wgs, int H, int W, int k, int B) {
 // Cost in us of a row-register launch of k steps, from what bounds it: the busiest CU
 // takes m tiles, each of which loads its window (load per window row) and in each
 // step pays its barrier (step) and updates its active rows (row each; tile rows
-// + k - 1 on average over the steps) at 28 VALU instructions per wave-row.  Fitted
+// + k - 1 on average over the steps) at 29 VALU instructions per wave-row.  Fitted
 // per build to 21 image sizes from 64^2 to 3840x2160 at k = 4 .. 16, the (build, k)
 // within 10 % of a size's fastest weighing most: the pair of least cost was the
-// fastest measured one at 18 of them, and within 3.5 % of it at the others.
+// fastest measured one at 17 of them, and within 3.8 % of it at the others.
 struct RowsCost {
     float launch, load, row, step;
     float us(int win, int m, int k, float active) const {
@@ -92,17 +92,29 @@ struct RowsCost {
                                     (float)k * (row * std::min(active, (float)win) + step));
     }
 };
-constexpr RowsCost kRowsCost16x2 = {3.95f, 0.0153f, 0.0096f, 0.1289f};   // waves x rows
-constexpr RowsCost kRowsCost16x3 = {2.03f, 0.0484f, 0.0084f, 0.2240f};
-constexpr RowsCost kRowsCost16x4 = {1.88f, 0.0481f, 0.0116f, 0.1789f};
-constexpr RowsCost kRowsCost16x5 = {1.54f, 0.0493f, 0.0117f, 0.2021f};
-constexpr RowsCost kRowsCost8x7 = {4.42f, 0.0186f, 0.0097f, 0.1270f};
-constexpr RowsCost kRowsCost8x9 = {4.99f, 0.0210f, 0.0090f, 0.1318f};
-constexpr RowsCost kRowsCost8x10 = {5.49f, 0.0180f, 0.0092f, 0.1958f};
-constexpr RowsCost kRowsCost16x4two = {4.14f, 0.0225f, 0.0083f, 0.1409f};  // two per CU
+constexpr RowsCost kRowsCost16x2 = {2.41f, 0.0472f, 0.0103f, 0.1530f};   // waves x rows
+constexpr RowsCost kRowsCost16x3 = {2.01f, 0.0468f, 0.0084f, 0.1960f};
+constexpr RowsCost kRowsCost16x4 = {1.86f, 0.0484f, 0.0089f, 0.1974f};
+constexpr RowsCost kRowsCost16x5 = {1.56f, 0.0488f, 0.0087f, 0.2316f};
+constexpr RowsCost kRowsCost8x7 = {4.68f, 0.0152f, 0.0094f, 0.1509f};
+constexpr RowsCost kRowsCost8x9 = {5.23f, 0.0166f, 0.0087f, 0.1924f};
+constexpr RowsCost kRowsCost16x4two = {3.88f, 0.0235f, 0.0087f, 0.0956f};  // two per CU
 
-// LDS of one work-group: the first and last row of every wave's strip, double
-// buffered (another wave reads them), and its other rows (read by the wave alone).
+// LDS of one work-group in hs_rows_tile: per wave the first and last row of its strip, double
+// buffered (the neighbouring waves read them), and its other rows (read by the wave
+// alone), between a wave above the first and one below the last.
+template <int NW, int P>
+struct HsStripLds {
+    float2 wave[NW + 2][P + 2][HS_ROWS_COLS];
+};
+// a wave's rows in it: first and last of buffer 0, of buffer 1, the others
+template <int P>
+constexpr unsigned hs_strip_row(int buf, int j) {
+    return 512u * (unsigned)(j == 0 ? 2 * buf : j == P - 1 ? 2 * buf + 1 : 3 + j);
+}
+typedef float hs_f2 __attribute__((ext_vector_type(2)));
+using hs_lds_f2 = __attribute__((address_space(3))) hs_f2;
+// the same for kernels that index it themselves
 template <int NW, int P>
 struct HsRowsLds {
     float2 edge[2][NW][2][HS_ROWS_COLS];
@@ -121,15 +133,15 @@ struct HsSetup {
 constexpr int HS_CUBE_OX[2][4] = {{0, 1, 0, 1}, {0, 0, 1, 1}};
 constexpr int HS_CUBE_OY[2][4] = {{0, 0, 1, 1}, {0, 1, 0, 1}};
 
-// 16 of a cell's 28 VALU instructions take a weight, and run at up to twice the rate
+// 16 of a cell's 29 VALU instructions take a weight, and run at up to twice the rate
 // when it is in a vector register (in_vgpr).  A build holds as many of the eight
-// there as its register budget leaves; the tall and the two-per-CU ones, which
-// have room for 2 to 6, also come as TWO builds for stencils whose first four and last
+// there as its register budget leaves; two of the two-per-CU ones, which
+// have room for 2, also come as TWO builds for stencils whose first four and last
 // four weights are equal (Horn and Schunck's own), which need two registers.
 // Per 8 iterations, scalar weights / as many as fit / TWO: 1920x1080 (16 x 4 rows) 32.3 /
 // 29.7 / 27.8 us, 2560x1440 (8 x 9) 50.4 / 47.2 / 45.2.
 template <int NW, int P, bool PRE>
-constexpr int kRowsVgprWeights = NW == 16 && !PRE ? 2 : P == 10 ? 2 : P == 9 ? 6 : 8;
+constexpr int kRowsVgprWeights = (NW == 16 && !PRE) || P == 9 ? 2 : 8;
 template <int NW, int P, bool PRE>
 constexpr bool kRowsTwoBuild = kRowsVgprWeights<NW, P, PRE> < 8;
 inline bool hs_two_weights(const float *w) {
@@ -159,7 +171,8 @@ struct HsTri {
 template <int NW, int P, bool PRE, int G, bool TWO, bool LOUT = false, bool SETUP = false>
 __device__ __forceinline__ void hs_rows_tile(const HsImage &a, int txi, int tyi, int tw, int th,
                                              int k, const float (&weights)[8],
-                                             HsRowsLds<NW, P> &lds, const HsSetup *su = nullptr) {
+                                             HsStripLds<NW, P> &lds,
+                                             const HsSetup *su = nullptr) {
     static_assert(P >= 2, "a strip has a first and a last row");
     constexpr int WV = kRowsVgprWeights<NW, P, PRE>;
     float w[8];
@@ -263,10 +276,30 @@ __device__ __forceinline__ void hs_rows_tile(const HsImage &a, int txi, int tyi,
     const int jb = H - 1 - gy0 - r0;  // the image's last row, as a strip row
     const bool in = gx >= x0 && gx < x1;
 
-    auto slot = [&](int buf, int j) -> float2 * {
-        if (j == 0) return lds.edge[buf][wave][0];
-        if (j == P - 1) return lds.edge[buf][wave][1];
-        return lds.row[wave][j - 1];
+    // LDS byte addresses of a row's left neighbour, cell and right neighbour in the slot of
+    // the wave above: every access is one of the three plus a constant
+    constexpr unsigned SLOT = 512u * (P + 2);
+    const unsigned base = (unsigned)(uintptr_t)(__attribute__((address_space(3))) char *)
+                              reinterpret_cast<char *>(&lds) + (unsigned)wave * SLOT;
+    unsigned al = base + 8u * (unsigned)li, ac = base + 8u * (unsigned)lane,
+             ar = base + 8u * (unsigned)ri;
+    asm volatile("" : "+v"(al), "+v"(ac), "+v"(ar));
+    auto get = [](unsigned addr) {
+        const hs_f2 x = *(const hs_lds_f2 *)(uintptr_t)addr;
+        return make_float2(x.x, x.y);
+    };
+    auto put = [&](unsigned row, float x, float y) {
+        const hs_f2 z = {x, y};
+        *(hs_lds_f2 *)(uintptr_t)(ac + row) = z;
+    };
+    // the row above the window or the image is the strip's own first row, the one below
+    // its last: the wave keeps a copy in the neighbouring slot (a strip that ends with
+    // the image's last row has none but such rows below it)
+    const bool dup_up = wave == 0, dup_down = jb == P - 1 || wave == NW - 1;
+    auto put_row = [&](int buf, int j, float x, float y) {
+        put(SLOT + hs_strip_row<P>(buf, j), x, y);
+        if (j == 0 && dup_up) put(hs_strip_row<P>(buf, P - 1), x, y);
+        if (j == P - 1 && dup_down) put(2 * SLOT + hs_strip_row<P>(buf, 0), x, y);
     };
     // a wave's LDS writes before its reads of the same row (a wavefront's LDS
     // accesses are performed in order; this keeps the compiler's order)
@@ -277,13 +310,16 @@ __device__ __forceinline__ void hs_rows_tile(const HsImage &a, int txi, int tyi,
     };
     float2 L[PRE ? P : 1], R[PRE ? P : 1];
 #pragma unroll
-    for (int j = 0; j < P; ++j) slot(0, j)[lane] = make_float2(u[j], v[j]);
+    for (int j = 0; j < P; ++j) put_row(0, j, u[j], v[j]);
+    // (a strip that never is active writes no other edge rows)
+    put_row(1, 0, u[0], v[0]);
+    put_row(1, P - 1, u[P - 1], v[P - 1]);
     wave_fence();
     if (PRE) {
 #pragma unroll
         for (int j = 0; j < P; ++j) {
-            L[j] = slot(0, j)[li];
-            R[j] = slot(0, j)[ri];
+            L[j] = get(al + SLOT + hs_strip_row<P>(0, j));
+            R[j] = get(ar + SLOT + hs_strip_row<P>(0, j));
         }
     }
     // linearisation output: the strip's offset from the plane's start, and the
@@ -294,37 +330,38 @@ __device__ __forceinline__ void hs_rows_tile(const HsImage &a, int txi, int tyi,
     if (LOUT)
         for (int j = 0; j < P; ++j)
             if (gy0 + r0 + j >= y0 && gy0 + r0 + j < y1) tile_rows |= 1u << j;
+    // Steps in which the strip has active rows (the tile grown by k - it, inside the
+    // image): the first `live` ones.  All its rows are updated in them; the inactive
+    // ones hold values that no active row reads.  A branch per row costs copies of its old
+    // and new values and its scalar tests, 5 VALU and 5 SALU instructions per row
+    // with P = 4, against 1.5 rows more per strip at the window's ends.
+    const int live = gy0 + r0 >= H ? 0
+                                   : clampi(min(k - 1 + r0 + P - (y0 - gy0), k - 1 + y1 - gy0 - r0),
+                                            0, k);
     // BOT: the image's last row is in the strip and not its last row
     auto steps = [&](auto bot_c) {
         constexpr bool BOT = decltype(bot_c)::value;
-        for (int it = 1; it <= k; ++it) {
-            // step it reads edge buffer (it - 1) & 1 and writes the other, which
-            // was last read in step it - 1, before this barrier.  (A row that is
-            // not active in a step is not written, and never read as valid later.)
+        // buf_c: the edge buffer step it reads, (it - 1) & 1; it writes the other, which
+        // was last read in step it - 1, before this barrier
+        auto step = [&](auto buf_c, int it) {
+            constexpr int buf = decltype(buf_c)::value;
             __syncthreads();
-            const int buf = (it - 1) & 1;
-            // active strip rows [lo, hi): the tile grown by k - it, inside the image
-            const int lo = max(y0 - (k - it), 0) - gy0 - r0;
-            const int hi = min(y1 + (k - it), H) - gy0 - r0;
             // (opaque per step: otherwise every row's output address is kept
             // across the loop)
             if (LOUT) asm volatile("" : "+v"(lo0));
             const float *const lub = LOUT ? a.lub + (int64_t)(it - 1) * a.lstride : nullptr;
             const float *const lvb = LOUT ? a.lvb + (int64_t)(it - 1) * a.lstride : nullptr;
-            if (lo >= P || hi <= 0) continue;
-            const float2 *const ra =
-                (gy0 + r0 == 0 || wave == 0) ? lds.edge[buf][wave][0] : lds.edge[buf][wave - 1][1];
-            const float2 *const rb = (jb == P - 1 || wave == NW - 1) ? lds.edge[buf][wave][1]
-                                                                     : lds.edge[buf][wave + 1][0];
             auto row = [&](int j) {
                 HsTri q;
                 q.c = make_float2(u[j], v[j]);
-                q.l = PRE ? L[PRE ? j : 0] : slot(buf, j)[li];
-                q.r = PRE ? R[PRE ? j : 0] : slot(buf, j)[ri];
+                q.l = PRE ? L[PRE ? j : 0] : get(al + SLOT + hs_strip_row<P>(buf, j));
+                q.r = PRE ? R[PRE ? j : 0] : get(ar + SLOT + hs_strip_row<P>(buf, j));
                 return q;
             };
             // the old rows above the group (prev) and its first (cur)
-            HsTri prev = {ra[li], ra[lane], ra[ri]};
+            constexpr unsigned above = hs_strip_row<P>(buf, P - 1);
+            constexpr unsigned below = 2 * SLOT + hs_strip_row<P>(buf, 0);
+            HsTri prev = {get(al + above), get(ac + above), get(ar + above)};
             HsTri cur = row(0);
 #pragma unroll
             for (int j0 = 0; j0 < P; j0 += G) {
@@ -336,8 +373,8 @@ __device__ __forceinline__ void hs_rows_tile(const HsImage &a, int txi, int tyi,
                 if (j0 + n < P)
                     rows[n] = row(j0 + n < P ? j0 + n : 0);
                 else
-                    rows[n] = {rb[li], rb[lane], rb[ri]};
-                if (j0 + n > lo && j0 < hi) {
+                    rows[n] = {get(al + below), get(ac + below), get(ar + below)};
+                {
                     float ub[G], vb[G], s2[G], q[G];
 #pragma unroll
                     for (int i = 0; i < n; ++i) {
@@ -389,7 +426,7 @@ __device__ __forceinline__ void hs_rows_tile(const HsImage &a, int txi, int tyi,
                         const float p2 = cy[j] * q[i];
                         u[j] = ub[i] - p1;
                         v[j] = vb[i] - p2;
-                        slot(buf ^ 1, j)[lane] = make_float2(u[j], v[j]);
+                        put_row(buf ^ 1, j, u[j], v[j]);
                     }
                     if (LOUT && in) {
                         const char *const pub = reinterpret_cast<const char *>(lub);
@@ -406,15 +443,24 @@ __device__ __forceinline__ void hs_rows_tile(const HsImage &a, int txi, int tyi,
                     if (PRE) {
 #pragma unroll
                         for (int i = 0; i < n; ++i) {
-                            L[PRE ? j0 + i : 0] = slot(buf ^ 1, j0 + i)[li];
-                            R[PRE ? j0 + i : 0] = slot(buf ^ 1, j0 + i)[ri];
+                            L[PRE ? j0 + i : 0] = get(al + SLOT + hs_strip_row<P>(buf ^ 1, j0 + i));
+                            R[PRE ? j0 + i : 0] = get(ar + SLOT + hs_strip_row<P>(buf ^ 1, j0 + i));
                         }
                     }
                 }
                 prev = rows[n - 1];
                 cur = rows[n];
             }
+        };
+        // two steps a round, so that a row's old and new values change places
+        // without copies and the buffers' addresses are constants
+        int it = 1;
+        while (it <= live) {
+            step(std::integral_constant<int, 0>(), it++);
+            if (it > live) break;
+            step(std::integral_constant<int, 1>(), it++);
         }
+        for (; it <= k; ++it) __syncthreads();
     };
     if (jb >= 0 && jb < P - 1)
         steps(std::true_type());

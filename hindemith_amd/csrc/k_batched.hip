@@ -395,7 +395,7 @@ struct MultiRowsArgs {
 
 template <int NW, int P, bool PRE, int G, bool TWO, bool FIRST>
 __device__ __forceinline__ void multi_rows_body(const MultiRowsArgs &b, int ph, int kk) {
-    __shared__ HsRowsLds<NW, P> lds;
+    __shared__ HsStripLds<NW, P> lds;
     // phases alternate the walk over each XCD's share of the list
     const int w = xcd_remap(blockIdx.x, b.total_tiles, (ph & 1) == 0);
     const PairDesc &D = b.tiles[w];
@@ -483,14 +483,13 @@ static const BVariant kBVariants[] = {
     HB_S(1024, 64, 32, 4, true, true),   // 9: stepped, as variant 25
     HB_S(1024, 64, 32, 8, true, false),  // 10: stepped, as variant 17
     HB_S(512, 64, 32, 4, true, true),    // 11: stepped, as variant 26
-    // 12-18: stepped, row-register tiles (tile at k = 8), as the single-image
+    // 12-17: stepped, row-register tiles (tile at k = 8), as the single-image
     // variants 29, 30, 32, 33, 34, 35 and 36
     HB_R(16, 2, true, 2, 4, 1, 12, kRowsCost16x2),
     HB_R(16, 3, true, 3, 4, 1, 16, kRowsCost16x3),
     HB_R(16, 5, true, 5, 4, 1, 16, kRowsCost16x5),
     HB_R(8, 7, false, 4, 4, 2, 16, kRowsCost8x7),
     HB_R(8, 9, false, 3, 4, 2, 16, kRowsCost8x9),
-    HB_R(8, 10, false, 2, 4, 2, 16, kRowsCost8x10),
     HB_R(16, 4, false, 1, 8, 2, 16, kRowsCost16x4two),
 };
 #undef HB_V

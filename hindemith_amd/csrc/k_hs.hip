@@ -131,7 +131,7 @@ __global__ __launch_bounds__(NT) void hs_strip_kernel(HsArgs a, Taps taps) {
 // 8-tap averaging offsets.  WPE: waves per SIMD the build is held to.
 template <int NW, int P, bool PRE, int G, bool TWO, bool LOUT, bool SETUP>
 __device__ __forceinline__ void hs_rows_body(const HsArgs &a, const Taps &taps, const HsSetup *su) {
-    __shared__ HsRowsLds<NW, P> lds;
+    __shared__ HsStripLds<NW, P> lds;
     const int64_t off = (int64_t)blockIdx.y * a.bstride;
     HsImage im;
     im.Ix = a.Ix + off;
@@ -405,12 +405,12 @@ static const HsVariant kVariants[] = {
       hs_tb_kernel<1024, 64, 32, 8, 9, false, true, true>,
       hs_tb_kernel<1024, 64, 32, 8, 0, false, true, true>},
      nullptr, true},
-    // 29-36: row-register forms, chosen by hs_rows_choice.  One work-group of 16
+    // 29-35: row-register forms, chosen by hs_rows_choice.  One work-group of 16
     // waves per CU, for images that give a CU at most one tile: the window's
-    // height sets how many pixels a CU takes (neighbours prefetched; 64 to 118
+    // height sets how many pixels a CU takes (neighbours prefetched; 64 to 119
     // VGPRs).  Two work-groups per CU for larger images, so that one's loads
     // and barriers overlap the other's steps: 8 waves at up to 128 VGPRs, or 16 at
-    // 63 (one row at a time).  The linearisation builds of the last two would spill.
+    // 62 (one row at a time; its linearisation build would spill).
     HS_R(16, 2, true, 2, 4, 1, 12, kRowsCost16x2,
          HS_RL(16, 2, true, 2, 4)),   // 29: window 64 x 32
     HS_R(16, 3, true, 3, 4, 1, 16, kRowsCost16x3,
@@ -423,10 +423,8 @@ static const HsVariant kVariants[] = {
          HS_RL(8, 7, false, 4, 4)),   // 33: 64 x 56
     HS_R(8, 9, false, 3, 4, 2, 16, kRowsCost8x9,
          HS_RL(8, 9, false, 3, 4)),   // 34: 64 x 72
-    HS_R(8, 10, false, 2, 4, 2, 16, kRowsCost8x10,
-         nullptr, nullptr),  // 35: 64 x 80
     HS_R(16, 4, false, 1, 8, 2, 16, kRowsCost16x4two,
-         nullptr, nullptr),  // 36: 64 x 64
+         nullptr, nullptr),  // 35: 64 x 64
 };
 #undef HS_R
 #undef HS_RL
@@ -495,6 +493,10 @@ static void hs_rows_choice(int H, int W, int B, int iters, bool in_place, bool l
         const int k_lo = std::min(iters, 5), k_hi = std::min(iters, V.kmax);
         for (int n = (iters + k_hi - 1) / k_hi; n <= (iters + k_lo - 1) / k_lo; ++n) {
             const int kk = (iters + n - 1) / n;
+            // two work-groups per CU pay only where some CU takes two
+            if (V.wgs > 1 &&
+                (int64_t)hs_rows_geom(V.nw * V.rows, V.wgs, H, W, kk, B).ntiles * B <= kCus)
+                continue;
             const float us = (float)n * rows_launch_us(V, H, W, kk, B) + (n & 1 ? copy_us : 0.0f);
             if (us < best) {
                 best = us;
