@@ -493,12 +493,11 @@ static void hs_rows_choice(int H, int W, int B, int iters, bool in_place, bool l
         const int k_lo = std::min(iters, 5), k_hi = std::min(iters, V.kmax);
         for (int n = (iters + k_hi - 1) / k_hi; n <= (iters + k_lo - 1) / k_lo; ++n) {
             const int kk = (iters + n - 1) / n;
-            // two work-groups per CU pay only where some CU takes two
-            if (V.wgs > 1 &&
-                (int64_t)hs_rows_geom(V.nw * V.rows, V.wgs, H, W, kk, B).ntiles * B <= kCus)
-                continue;
             const float us = (float)n * rows_launch_us(V, H, W, kk, B) + (n & 1 ? copy_us : 0.0f);
-            if (us < best) {
+            // (two work-groups per CU pay only where some CU takes two)
+            if (us < best &&
+                (V.wgs == 1 ||
+                 (int64_t)hs_rows_geom(V.nw * V.rows, V.wgs, H, W, kk, B).ntiles * B > kCus)) {
                 best = us;
                 variant = vi;
                 k = kk;

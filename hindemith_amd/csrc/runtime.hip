@@ -298,8 +298,8 @@ struct ScalarStmt {
 };
 
 // A result's host copy.  Pinned, and kept while the record lives: a fresh pageable one per
-// run costs a page fault and a clearing pass per page besides a staged copy
-// (1080p, two planes of flow: see hmx_run).
+// run costs a page fault and a clearing pass per page besides a staged copy (the
+// canonical program at 1920x1080, two planes: 5.24 ms a call, 4.59 with these).
 struct HostResult {
     char *p = nullptr;
     int64_t cap = 0, bytes = 0;
