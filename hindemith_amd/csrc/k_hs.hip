@@ -515,7 +515,10 @@ static void default_choice(int H, int W, int B, int iters, bool in_place, bool c
                            int &variant, int &k) {
     variant = 24;
     k = 8;
-    if (canonical) hs_rows_choice(H, W, B, std::max(iters, 1), in_place, false, variant, k);
+    // (an empty image has no tiles to weigh: the call that asks is refused or fails at
+    // its launch, whatever the choice)
+    if (canonical && H > 0 && W > 0)
+        hs_rows_choice(H, W, B, std::max(iters, 1), in_place, false, variant, k);
 }
 
 int launch_hs_tb(int variant, const float *Ix, const float *Iy, const float *It,
@@ -946,9 +949,11 @@ extern "C" int hmx_hs_jacobi(const float *Ix, const float *Iy, const float *It,
                              const float *den, float alpha2, int H, int W, int nda,
                              const float *wa, const int *oxa, const int *oya, int iters,
                              float *u, float *v, float *work_u, float *work_v, void *stream) {
+    int rc = validate_jacobi(Ix, Iy, It, H, W, u, v, work_u, work_v);
+    if (rc) return rc;
     int variant, k;
     Taps t;
-    int rc = make_taps(t, nda, wa, oxa, oya);
+    rc = make_taps(t, nda, wa, oxa, oya);
     if (rc) return rc;
     hs_choice(H, W, 1, iters, true, t, variant, k);
     return hmx_hs_jacobi_cfg(Ix, Iy, It, den, alpha2, H, W, nda, wa, oxa, oya, iters, u, v,
