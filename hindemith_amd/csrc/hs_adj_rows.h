@@ -99,13 +99,16 @@ __global__ __launch_bounds__(64 * NW, WPE) void hs_adj_rows_kernel(AdjRowsArgs a
     const bool in = gx >= x0 && gx < x1;
     auto tile_row = [&](int j) { return gy0 + r0 + j >= y0 && gy0 + r0 + j < y1; };
 
-    // byte offsets from the image start fit 32 bits (H, W < 32768); cells outside
-    // the image load the pixel they clamp to
+    // byte offsets from the strip's first image row (uniform over the wave, 64 bits) fit
+    // 32 bits; cells outside the image load the pixel they clamp to
+    const int rs = min(gy0 + r0, H - 1);
+    const int64_t strip = off + (int64_t)rs * W;
     const unsigned rowb = (unsigned)W * 4u;
     const unsigned co = (unsigned)clampi(gx, 0, W - 1) * 4u;
-    auto at = [&](int j) { return (unsigned)min(gy0 + r0 + j, H - 1) * rowb + co; };
+    auto at = [&](int j) { return (unsigned)(min(gy0 + r0 + j, H - 1) - rs) * rowb + co; };
     auto ld = [&](const float *plane, unsigned o) {
-        return ld_g(reinterpret_cast<const float *>(reinterpret_cast<const char *>(plane + off) + o));
+        return ld_g(reinterpret_cast<const float *>(
+            reinterpret_cast<const char *>(plane + strip) + o));
     };
     float cx[P], cy[P], ct[P], cd[P], cr[P], u[P], v[P];
 #pragma unroll
@@ -443,7 +446,7 @@ __global__ __launch_bounds__(64 * NW, WPE) void hs_adj_rows_kernel(AdjRowsArgs a
             if (!tile_row(j)) continue;
             const unsigned o = at(j);
             auto st = [&](float *plane, float x) {
-                *(gfloat *)(reinterpret_cast<char *>(plane + off) + o) = x;
+                *(gfloat *)(reinterpret_cast<char *>(plane + strip) + o) = x;
             };
             st(a.gu_out, g[j].x);
             st(a.gv_out, g[j].y);

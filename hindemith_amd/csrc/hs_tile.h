@@ -226,23 +226,23 @@ __device__ __forceinline__ void hs_tile(const HsImage &a, int t, int k,
     // Ghosts and cells outside the region hold -1.
     float cx[P], cy[P], ct[P], cd[P], cr[FDIV ? P : 1];
     int pk[P];
+    // The region's first image pixel: byte offsets from it fit 32 bits, so each load is
+    // a uniform base plus one per-cell offset register, for planes of any size.
+    const int left = max(gx0, 0), top = max(gy0, 0);
+    const int64_t first = ((int64_t)top * a.W + left) * (int64_t)sizeof(float);
+    const char *const pIx = reinterpret_cast<const char *>(a.Ix) + first;
+    const char *const pIy = reinterpret_cast<const char *>(a.Iy) + first;
+    const char *const pIt = reinterpret_cast<const char *>(a.It) + first;
+    const char *const pu = reinterpret_cast<const char *>(a.u_in) + first;
+    const char *const pv = reinterpret_cast<const char *>(a.v_in) + first;
+    const char *const pd = a.den ? reinterpret_cast<const char *>(a.den) + first : nullptr;
+    const unsigned rowb = (unsigned)a.W * (unsigned)sizeof(float);
     if (!clipped) {
         // Unclipped tile (most of them): the region is the window's top-left
         // (TW + 2k) x (TH + 2k) cells and every one of them is an image pixel,
         // so a cell's offset, last step and border flags (none) follow from
         // its window position alone.  All of a thread's loads are issued
         // before any of them is used.
-        // Byte offsets from the region's corner fit 32 bits (H, W < 32768),
-        // so each load is a uniform base plus one per-cell offset register.
-        const int64_t corner = ((int64_t)gy0 * a.W + gx0) * (int64_t)sizeof(float);
-        const char *const pIx = reinterpret_cast<const char *>(a.Ix) + corner;
-        const char *const pIy = reinterpret_cast<const char *>(a.Iy) + corner;
-        const char *const pIt = reinterpret_cast<const char *>(a.It) + corner;
-        const char *const pu = reinterpret_cast<const char *>(a.u_in) + corner;
-        const char *const pv = reinterpret_cast<const char *>(a.v_in) + corner;
-        const char *const pd =
-            a.den ? reinterpret_cast<const char *>(a.den) + corner : nullptr;
-        const unsigned rowb = (unsigned)a.W * (unsigned)sizeof(float);
         float ui[P], vi[P];
         bool in[P];
         int rxs[P], rys[P];
@@ -292,15 +292,7 @@ __device__ __forceinline__ void hs_tile(const HsImage &a, int t, int k,
     } else {
         // Clipped tile: region cells outside the image are ghosts and load the
         // pixel their coordinates clamp to; image cells also load their
-        // coefficients.  Byte offsets from the image start fit 32 bits
-        // (H, W < 32768).  As above, every load is issued before any use.
-        const char *const bIx = reinterpret_cast<const char *>(a.Ix);
-        const char *const bIy = reinterpret_cast<const char *>(a.Iy);
-        const char *const bIt = reinterpret_cast<const char *>(a.It);
-        const char *const bu = reinterpret_cast<const char *>(a.u_in);
-        const char *const bv = reinterpret_cast<const char *>(a.v_in);
-        const char *const bd = reinterpret_cast<const char *>(a.den);
-        const unsigned rowb = (unsigned)a.W * (unsigned)sizeof(float);
+        // coefficients.  As above, every load is issued before any use.
         float ui[P], vi[P];
         bool in[P], img[P];
         int gxs[P], gys[P], rxs[P], rys[P];
@@ -315,17 +307,18 @@ __device__ __forceinline__ void hs_tile(const HsImage &a, int t, int k,
             gys[j] = gy;
             in[j] = ((j + 1) * NT <= NPX || c < NPX) && rx < RW && ry < RH;
             img[j] = in[j] && gx >= 0 && gx < a.W && gy >= 0 && gy < a.H;
-            const unsigned o = (unsigned)clampi(gy, 0, a.H - 1) * rowb +
-                               (unsigned)clampi(gx, 0, a.W - 1) * (unsigned)sizeof(float);
+            const unsigned o =
+                (unsigned)(clampi(gy, top, a.H - 1) - top) * rowb +
+                (unsigned)(clampi(gx, left, a.W - 1) - left) * (unsigned)sizeof(float);
             if (in[j]) {
-                ui[j] = hs_ld_uv<COH>(bu + o);
-                vi[j] = hs_ld_uv<COH>(bv + o);
+                ui[j] = hs_ld_uv<COH>(pu + o);
+                vi[j] = hs_ld_uv<COH>(pv + o);
             }
             if (img[j]) {
-                cx[j] = ld_g(reinterpret_cast<const float *>(bIx + o));
-                cy[j] = ld_g(reinterpret_cast<const float *>(bIy + o));
-                ct[j] = ld_g(reinterpret_cast<const float *>(bIt + o));
-                if (bd) cd[j] = ld_g(reinterpret_cast<const float *>(bd + o));
+                cx[j] = ld_g(reinterpret_cast<const float *>(pIx + o));
+                cy[j] = ld_g(reinterpret_cast<const float *>(pIy + o));
+                ct[j] = ld_g(reinterpret_cast<const float *>(pIt + o));
+                if (pd) cd[j] = ld_g(reinterpret_cast<const float *>(pd + o));
             }
         }
 #pragma unroll
@@ -343,7 +336,7 @@ __device__ __forceinline__ void hs_tile(const HsImage &a, int t, int k,
                 const int g = (e & 1) ? -1 : (e & 2) ? 1 : (e & 4) ? -PITCH : (e & 8) ? PITCH : 0;
                 pk[j] = ((k - max(dx, dy)) << 27) | (e << 12) |
                         (LOUT ? (rys[j] << 16) | rxs[j] : SHARED && !COH ? (g & 0x1ff) : 0);
-                if (!bd) {
+                if (!pd) {
                     const float m1 = cx[j] * cx[j];
                     const float s1 = a.alpha2 + m1;
                     const float m2 = cy[j] * cy[j];
@@ -525,7 +518,7 @@ __device__ __forceinline__ void hs_tile(const HsImage &a, int t, int k,
     // Store the output tile from the final window (complete: every step ends
     // with a barrier) in tile order: thread tid stores tile cells tid + j*NT,
     // so a wavefront writes whole row segments, at byte offsets from the
-    // tile's corner (32 bits: H, W < 32768).
+    // tile's corner (which fit 32 bits).
     {
         const float2 *const fin = (DB ? uv + (k & 1) * NPX : uv) + k * PITCH + k;
         const int64_t corner = ((int64_t)y0 * a.W + x0) * (int64_t)sizeof(float);
@@ -605,15 +598,17 @@ __device__ __forceinline__ void hs_tile_ring(const HsImage &a, int t, int k,
     const int RW = x1 - x0 + 2 * k, RH = y1 - y0 + 2 * k;
     const bool clipped = (gx0 < 0) || (gy0 < 0) || (x1 + k > a.W) || (y1 + k > a.H);
 
-    // Byte offsets from the image start fit 32 bits (H, W < 32768): every
-    // load below is a uniform base plus one offset register.
+    // Byte offsets from the region's first image row fit 32 bits: every load below is a
+    // uniform base plus one offset register.
+    const int row0 = max(gy0, 0);
+    const int64_t corner = (int64_t)row0 * a.W;
     const unsigned rowb = (unsigned)a.W * (unsigned)sizeof(float);
-    const char *const bIx = reinterpret_cast<const char *>(a.Ix);
-    const char *const bIy = reinterpret_cast<const char *>(a.Iy);
-    const char *const bIt = reinterpret_cast<const char *>(a.It);
-    const char *const bd = reinterpret_cast<const char *>(a.den);
-    const char *const bu = reinterpret_cast<const char *>(a.u_in);
-    const char *const bv = reinterpret_cast<const char *>(a.v_in);
+    const char *const bIx = reinterpret_cast<const char *>(a.Ix + corner);
+    const char *const bIy = reinterpret_cast<const char *>(a.Iy + corner);
+    const char *const bIt = reinterpret_cast<const char *>(a.It + corner);
+    const char *const bd = a.den ? reinterpret_cast<const char *>(a.den + corner) : nullptr;
+    const char *const bu = reinterpret_cast<const char *>(a.u_in + corner);
+    const char *const bv = reinterpret_cast<const char *>(a.v_in + corner);
 
     // (u, v) of every region cell into window 0, row-major (coalesced); cells
     // outside the image load the pixel they clamp to (ghosts, see hs_tile)
@@ -622,7 +617,7 @@ __device__ __forceinline__ void hs_tile_ring(const HsImage &a, int t, int k,
         const int c = tid + j * NT;
         const int ry = c / PITCH, rx = c - ry * PITCH;
         if (((j + 1) * NT <= NPX || c < NPX) && rx < RW && ry < RH) {
-            const unsigned o = (unsigned)clampi(gy0 + ry, 0, a.H - 1) * rowb +
+            const unsigned o = (unsigned)(clampi(gy0 + ry, row0, a.H - 1) - row0) * rowb +
                                (unsigned)clampi(gx0 + rx, 0, a.W - 1) * (unsigned)sizeof(float);
             uv[c] = make_float2(ld_g(reinterpret_cast<const float *>(bu + o)),
                                 ld_g(reinterpret_cast<const float *>(bv + o)));
@@ -665,7 +660,8 @@ __device__ __forceinline__ void hs_tile_ring(const HsImage &a, int t, int k,
                                    : (gx == 0) | (gx == a.W - 1) << 1 | (gy == 0) << 2 |
                                          (gy == a.H - 1) << 3;
             pk[j] = (L << 27) | (e << 12);
-            const unsigned o = (unsigned)gy * rowb + (unsigned)gx * (unsigned)sizeof(float);
+            const unsigned o =
+                (unsigned)(gy - row0) * rowb + (unsigned)gx * (unsigned)sizeof(float);
             cx[j] = ld_g(reinterpret_cast<const float *>(bIx + o));
             cy[j] = ld_g(reinterpret_cast<const float *>(bIy + o));
             ct[j] = ld_g(reinterpret_cast<const float *>(bIt + o));

@@ -178,8 +178,8 @@ __global__ __launch_bounds__(NT, 8) void hs_adj_tb_kernel(AdjTbArgs a, Taps taps
     // the window's corner is pixel (x0 - MMAX, y0 - MMAX) for every tile
     const int wx0 = x0 - MMAX, wy0 = y0 - MMAX;
     // pixels are addressed from the tile's corner pixel by byte offsets that
-    // fit 32 bits (H, W < 32768): unsigned for the tile's own pixels (the
-    // load's uniform base plus one offset register), signed for the ring
+    // fit 32 bits: unsigned for the tile's own pixels (the load's uniform base
+    // plus one offset register), signed for the ring
     const int64_t corner = off + (int64_t)y0 * W + x0;
     const bool wt = rows_whole_lines(W);
     // tile slot j's pixel is NT / TW rows below slot 0's: one offset register
