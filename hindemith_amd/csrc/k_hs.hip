@@ -27,6 +27,7 @@
 #include <cstdlib>
 #include <map>
 #include <mutex>
+#include <tuple>
 #include <utility>
 #include <vector>
 
@@ -438,7 +439,12 @@ static constexpr int kNumVariants = sizeof(kVariants) / sizeof(kVariants[0]);
 constexpr int kLongSolve = 500;
 
 static std::mutex g_tune_mu;
-static std::map<std::pair<int, int>, std::pair<int, int>> g_tuned;  // (H,W) -> (variant,k)
+// (H, W, canonical averaging stencil) -> (variant, k)
+static std::map<std::tuple<int, int, bool>, std::pair<int, int>> g_tuned;
+// The tuner times solves of one image, this many iterations long or more.  With the
+// canonical stencil, batches and shorter solves (the adjoint's segments) are not what it
+// measured, and take the rule, which weighs both; other stencils have no such rule.
+constexpr int kTunedFrom = 96;
 
 // Whether a launch of variant V with these taps runs its row-register kernel.
 static bool hs_runs_rows(const HsVariant &V, const Taps &taps) {
@@ -834,17 +840,20 @@ int hs_jacobi_run(const float *Ix, const float *Iy, const float *It, const float
 }
 
 // (variant, k) for iters iterations of B images of one size: the tuned choice, if
-// hs_tune ran for the size, else the default.
+// hs_tune ran for the size and the kind of stencil (see kTunedFrom), else the default.
 void hs_choice(int H, int W, int B, int iters, bool in_place, const Taps &taps, int &variant,
                int &k) {
-    std::lock_guard<std::mutex> lk(g_tune_mu);
-    auto it = g_tuned.find({H, W});
-    if (it != g_tuned.end()) {
-        variant = it->second.first;
-        k = it->second.second;
-    } else {
-        default_choice(H, W, B, iters, in_place, hs_ring_taps(taps), variant, k);
+    const bool canonical = hs_ring_taps(taps);
+    if (!canonical || (B == 1 && iters >= kTunedFrom)) {
+        std::lock_guard<std::mutex> lk(g_tune_mu);
+        auto it = g_tuned.find({H, W, canonical});
+        if (it != g_tuned.end()) {
+            variant = it->second.first;
+            k = it->second.second;
+            return;
+        }
     }
+    default_choice(H, W, B, iters, in_place, canonical, variant, k);
 }
 
 static int validate_jacobi(const float *Ix, const float *Iy, const float *It, int H, int W,
@@ -974,9 +983,12 @@ extern "C" int hmx_hs_tune(const float *Ix, const float *Iy, const float *It, fl
     hipEvent_t e0, e1;
     HMX_HIP_TRY(hipEventCreate(&e0));
     HMX_HIP_TRY(hipEventCreate(&e1));
-    // min over reps of one timed run of iters iterations (after one warm-up run)
-    auto time_cfg = [&](int vi, int k, int iters, int reps, float &best_ms) -> int {
+    // min over reps of one timed run (after one warm-up run), in ms for iters iterations.
+    // A run is an even number of launches of k: an odd one copies the start state, and
+    // a shorter last one is not what a long solve consists of.
+    auto time_cfg = [&](int vi, int k, int iters0, int reps, float &best_ms) -> int {
         best_ms = 1e30f;
+        const int iters = (iters0 + 2 * k - 1) / (2 * k) * 2 * k;
         int r = hs_jacobi_run(Ix, Iy, It, nullptr, alpha2, H, W, t, iters, u, v, work_u, work_v,
                               vi, k, s);
         for (int i = 0; i < reps && !r; ++i) {
@@ -988,38 +1000,42 @@ extern "C" int hmx_hs_tune(const float *Ix, const float *Iy, const float *It, fl
             if (hipEventRecord(e1, s) != hipSuccess || hipEventSynchronize(e1) != hipSuccess ||
                 hipEventElapsedTime(&ms, e0, e1) != hipSuccess)
                 return fail(HMX_ERR_HIP, "tune: event timing");
-            best_ms = std::min(best_ms, ms);
+            best_ms = std::min(best_ms, ms * (float)iters0 / (float)iters);
         }
         return r;
     };
     // pass 1: every (variant, k) on a short run; pass 2: the four fastest on a
-    // run five times longer, so that near-equal candidates are told apart by
-    // more than launch noise (both iteration counts divide by every k tried)
+    // run three times longer, so that near-equal candidates are told apart by
+    // more than launch noise.  (Row-register variants stand for variant 24 with other
+    // stencils than the canonical one, which is a candidate itself.)
+    const bool canonical = hs_ring_taps(t);
     struct Cand {
         float ms;
         int v, k;
     };
     std::vector<Cand> cands;
-    for (int vi = 0; vi < kNumVariants && !rc; ++vi)
+    for (int vi = 0; vi < kNumVariants && !rc; ++vi) {
+        if (kVariants[vi].nw && !canonical) continue;
         for (int k = 1; k <= kVariants[vi].kmax && !rc; k *= 2) {
             float ms;
-            rc = time_cfg(vi, k, 48, 2, ms);
+            rc = time_cfg(vi, k, kTunedFrom, 2, ms);
             if (rc == HMX_ERR_TIMEOUT) {  // a persistent grid that gave up: not a candidate
                 rc = HMX_OK;
                 continue;
             }
             cands.push_back({ms, vi, k});
         }
+    }
     int best_v = 0, best_k = 1;
     if (!rc) {
         std::sort(cands.begin(), cands.end(),
                   [](const Cand &a, const Cand &b) { return a.ms < b.ms; });
         int dv, dk;
-        default_choice(H, W, 1, kLongSolve, true, hs_ring_taps(t), dv, dk);
+        default_choice(H, W, 1, kLongSolve, true, canonical, dv, dk);
         float best = 1e30f, dms = -1.0f;
         for (size_t i = 0; i < cands.size() && i < 4 && !rc; ++i) {
             float ms;
-            rc = time_cfg(cands[i].v, cands[i].k, 240, 3, ms);
+            rc = time_cfg(cands[i].v, cands[i].k, 3 * kTunedFrom, 3, ms);
             if (rc == HMX_ERR_TIMEOUT) {
                 rc = HMX_OK;
                 continue;
@@ -1034,7 +1050,7 @@ extern "C" int hmx_hs_tune(const float *Ix, const float *Iy, const float *It, fl
         // The default configuration stays unless a candidate beats it by more
         // than 2% on the long run: variants closer than that differ by less
         // than the spread between GPUs and runs, and should not flip.
-        if (!rc && dms < 0.0f) rc = time_cfg(dv, dk, 240, 3, dms);
+        if (!rc && dms < 0.0f) rc = time_cfg(dv, dk, 3 * kTunedFrom, 3, dms);
         if (!rc && dms <= 1.02f * best) {
             best_v = dv;
             best_k = dk;
@@ -1045,7 +1061,7 @@ extern "C" int hmx_hs_tune(const float *Ix, const float *Iy, const float *It, fl
     if (rc) return rc;
     {
         std::lock_guard<std::mutex> lk(g_tune_mu);
-        g_tuned[{H, W}] = {best_v, best_k};
+        g_tuned[{H, W, canonical}] = {best_v, best_k};
     }
     if (variant_out) *variant_out = best_v;
     if (k_out) *k_out = best_k;

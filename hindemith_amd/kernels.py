@@ -251,7 +251,8 @@ def hs_jacobi(Ix, Iy, It, alpha2, Avg, iters, u, v, work=None, den=None, variant
 
 
 def hs_tune(Ix, Iy, It, alpha2, Avg):
-    """Autotune (variant, k) for this image size; buffers are scratch copies."""
+    """Autotune (variant, k) for this image size and kind of averaging stencil (the
+    canonical one, or any other); buffers are scratch copies."""
     H, W = Ix.shape
     u = torch.zeros_like(Ix)
     v = torch.zeros_like(Ix)

@@ -257,11 +257,13 @@ int hmx_hs_variant_strip(int variant);
 int hmx_hs_recip_check(int e_lo, int e_hi, unsigned long long *bad, void *stream);
 /* The (variant, k) hmx_hs_jacobi and hmx_hs_solve use for an H x W image, the
  * canonical averaging stencil and a long solve: the tuned one if hmx_hs_tune ran
- * for that size in this process, else the default (which for other stencils and
+ * for that size and stencil in this process, else the default (which for other stencils and
  * for few iterations may be another).  No counterpart in the reference. */
 int hmx_hs_config(int H, int W, int *variant, int *k);
 /* Time every (variant, k) candidate on the given buffers (their contents are
- * overwritten) and cache the best for this H x W; returns the choice.  The
+ * overwritten) and cache the best for this H x W and kind of averaging stencil
+ * (the canonical one, or any other); returns the choice.  Canonical solves of one
+ * image of at least 96 iterations use it, and all solves with other stencils.  The
  * default configuration is kept unless a candidate is more than 2% faster. */
 int hmx_hs_tune(const float *Ix, const float *Iy, const float *It, float alpha2, int H, int W,
                 int nda, const float *wa, const int *oxa, const int *oya, float *u, float *v,
