@@ -484,7 +484,7 @@ static const BVariant kBVariants[] = {
     HB_S(1024, 64, 32, 8, true, false),  // 10: stepped, as variant 17
     HB_S(512, 64, 32, 4, true, true),    // 11: stepped, as variant 26
     // 12-17: stepped, row-register tiles (tile at k = 8), as the single-image
-    // variants 29, 30, 32, 33, 34, 35 and 36
+    // variants 29, 30, 32, 33, 34 and 35
     HB_R(16, 2, true, 2, 4, 1, 12, kRowsCost16x2),
     HB_R(16, 3, true, 3, 4, 1, 16, kRowsCost16x3),
     HB_R(16, 5, true, 5, 4, 1, 16, kRowsCost16x5),
@@ -517,6 +517,24 @@ static std::mutex g_bmu;
 static std::list<BatchPlan> g_plans;  // most recent first
 static constexpr size_t kMaxPlans = 8;
 static std::vector<std::pair<std::vector<int>, std::pair<int, int>>> g_btuned;
+// What batched_rows_choice picked for a list of sizes and an iteration count, most
+// recent first: a queue that is solved again does not search again (those 2000 pairs,
+// searched in each call 713 us a call, kept 179).
+struct BatchChoice {
+    std::vector<int> sizes;
+    int iters, variant, k;
+};
+static std::list<BatchChoice> g_bchoices;
+static constexpr size_t kMaxChoices = 32;
+
+static std::vector<int> pair_sizes(const hmx_pair *pairs, int npairs) {
+    std::vector<int> sig(2 * (size_t)npairs);
+    for (int i = 0; i < npairs; ++i) {
+        sig[2 * i] = pairs[i].H;
+        sig[2 * i + 1] = pairs[i].W;
+    }
+    return sig;
+}
 
 static void free_plan(BatchPlan &p) {
     if (p.exec) (void)hipGraphExecDestroy(p.exec);
@@ -553,22 +571,28 @@ static void pair_tiles(const BVariant &V, int k, int H, int W, int &tw, int &th,
 // The row-register variant and iterations per phase with the least cost for these
 // pairs, as hs_rows_choice for one image: the busiest CU's tiles times the mean
 // tile's rows.  At least two phases (a single one would read the planes it writes);
-// an odd phase count needs no copy (the third plane pair).
+// an odd phase count needs no copy (the third plane pair).  Of long lists every
+// step-th pair stands for its neighbours: the search takes 0.28 us of host time per pair
+// that it looks at (2000 pairs of 16 .. 48 pixels, 20 iterations: a first call 1275 us of
+// host time, 675 with kChoicePairs).
+constexpr int kChoicePairs = 128;
 static void batched_rows_choice(const hmx_pair *pairs, int npairs, int iters, int &variant,
                                 int &k) {
+    const int step = (npairs + kChoicePairs - 1) / kChoicePairs;
+    const int seen = (npairs + step - 1) / step;
     float best = 1e30f;
     for (int vi = 0; vi < kNumBVariants; ++vi) {
         const BVariant &V = kBVariants[vi];
         if (!V.nw) continue;
         for (int kk = std::min(5, (iters + 1) / 2); kk <= std::min(V.kmax, (iters + 1) / 2); ++kk) {
             int64_t tiles = 0, active = 0;
-            for (int i = 0; i < npairs; ++i) {
+            for (int i = 0; i < npairs; i += step) {
                 int tw, th, nx, ny;
                 pair_tiles(V, kk, pairs[i].H, pairs[i].W, tw, th, nx, ny);
                 tiles += (int64_t)nx * ny;
                 active += (int64_t)nx * ny * std::min(th + kk - 1, pairs[i].H);
             }
-            const int m = (int)((tiles + kCus - 1) / kCus);
+            const int m = (int)((tiles * npairs / seen + kCus - 1) / kCus);
             const int nph = (iters + kk - 1) / kk;
             const float us = (float)nph * V.cost.us(V.nw * V.rows, m, kk,
                                                (float)active / (float)tiles);
@@ -793,20 +817,32 @@ static int batched_impl(const hmx_pair *pairs, int npairs, const SetupTaps &st, 
     if (variant < 0) {  // autotuned choice for this size signature, else default
         variant = 8;  // stepped, double-buffered, reciprocal quotient
         k = 8;
-        std::vector<int> sig;
-        for (int i = 0; i < npairs; ++i) {
-            sig.push_back(pairs[i].H);
-            sig.push_back(pairs[i].W);
+        std::vector<int> sig = pair_sizes(pairs, npairs);
+        const bool rule = iters >= 2 && canonical;
+        bool known = false;
+        {
+            std::lock_guard<std::mutex> lk(g_bmu);
+            for (auto &e : g_btuned)
+                if (e.first == sig) {
+                    variant = e.second.first;
+                    k = e.second.second;
+                    known = true;
+                }
+            for (auto it = g_bchoices.begin(); rule && !known && it != g_bchoices.end(); ++it)
+                if (it->iters == iters && it->sizes == sig) {
+                    variant = it->variant;
+                    k = it->k;
+                    known = true;
+                    g_bchoices.splice(g_bchoices.begin(), g_bchoices, it);
+                    break;
+                }
         }
-        std::lock_guard<std::mutex> lk(g_bmu);
-        bool tuned = false;
-        for (auto &e : g_btuned)
-            if (e.first == sig) {
-                variant = e.second.first;
-                k = e.second.second;
-                tuned = true;
-            }
-        if (!tuned && iters >= 2 && canonical) batched_rows_choice(pairs, npairs, iters, variant, k);
+        if (!known && rule) {
+            batched_rows_choice(pairs, npairs, iters, variant, k);
+            std::lock_guard<std::mutex> lk(g_bmu);
+            g_bchoices.push_front({std::move(sig), iters, variant, k});
+            if (g_bchoices.size() > kMaxChoices) g_bchoices.pop_back();
+        }
     }
     HMX_REQUIRE(variant < kNumBVariants, "hmx_hs_batched: unknown variant");
     HMX_REQUIRE(k >= 1 && k <= kBVariants[variant].kmax, "hmx_hs_batched: k out of range");
@@ -989,14 +1025,9 @@ extern "C" int hmx_hs_batched_tune(const hmx_pair *pairs, int npairs, int ndx, c
     (void)hipEventDestroy(e0);
     (void)hipEventDestroy(e1);
     if (rc) return rc;
-    std::vector<int> sig;
-    for (int i = 0; i < npairs; ++i) {
-        sig.push_back(pairs[i].H);
-        sig.push_back(pairs[i].W);
-    }
     {
         std::lock_guard<std::mutex> lk(g_bmu);
-        g_btuned.push_back({sig, {bv, bk}});
+        g_btuned.push_back({pair_sizes(pairs, npairs), {bv, bk}});
     }
     if (variant_out) *variant_out = bv;
     if (k_out) *k_out = bk;
@@ -1007,5 +1038,6 @@ extern "C" int hmx_hs_batched_release(void) {
     std::lock_guard<std::mutex> lk(g_bmu);
     for (auto &p : g_plans) free_plan(p);
     g_plans.clear();
+    g_bchoices.clear();
     return HMX_OK;
 }
