@@ -10,6 +10,7 @@
 #include "hmx_common.h"
 
 #include <algorithm>
+#include <type_traits>
 #include <vector>
 
 #pragma clang fp contract(off)
@@ -77,11 +78,14 @@ static int launch_csr_L(int L, int nrows, const int *rows, const int *indptr,
 // lane's bit for bit.  The per-entry read of the direct form waits for its
 // index before its x gather, entry after entry; here a lane's gathers are
 // independent and in flight together.  What bounds it: the two memory latencies
-// (index, gather) of a wave against how few of its reads are in flight.  With
+// (index, gather) of a wave against how few of its reads are in flight.  With up to
 // CSRW_U = 5 entries per lane read at once (a 5-point operator's span in one
 // pass) the 2048^2 operator takes 45 us, 4.4 TB/s, against 60 us for a loop that
-// the compiler unrolled with each entry's gather behind its own index.  A wave whose span exceeds its LDS
-// share (CSRW_CAP entries) runs the direct loop.  Waves synchronise only with
+// the compiler unrolled with each entry's gather behind its own index.  A pass reads as
+// many 64-entry chunks as the span has: always five cost 2^20 rows of 1, 2, 3, 7 and 8
+// entries 13.5, 19.4, 25.1, 47.4 and 53.1 us, against 10.2, 15.6, 21.1, 43.4 and
+// 48.7.  A wave whose span exceeds its LDS share (CSRW_CAP entries) runs the direct
+// loop.  Waves synchronise only with
 // themselves (no work-group barrier), so a wave past the last row just exits.
 constexpr int CSRW_NT = 256, CSRW_CAP = 640, CSRW_U = 5;
 
@@ -98,29 +102,46 @@ __global__ __launch_bounds__(CSRW_NT) void csr_wave_rows_kernel(int nrows,
     const int64_t row = row0 + lane;
     const bool has = row < nrows;
     const int64_t last = row0 + 64 < nrows ? row0 + 64 : nrows;
-    const int base = indptr[row0];
-    const int span = indptr[last] - base;  // the same value in every lane
+    const int first = indptr[row0], past = indptr[last];  // the same values in every lane
     const int beg = has ? indptr[row] : 0, end = has ? indptr[row + 1] : 0;
+    const int base = __builtin_amdgcn_readfirstlane(first);
+    const int span = __builtin_amdgcn_readfirstlane(past) - base;
     float acc = 0.0f;
     if (span <= CSRW_CAP) {
         float2 *S = stage[wave];
-        // CSRW_U entries per lane at a time: their indices and values are read
-        // together, then the gathers (past the span a lane repeats its first entry)
-        for (int k0 = lane; k0 < span; k0 += 64 * CSRW_U) {
-            int id[CSRW_U];
-            float d[CSRW_U];
+        // U entries per lane from span entry k0: their indices and values are read
+        // together, then the gathers (past the span a lane repeats the last entry, into
+        // cells that no row reads: whole chunks fit the share)
+        static_assert(CSRW_CAP % 64 == 0, "whole chunks");
+        auto take = [&](int k0, auto u_c, auto whole_c) {
+            constexpr int U = decltype(u_c)::value;
+            constexpr bool WHOLE = decltype(whole_c)::value;  // no lane is past the span
+            int id[U];
+            float d[U], xv[U];
 #pragma unroll
-            for (int q = 0; q < CSRW_U; ++q) {
-                const int j = base + (k0 + 64 * q < span ? k0 + 64 * q : k0);
+            for (int q = 0; q < U; ++q) {
+                const int k = k0 + 64 * q + lane;
+                const int j = base + (WHOLE ? k : min(k, span - 1));
                 id[q] = indices[j];
                 d[q] = data[j];
             }
-            float xv[CSRW_U];
 #pragma unroll
-            for (int q = 0; q < CSRW_U; ++q) xv[q] = x[id[q]];
+            for (int q = 0; q < U; ++q) xv[q] = x[id[q]];
 #pragma unroll
-            for (int q = 0; q < CSRW_U; ++q)
-                if (k0 + 64 * q < span) S[k0 + 64 * q] = make_float2(d[q], xv[q]);
+            for (int q = 0; q < U; ++q)
+                S[k0 + 64 * q + lane] = make_float2(d[q], xv[q]);
+        };
+        int k0 = 0;
+        for (; k0 + 64 * CSRW_U <= span; k0 += 64 * CSRW_U)
+            take(k0, std::integral_constant<int, CSRW_U>(), std::true_type());
+        static_assert(CSRW_U == 5, "a case for each count");
+        switch ((span - k0 + 63) / 64) {  // uniform
+            case 0: break;
+            case 1: take(k0, std::integral_constant<int, 1>(), std::false_type()); break;
+            case 2: take(k0, std::integral_constant<int, 2>(), std::false_type()); break;
+            case 3: take(k0, std::integral_constant<int, 3>(), std::false_type()); break;
+            case 4: take(k0, std::integral_constant<int, 4>(), std::false_type()); break;
+            default: take(k0, std::integral_constant<int, 5>(), std::false_type()); break;
         }
         // the wave's LDS writes before its reads (a wavefront's LDS accesses
         // are performed in order; the fences keep the compiler's order)
