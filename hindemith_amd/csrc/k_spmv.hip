@@ -263,8 +263,10 @@ __global__ __launch_bounds__(RB_NT) void csr_rowblock_kernel(const int *__restri
 // resident.  Both passes: 430 us with 512 rows a work-group and SL_U entries per
 // thread in flight, 485 with 256 rows and one entry at a time; 2 to 4 rows per thread
 // take 421 - 540, fewer resident waves 478 - 625, and a persistent form that
-// prefetches the next rows' entries 550 - 590.
-constexpr int SL_N = 8, SL_RB = 512, SL_U = 4, SL_CAP = SL_RB * SL_U;
+// prefetches the next rows' entries 550 - 590.  A long row's sum is a chain of LDS
+// latencies that its whole work-group waits for: with SL_R reads in flight, 2^20 rows of 2
+// entries and every 500th of 700 take 53 us, one by one 98 (66 with 256 rows a group).
+constexpr int SL_N = 8, SL_RB = 512, SL_U = 4, SL_CAP = SL_RB * SL_U, SL_R = 8;
 
 __global__ __launch_bounds__(SL_RB) void csr_slice_kernel(int M, const int *__restrict__ sptr,
                                                           const int *__restrict__ sidx,
@@ -305,7 +307,15 @@ __global__ __launch_bounds__(SL_RB) void csr_slice_kernel(int M, const int *__re
             if (tid + q * SL_RB < m) prod[tid + q * SL_RB] = d[q] * xv[q];
         __syncthreads();
         const int lo = max(a, cb) - cb, hi = min(e, cb + m) - cb;
-        for (int k = lo; k < hi; ++k) acc += prod[k];
+        int k = lo;
+        for (; k + SL_R <= hi; k += SL_R) {  // SL_R reads in flight, added in the same order
+            float p[SL_R];
+#pragma unroll
+            for (int q = 0; q < SL_R; ++q) p[q] = prod[k + q];
+#pragma unroll
+            for (int q = 0; q < SL_R; ++q) acc += p[q];
+        }
+        for (; k < hi; ++k) acc += prod[k];
         __syncthreads();
     }
     if (row < r1) __builtin_nontemporal_store(acc, partial + (int64_t)s * M + row);
