@@ -83,8 +83,9 @@ static int launch_csr_L(int L, int nrows, const int *rows, const int *indptr,
 // pass) the 2048^2 operator takes 45 us, 4.4 TB/s, against 60 us for a loop that
 // the compiler unrolled with each entry's gather behind its own index.  A pass reads as
 // many 64-entry chunks as the span has: always five cost 2^20 rows of 1, 2, 3, 7 and 8
-// entries 13.5, 19.4, 25.1, 47.4 and 53.1 us, against 10.2, 15.6, 21.1, 43.4 and
-// 48.7.  A wave whose span exceeds its LDS share (CSRW_CAP entries) runs the direct
+// entries 13.6, 19.5, 25.1, 47.4 and 53.1 us, against 9.9, 15.3, 20.7, 43.6 and
+// 49.3.  (Full passes without their lanes' conditions take the 2048^2 operator, read
+// from memory among other kernels, 2 us longer.)  A wave whose span exceeds its LDS share (CSRW_CAP entries) runs the direct
 // loop.  Waves synchronise only with
 // themselves (no work-group barrier), so a wave past the last row just exits.
 constexpr int CSRW_NT = 256, CSRW_CAP = 640, CSRW_U = 5;
@@ -110,18 +111,15 @@ __global__ __launch_bounds__(CSRW_NT) void csr_wave_rows_kernel(int nrows,
     if (span <= CSRW_CAP) {
         float2 *S = stage[wave];
         // U entries per lane from span entry k0: their indices and values are read
-        // together, then the gathers (past the span a lane repeats the last entry, into
-        // cells that no row reads: whole chunks fit the share)
-        static_assert(CSRW_CAP % 64 == 0, "whole chunks");
-        auto take = [&](int k0, auto u_c, auto whole_c) {
+        // together, then the gathers (past the span a lane repeats its first entry)
+        auto take = [&](int k0, auto u_c) {
             constexpr int U = decltype(u_c)::value;
-            constexpr bool WHOLE = decltype(whole_c)::value;  // no lane is past the span
             int id[U];
             float d[U], xv[U];
+            if (k0 >= span) return;
 #pragma unroll
             for (int q = 0; q < U; ++q) {
-                const int k = k0 + 64 * q + lane;
-                const int j = base + (WHOLE ? k : min(k, span - 1));
+                const int j = base + (k0 + 64 * q < span ? k0 + 64 * q : k0);
                 id[q] = indices[j];
                 d[q] = data[j];
             }
@@ -129,19 +127,18 @@ __global__ __launch_bounds__(CSRW_NT) void csr_wave_rows_kernel(int nrows,
             for (int q = 0; q < U; ++q) xv[q] = x[id[q]];
 #pragma unroll
             for (int q = 0; q < U; ++q)
-                S[k0 + 64 * q + lane] = make_float2(d[q], xv[q]);
+                if (k0 + 64 * q < span) S[k0 + 64 * q] = make_float2(d[q], xv[q]);
         };
-        int k0 = 0;
-        for (; k0 + 64 * CSRW_U <= span; k0 += 64 * CSRW_U)
-            take(k0, std::integral_constant<int, CSRW_U>(), std::true_type());
         static_assert(CSRW_U == 5, "a case for each count");
+        int k0 = 0;
+        for (; span - k0 > 64 * (CSRW_U - 1); k0 += 64 * CSRW_U)
+            take(k0 + lane, std::integral_constant<int, CSRW_U>());
         switch ((span - k0 + 63) / 64) {  // uniform
-            case 0: break;
-            case 1: take(k0, std::integral_constant<int, 1>(), std::false_type()); break;
-            case 2: take(k0, std::integral_constant<int, 2>(), std::false_type()); break;
-            case 3: take(k0, std::integral_constant<int, 3>(), std::false_type()); break;
-            case 4: take(k0, std::integral_constant<int, 4>(), std::false_type()); break;
-            default: take(k0, std::integral_constant<int, 5>(), std::false_type()); break;
+            case 1: take(k0 + lane, std::integral_constant<int, 1>()); break;
+            case 2: take(k0 + lane, std::integral_constant<int, 2>()); break;
+            case 3: take(k0 + lane, std::integral_constant<int, 3>()); break;
+            case 4: take(k0 + lane, std::integral_constant<int, 4>()); break;
+            default: break;
         }
         // the wave's LDS writes before its reads (a wavefront's LDS accesses
         // are performed in order; the fences keep the compiler's order)
