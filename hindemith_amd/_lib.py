@@ -90,7 +90,9 @@ _SIGS = {
 }
 _RESTYPE = {"hmx_last_error": c_char_p, "hmx_version": c_char_p}
 _RESTYPE_ARGS = {"hmx_hs_forward_workspace": ([c_int, c_int, c_int], c_int64),
-                 "hmx_hs_adjoint_workspace": ([c_int, c_int, c_int, c_int], c_int64)}
+                 "hmx_hs_adjoint_workspace": ([c_int, c_int, c_int, c_int], c_int64),
+                 "hmx_hs_adjoint_workspace_taps": ([c_int, c_int, c_int, c_int, c_int, vp, vp, vp],
+                                                   c_int64)}
 
 _lib = None
 _load_error = None

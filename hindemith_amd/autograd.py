@@ -6,11 +6,11 @@ frame stacks and per-pair ``alpha`` (B,) on the GPU and returns the flow
 and keeps the state every ``ckpt_every`` iterations (every 8 for the canonical
 averaging stencil, where that takes no more memory); the backward pass
 (hand-written adjoint kernels, libhmx ``hmx_hs_adjoint``) recomputes one segment
-at a time and walks it backwards, so memory is at most
-(iters/ckpt_every + ckpt_every) state pairs instead of iters.  For stencils
-other than the canonical one the forward keeps the last segment's linearisation
-(up to ckpt_every more pairs of planes), so the backward recomputes every
-segment but that one.
+at a time and walks it backwards, so checkpoints and recomputed planes are at most
+ceil(iters/ckpt_every) + ckpt_every pairs instead of iters.  For stencils
+other than the canonical one the recompute ping-pongs through two pairs more, and the
+forward keeps the last segment's linearisation (up to ckpt_every more), so the
+backward recomputes every segment but that one.
 Gradients flow to I1, I2, alpha and, when given, the initial flow u0, v0.
 """
 from __future__ import annotations
@@ -51,8 +51,9 @@ def _canonical(avg):
 def _segment(iters, every):
     """Checkpoint interval of the canonical stencil's passes.  Its backward works in
     blocks of 8 steps from the state before each: a checkpoint per block saves it
-    the recompute of those states, where that keeps no more pairs of planes than
-    one checkpoint per interval and one pair per step of an interval would."""
+    the recompute of those states (and the planes to keep them in), where that keeps no
+    more pairs of planes than one checkpoint per interval and one pair per step of
+    an interval would."""
     return _BLOCK if -(-iters // _BLOCK) <= -(-iters // every) + every else every
 
 
@@ -109,9 +110,11 @@ class HornSchunckFunction(torch.autograd.Function):
         ga = torch.empty_like(alpha)
         gu0 = torch.empty_like(I1) if ctx.has_u0 else None
         gv0 = torch.empty_like(I1) if ctx.has_u0 else None
-        ws = torch.empty(int(L.hmx_hs_adjoint_workspace(B, H, W, ctx.ckpt_every)) // 4 + 1,
-                         device=I1.device, dtype=torch.float32)
         keep, targs = _tap_args(ctx.taps)
+        need = int(L.hmx_hs_adjoint_workspace_taps(B, H, W, ctx.ckpt_every, *targs[-4:]))
+        if need < 0:
+            check(-need, "hs_adjoint_workspace")
+        ws = torch.empty(need // 4 + 1, device=I1.device, dtype=torch.float32)
         null = ctypes.c_void_p(0)
         check(L.hmx_hs_adjoint(_ptr(I1), _ptr(I2), B, H, W, _ptr(alpha), *targs, ctx.iters,
                                ctx.ckpt_every, _ptr(ckpt), _ptr(lin) if ctx.lin else null,

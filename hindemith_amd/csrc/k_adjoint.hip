@@ -596,6 +596,30 @@ static int64_t adj_tiles(int H, int W) {
 int launch_hs_copy2(const float *u, const float *v, float *wu, float *wv, int64_t n,
                     hipStream_t s);
 
+// The canonical averaging stencil runs fused reverse blocks (hs_adj_rows.h);
+// HMX_ADJ_GENERIC=1 and HMX_LIN_STAGED=1 take the two-launch form, same
+// results bit for bit.
+static bool adj_fused(const Taps &av) {
+    auto set = [](const char *name) {
+        const char *e = std::getenv(name);
+        return e && e[0] == '1';
+    };
+    return hs_ring_taps(av) && !set("HMX_ADJ_GENERIC") && !set("HMX_LIN_STAGED");
+}
+
+// Plane pairs that walking a segment of up to ckpt_every steps back takes: states the
+// recompute ping-pongs through, and those it keeps (lin): the two-launch form every
+// step's (ubar, vbar), the fused blocks the state before each block but the first.
+struct AdjPlanes {
+    int64_t states, lin;
+};
+static AdjPlanes adj_planes(bool fused, int ckpt_every) {
+    const int64_t every = std::max(ckpt_every, 1);
+    const int64_t blocks = (every + ADJR_MMAX - 1) / ADJR_MMAX;
+    if (fused) return {blocks > 1 ? 1 : 0, blocks - 1};
+    return {2, every};
+}
+
 }  // namespace hmx
 
 using namespace hmx;
@@ -605,13 +629,25 @@ extern "C" int hmx_hs_ckpt_count(int iters, int ckpt_every) {
     return (iters + ckpt_every - 1) / ckpt_every;
 }
 
+// Bytes of the adjoint's workspace: Ix Iy It | gIx gIy gIt | 2 gradient ping-pong
+// pairs | per-pixel alpha terms | `states` recompute state pairs | `lin` pairs of a
+// segment | alpha^2 per pair | fp64 partial sums of the alpha terms
+static int64_t adj_workspace(int64_t n, int64_t B, AdjPlanes P) {
+    const int64_t floats = 3 * n + 3 * n + 4 * n + n + 2 * n * (P.states + P.lin);
+    return floats * 4 + B * 4 + 256 + B * GALPHA_CHUNKS * 8;
+}
+
 extern "C" int64_t hmx_hs_adjoint_workspace(int B, int H, int W, int ckpt_every) {
-    const int64_t n = (int64_t)B * H * W;
-    // Ix Iy It | gIx gIy gIt | 2 gradient ping-pong pairs | 2 recompute state
-    // ping-pong pairs | per-pixel alpha terms | (ubar, vbar) of every step of
-    // one segment | alpha^2 per pair | fp64 partial sums of the alpha terms
-    const int64_t floats = 3 * n + 3 * n + 4 * n + 4 * n + n + 2 * n * std::max(ckpt_every, 1);
-    return floats * 4 + (int64_t)B * 4 + 256 + (int64_t)B * GALPHA_CHUNKS * 8;
+    return adj_workspace((int64_t)B * H * W, B, adj_planes(false, ckpt_every));
+}
+
+extern "C" int64_t hmx_hs_adjoint_workspace_taps(int B, int H, int W, int ckpt_every, int nda,
+                                                 const float *wa, const int *oxa,
+                                                 const int *oya) {
+    Taps av;
+    const int rc = make_taps(av, nda, wa, oxa, oya);
+    if (rc) return -rc;
+    return adj_workspace((int64_t)B * H * W, B, adj_planes(adj_fused(av), ckpt_every));
 }
 
 extern "C" int64_t hmx_hs_forward_workspace(int B, int H, int W) {
@@ -715,24 +751,19 @@ extern "C" int hmx_hs_adjoint(const float *I1, const float *I2, int B, int H, in
     }
     float *gIx = ws + 3 * n, *gIy = ws + 4 * n, *gIt = ws + 5 * n;
     float *g[2][2] = {{ws + 6 * n, ws + 7 * n}, {ws + 8 * n, ws + 9 * n}};
-    float *rs[2][2] = {{ws + 10 * n, ws + 11 * n}, {ws + 12 * n, ws + 13 * n}};
-    float *ga2 = ws + 14 * n;  // per-pixel running sums of the alpha term
-    float *lin = ws + 15 * n;  // slot j: ubar, vbar of the segment's step j
-    float *alpha2 = lin + 2 * n * ckpt_every;
+    float *ga2 = ws + 10 * n;  // per-pixel running sums of the alpha term
+    const bool fused = adj_fused(T.av);
+    const AdjPlanes planes = adj_planes(fused, ckpt_every);
+    float *rs0 = ws + 11 * n;  // states (pairs)
+    float *rs[2][2] = {{rs0, rs0 + n}, {rs0 + 2 * n, rs0 + 3 * n}};  // (fused: one pair at most)
+    float *lin = rs0 + 2 * n * planes.states;  // pair j: see AdjPlanes
+    float *alpha2 = lin + 2 * n * planes.lin;
     double *partial = (double *)(((uintptr_t)(alpha2 + B) + 255) & ~(uintptr_t)255);
 
     hipLaunchKernelGGL(alpha_sq_kernel, dim3((B + 63) / 64), dim3(64), 0, s, alpha, alpha2, B);
     HMX_LAUNCH_CHECK("alpha_sq");
     rc = fwd_workspace ? HMX_OK : setup_batch(I1, I2, B, H, W, T.dx, T.dy, T.dt, Ix, Iy, It, s);
     if (rc) return rc;
-    // The canonical averaging stencil runs fused reverse blocks (hs_adj_rows.h);
-    // HMX_ADJ_GENERIC=1 and HMX_LIN_STAGED=1 take the two-launch form, same
-    // results bit for bit.
-    auto set = [](const char *name) {
-        const char *e = std::getenv(name);
-        return e && e[0] == '1';
-    };
-    const bool fused = hs_ring_taps(T.av) && !set("HMX_ADJ_GENERIC") && !set("HMX_LIN_STAGED");
     if (!fused || iters == 0) {  // (a fused block starts them at zero itself)
         rc = launch_fill_f32(gIx, 0.0f, 3 * n, s);
         if (!rc) rc = launch_fill_f32(ga2, 0.0f, n, s);

@@ -285,9 +285,15 @@ int hmx_hs_solve(const float *I1, const float *I2, int H, int W, float alpha2,
 
 /* Number of checkpoints ceil(iters / ckpt_every). */
 int hmx_hs_ckpt_count(int iters, int ckpt_every);
-/* Workspace bytes for hmx_hs_forward_ckpt / hmx_hs_adjoint. */
+/* Workspace bytes for hmx_hs_forward_ckpt / hmx_hs_adjoint (the latter's for any
+ * averaging stencil). */
 int64_t hmx_hs_forward_workspace(int B, int H, int W);
 int64_t hmx_hs_adjoint_workspace(int B, int H, int W, int ckpt_every);
+/* The bytes hmx_hs_adjoint takes with this averaging stencil: for the canonical one
+ * 2 x B x H x W floats per 8-step block of a segment but the first, instead of per
+ * step.  Negative: the HMX_ERR_* code of a bad stencil. */
+int64_t hmx_hs_adjoint_workspace_taps(int B, int H, int W, int ckpt_every, int nda,
+                                      const float *wa, const int *oxa, const int *oya);
 
 /* Forward solve that stores the state (u, v) every ckpt_every iterations:
  * ckpt holds hmx_hs_ckpt_count() x 2 x B x H x W floats (state before
