@@ -21,6 +21,7 @@
 //     CSR launch;
 //   * a loop whose body is exactly the Horn-Schunck Jacobi update is replaced
 //     by the fused, temporally blocked HS kernel (k_hs.hip).
+#include "host_result.h"
 #include "program.h"
 
 #include <algorithm>
@@ -295,14 +296,6 @@ struct Node {
 
 struct ScalarStmt {
     int op, dst, a, b;  // symbol ids (b = -1 for unary/copy)
-};
-
-// A result's host copy.  Pinned, and kept while the record lives: a fresh pageable one per
-// run costs a page fault and a clearing pass per page besides a staged copy (the
-// canonical program at 1920x1080, two planes: 5.24 ms a call, 4.59 with these).
-struct HostResult {
-    char *p = nullptr;
-    int64_t cap = 0, bytes = 0;
 };
 
 struct Record {
@@ -1181,19 +1174,27 @@ static int allocate(Record &R) {
     return HMX_OK;
 }
 
+// 1 GiB of page-locked results (64 programs of two 1920x1080 planes); the others' are
+// pageable.
+static PinnedBudget g_pinned(int64_t(1) << 30);
+static void *pin_host(size_t bytes) {
+    void *p = nullptr;
+    if (hipHostMalloc(&p, bytes, hipHostMallocDefault) == hipSuccess) return p;
+    (void)hipGetLastError();  // (a refusal is not the next call's error)
+    return nullptr;
+}
+static void unpin_host(void *p) { (void)hipHostFree(p); }
+
 // The host copies that the plan's RETURN nodes need.
 static int allocate_results(Record &R, const std::vector<Node> &nodes) {
     for (const Node &n : nodes) {
         if (n.t == Node::RETURN) {
             if (R.results.size() < n.syms.size()) R.results.resize(n.syms.size());
             for (size_t i = 0; i < n.syms.size(); ++i) {
-                HostResult &h = R.results[i];
                 const int64_t bytes = R.syms[n.syms[i]].bytes[0];
-                if (h.cap >= bytes) continue;
-                if (h.p) (void)hipHostFree(h.p);
-                h = HostResult();
-                HMX_HIP_TRY(hipHostMalloc((void **)&h.p, (size_t)bytes, hipHostMallocDefault));
-                h.cap = bytes;
+                if (!host_result_reserve(R.results[i], bytes, g_pinned, pin_host, unpin_host))
+                    return fail(HMX_ERR_HIP, "no host memory for the result " +
+                                                 R.syms[n.syms[i]].name);
             }
         }
         int rc = allocate_results(R, n.body);
@@ -1206,8 +1207,7 @@ static void release_record(Record &R) {
     if (R.stream) (void)hipStreamSynchronize(R.stream);
     for (void *p : R.allocs) (void)hipFree(p);
     R.allocs.clear();
-    for (HostResult &h : R.results)
-        if (h.p) (void)hipHostFree(h.p);
+    for (HostResult &h : R.results) host_result_free(h, g_pinned, unpin_host);
     R.results.clear();
     R.nresults = 0;
     for (Group &g : R.groups) g.partials = nullptr;
@@ -1763,7 +1763,7 @@ extern "C" int hmx_result_read(int rec, int i, void *host, int64_t nbytes) {
         return fail(HMX_ERR_INVALID, "result " + std::to_string(i) + ": expected " +
                                          std::to_string(R->results[i].bytes) + " bytes");
     if (!host) return fail(HMX_ERR_INVALID, "null destination");
-    std::memcpy(host, R->results[i].p, (size_t)nbytes);
+    if (nbytes > 0) std::memcpy(host, R->results[i].p, (size_t)nbytes);
     return HMX_OK;
 }
 
