@@ -156,7 +156,8 @@ struct HsTri {
 };
 
 // Tile (txi, tyi) of the grid of tw x th tiles of image a, k steps; w: the
-// averaging weights in the canonical tap order.  The host keeps tw + 2k <= 64
+// averaging weights in the canonical tap order; off: the image's first element in the
+// planes (of a batch).  The host keeps tw + 2k <= 64
 // and th + 2k <= NW * P.
 // PRE: a row's left and right neighbours for the next step are read as soon as
 // the row is written, so their latency is a step away from their use (four
@@ -172,7 +173,7 @@ template <int NW, int P, bool PRE, int G, bool TWO, bool LOUT = false, bool SETU
 __device__ __forceinline__ void hs_rows_tile(const HsImage &a, int txi, int tyi, int tw, int th,
                                              int k, const float (&weights)[8],
                                              HsStripLds<NW, P> &lds,
-                                             const HsSetup *su = nullptr) {
+                                             const HsSetup *su = nullptr, int64_t off = 0) {
     static_assert(P >= 2, "a strip has a first and a last row");
     constexpr int WV = kRowsVgprWeights<NW, P, PRE>;
     float w[8];
@@ -197,7 +198,7 @@ __device__ __forceinline__ void hs_rows_tile(const HsImage &a, int txi, int tyi,
     // image's start, 3840x2160, 500 it: 5902 -> 5804 us (the stores need no 64-bit vector
     // additions); a uniform base for every row, 10 SALU instructions a row, 5949 -> 6080.
     const int rs = min(gy0 + r0, H - 1);
-    const int64_t strip = (int64_t)rs * W;
+    const int64_t strip = off + (int64_t)rs * W;
     const unsigned rowb = (unsigned)W * 4u;
 
     float cx[P], cy[P], ct[P], cd[P], cr[P], u[P], v[P];
