@@ -628,7 +628,9 @@ def main():
         "config": {"workload": f"horn_schunck_jacobi_{W}x{H}_fp32_{iters}it", "height": H,
                    "width": W, "iters": iters, "alpha": 1.0,
                    "kernel_variant": variant, "iters_per_launch": k,
-                   "tile": [vinfo["tile_w"], vinfo["tile_h"]],
+                   # (a row-register variant's tile follows from the image and k)
+                   "tile": None if vinfo["kernel"] == "hs_rows_kernel" else
+                   [vinfo["tile_w"], vinfo["tile_h"]],
                    "hbm_roofline_fraction_of_metric": round(value / (HBM_PEAK_GBS * 1e9 /
                                                                      BYTES_PER_PX_ITER / 1e6), 4),
                    "endpoint_error_px": round(epe, 4),
