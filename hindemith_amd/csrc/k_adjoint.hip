@@ -798,8 +798,8 @@ extern "C" int hmx_hs_adjoint(const float *I1, const float *I2, int B, int H, in
             // blocks from the last to the first
             const float *cu = ckpt + (int64_t)(2 * c) * n, *cv = cu + n;
             const int nb = (len + ADJR_MMAX - 1) / ADJR_MMAX, bs = (len + nb - 1) / nb;
-            int variant, k;
-            hs_choice(H, W, B, bs, false, T.av, variant, k);
+            int variant = 0, k = 1;
+            if (nb > 1) hs_choice(H, W, B, bs, false, T.av, variant, k);
             const float *su = cu, *sv = cv;
             for (int b = 1; b < nb && !rc; ++b) {
                 float *du = lin + (int64_t)2 * (b - 1) * n, *dv = du + n;
