@@ -257,7 +257,7 @@ __global__ __launch_bounds__(RB_NT) void csr_rowblock_kernel(const int *__restri
 // entries a row) miss it and fetch a line from the L2 each (92 % hits there), 0.33
 // per CU and clock, two thirds of what the line width allows; every other phase
 // (row pointers, entries, sums) hides behind them only with all 32 waves of a CU
-// resident.  Both passes: 430 us with 512 rows a work-group and SL_U entries per
+// resident.  Both passes: 420 us with 512 rows a work-group and SL_U entries per
 // thread in flight, 485 with 256 rows and one entry at a time; 2 to 4 rows per thread
 // take 421 - 540, fewer resident waves 478 - 625, and a persistent form that
 // prefetches the next rows' entries 550 - 590.  A long row's sum is a chain of LDS

@@ -301,7 +301,8 @@ int64_t hmx_hs_adjoint_workspace_taps(int B, int H, int W, int ckpt_every, int n
  * lin_last (may be null): receives the last checkpoint segment's
  * linearisation, 2 x L x B x H x W floats for its L iterations (iteration j's
  * ubar plane at 2j, vbar at 2j + 1), which lets hmx_hs_adjoint skip that
- * segment's recompute.  workspace keeps the derivative planes Ix, Iy, It (its
+ * segment's recompute with stencils other than the canonical one (whose adjoint does
+ * not read it: pass null).  workspace keeps the derivative planes Ix, Iy, It (its
  * first 3 x B x H x W floats), which hmx_hs_adjoint may read instead of
  * recomputing them. */
 int hmx_hs_forward_ckpt(const float *I1, const float *I2, int B, int H, int W,
